@@ -505,9 +505,9 @@ def bpa_leg(V, W, h=1e3, cpu=True):
     """The BPA 3-D stress balance (solve_BPA) on the reference's own BPA
     integrated test, ISMIP-HOM experiment A at L = 160 km with its settings:
     one solve from zero velocity on a 1 km mesh (timed after one untimed
-    solve), its stage times, and the BPA block product timed back to back
-    (HIP events; algorithmic bytes: blocks + column indices + row pointers +
-    x + y).  With cpu: the oracle's restatement of the reference iteration
+    solve), its stage times, and the BPA system's product timed back to back
+    (HIP events; algorithmic bytes: 2-D operator entries + row pointers +
+    per-triangle gradients + viscosity fields + x + y).  With cpu: the oracle's restatement of the reference iteration
     (GMRES(30) + ILU(0)) and the engine on the reference's 8 km mesh, and the
     largest velocity difference between the two."""
     import numpy as np
@@ -531,7 +531,7 @@ def bpa_leg(V, W, h=1e3, cpu=True):
                   "seconds_per_solve": t, "solves_per_s": 1.0 / t, "picard": info.n_visc_its,
                   "krylov": info.n_Axb_its, "rel_residual": info.rel_residual, "stage_ms": stages,
                   "max_surface_speed": float(np.hypot(u, v).reshape(w.nz, -1)[0].max())}
-    res["roofline_block_product"] = {"kernel": "k_bsr_spmv<double, OP_PLAIN> on the BPA system (back to back)",
+    res["roofline_block_product"] = {"kernel": "k_bpa_product<false> (rows formed from the 2-D operators; back to back)",
                                      "bound": "hbm", "avg_ms": spmv_ms, "algorithmic_bytes": spmv_bytes,
                                      "achieved": spmv_bytes / (spmv_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS,
                                      "unit": "GB/s", "frac": spmv_bytes / (spmv_ms * 1e-3) / 1e9 / HBM_PEAK_GBS}

@@ -110,6 +110,28 @@ def test_state_and_system_match_oracle(V, OB, L, name):
     s.close()
 
 
+@pytest.mark.parametrize("nz,h", [(3, 40e3), (4, 9e3), (32, 17e3)])
+def test_product_matches_oracle_at_the_ends_of_its_range(V, OB, L, nz, h):
+    """The matrix-free product and its residual norms at the smallest and
+    largest layer counts, on meshes smaller and larger than a workgroup, with
+    u and v rows of different kinds on one border and uneven layers.  Same
+    bounds as above: the same sums in another order, FP64."""
+    c = Case(h=h, zeta=np.linspace(0.0, 1.0, nz) ** 1.3)
+    m = c.mesh
+    kw = dict(glens_n=3.0, sliding_law=1, slid_weertman_m=3.0, bc_u=[0, 1, 0, 1], bc_v=[1, 0, 0, 1])
+    inp = _bumpy(c)
+    u, v = _field(c, 5)
+    print(f"BPA product nT={m.nT} nz={nz}", flush=True)
+    s = _solver(V, c, **kw)
+    gpu = s.bpa_residual(u, v, **_bpa_kw(inp))
+    s.close()
+    ora = OB.bpa_residual(c.md, c.aa, c.zs, params(L, **kw), inp, u, v)
+    assert max_rel(gpu["b"], ora["b"]) < 1e-11
+    scale = max(np.abs(ora["b"]).max(), np.abs(ora["r"]).max())
+    assert np.abs(gpu["r"] - ora["r"]).max() < 1e-10 * scale
+    assert abs(gpu["rel_residual"] - ora["rel_residual"]) < 1e-9 * ora["rel_residual"]
+
+
 def test_periodic_borders_match_oracle(V, OB, L):
     """'periodic_ISMIP-HOM' borders on a square centred on the origin: the
     lagged copy rows per layer."""

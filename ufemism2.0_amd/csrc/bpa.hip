@@ -13,10 +13,12 @@
 // with them, and every stiffness entry, is formed on the fly from the 2-D
 // operators (a->b, b->a, b->b 2nd order, a->a), the three-point zeta stencils
 // and the zeta gradients, which are themselves formed per point from a few
-// per-vertex / per-triangle thickness and surface gradients.  Block row
-// (ti, k) has the pattern {b->b row of ti} x {three layers of the zeta
-// stencil of k}, in that order, so entry p of a row is (b->b entry p / 3,
-// layer p % 3) with no lookup table.
+// per-vertex / per-triangle thickness and surface gradients.  The stiffness
+// matrix itself is not stored either: block row (ti, k) couples the triangles
+// of ti's b->b row over the three layers of the zeta stencil of k, and every
+// one of its blocks is a combination of that row's five 2-D coefficients, so
+// the product A x is formed from those (k_bpa_product).  Only the blocks of a
+// triangle's own column are written out, for the column solve below.
 //
 // The linear solve is GMRES(gmres_restart) (PETSc's default KSP method)
 // preconditioned by an exact solve of each triangle's column: the block
@@ -67,6 +69,7 @@ struct ZOps {
   const double *kkm, *kkd;     // [nz-1][2] k -> ks: map, d/dzeta (layers ks, ks+1)
   const int *ksc;              // [nz][2] ks -> k: staggered layers
   const double *ksm, *ksd;     // [nz][2] map, d/dzeta
+  double rsurf, rbase;         // 1 / spacing of the first and the last two layers
 };
 
 __device__ __forceinline__ int zbase(int k, int nz) { return min(max(k - 1, 0), nz - 3); }
@@ -74,7 +77,8 @@ __device__ __forceinline__ int zbase(int k, int nz) { return min(max(k - 1, 0), 
 // Per-triangle thickness and surface gradients (zeta_gradients.f90:108-137):
 // 0 Hi_b, 1 dHs/dx, 2 dHs/dy, 3 dHi/dx, 4 dHi/dy, 5 d2Hs/dx2, 6 d2Hs/dxdy,
 // 7 d2Hs/dy2, 8 d2Hi/dx2, 9 d2Hi/dxdy, 10 d2Hi/dy2 (b grid), 11 d(Hs-Hi)/dx,
-// 12 d(Hs-Hi)/dy (the ice base, calc_driving_stress of BPA_main.f90:1739-1742).
+// 12 d(Hs-Hi)/dy (the ice base, calc_driving_stress of BPA_main.f90:1739-1742),
+// 13 1 / max(10 m, Hi_b).
 constexpr int kZt = 16;
 
 struct ZGrad {
@@ -84,13 +88,13 @@ struct ZGrad {
 // zeta gradients at a b-grid point on level zeta (zeta_gradients.f90:160-196)
 __device__ __forceinline__ ZGrad zgrad_tri(const double *__restrict__ zt, double zeta) {
   ZGrad g;
-  const double h = fmax(10.0, zt[0]);
-  g.zx = (1.0 / h) * (zt[1] - zeta * zt[3]);
-  g.zy = (1.0 / h) * (zt[2] - zeta * zt[4]);
-  g.zz = -1.0 / h;
-  g.zxx = (zt[3] * -1.0 / h) * g.zx + (1.0 / h) * (zt[5] - zeta * zt[8]);
-  g.zxy = (zt[4] * -1.0 / h) * g.zx + (1.0 / h) * (zt[6] - zeta * zt[9]);
-  g.zyy = (zt[4] * -1.0 / h) * g.zy + (1.0 / h) * (zt[7] - zeta * zt[10]);
+  const double r = zt[13];
+  g.zx = r * (zt[1] - zeta * zt[3]);
+  g.zy = r * (zt[2] - zeta * zt[4]);
+  g.zz = -r;
+  g.zxx = -(zt[3] * r) * g.zx + r * (zt[5] - zeta * zt[8]);
+  g.zxy = -(zt[4] * r) * g.zx + r * (zt[6] - zeta * zt[9]);
+  g.zyy = -(zt[4] * r) * g.zy + r * (zt[7] - zeta * zt[10]);
   return g;
 }
 
@@ -108,7 +112,7 @@ struct BpaParams {
   double relax_copy;  // C%visc_it_relax of the lagged copy rows
   SlidingLaw sl;
   int do_subgrid;
-  int bc_u[4], bc_v[4];
+  int infinite;  // bit 4 uv + side: the border condition of u (uv = 0) or v on that side is 'infinite'
 };
 
 // ---------------------------------------------------------------------------
@@ -157,6 +161,7 @@ __global__ void __launch_bounds__(kBlock) k_zg_tri(int nT, const int *__restrict
   double *z = zt + (size_t)ti * kZt;
 #pragma unroll
   for (int i = 0; i < 13; ++i) z[i] = o[i];
+  z[13] = 1.0 / fmax(10.0, o[0]);
 }
 
 // b->a second derivatives of Hs and Hi (only for the ak outputs of the
@@ -255,7 +260,7 @@ __global__ void __launch_bounds__(kBlock) k_bpa_vertex(
     const double dzu = d0 * q0.x + d1 * q1.x + d2 * q2.x, dzv = d0 * q0.y + d1 * q1.y + d2 * q2.y;
     ux += zx * cm * dzu; uy += zy * cm * dzu; vx += zx * cm * dzv; vy += zy * cm * dzv;
     // vertical shear on the staggered layers s0, s1 of this triangle, mapped to layer k
-    const double zzs = -1.0 / fmax(10.0, zt[(size_t)ti * kZt]);
+    const double zzs = -zt[(size_t)ti * kZt + 13];
     const double2 a0 = col[s0], a1 = col[s0 + 1], c0 = col[s1], c1 = col[s1 + 1];
     const double us0 = zzs * (z.kkd[2 * s0] * a0.x + z.kkd[2 * s0 + 1] * a1.x);
     const double vs0 = zzs * (z.kkd[2 * s0] * a0.y + z.kkd[2 * s0 + 1] * a1.y);
@@ -295,7 +300,7 @@ __global__ void __launch_bounds__(kBlock) k_bpa_bks(int nT, ZOps z, const int *_
     ux += m * (w0 * a.x + w1 * b.x); uy += m * (w0 * a.y + w1 * b.y);
     vx += m * (w0 * a.z + w1 * b.z); vy += m * (w0 * a.w + w1 * b.w);
   }
-  const double zz = -1.0 / fmax(10.0, zt[(size_t)ti * kZt]);
+  const double zz = -zt[(size_t)ti * kZt + 13];
   const double2 c0 = x[(size_t)ti * nz + ks], c1 = x[(size_t)ti * nz + ks + 1];
   const double uz = zz * (z.kkd[2 * ks] * c0.x + z.kkd[2 * ks + 1] * c1.x);
   const double vz = zz * (z.kkd[2 * ks] * c0.y + z.kkd[2 * ks + 1] * c1.y);
@@ -351,17 +356,37 @@ __global__ void __launch_bounds__(kBlock) k_bpa_coef(int nT, ZOps z, const int *
 // stiffness matrix (solve_BPA_linearised, BPA_main.f90:330-1723)
 // ---------------------------------------------------------------------------
 
+// One entry of the 2-D b->b row of a triangle as the product reads it: three
+// 16-byte loads, the same for all layers of the row.
+struct alignas(16) BpaEntry {
+  double hx, hy, hxx, hxy, hyy;
+  int tj;
+  int adj;  // 1: tj shares an edge with the row's triangle ('infinite' borders)
+};
+
 struct BpaSys {
   int nT, nz;
-  const int *ptr, *crow;        // block rows ti*nz+k, entry -> row
-  const int *bb_ptr, *bb_ind, *TriC, *TriBI;
-  const double *bb_ddx, *bb_ddy, *bb_d2dx2, *bb_d2dxdy, *bb_d2dy2;
+  const int *bb_ptr, *bb_diag, *TriC, *TriBI;
+  const BpaEntry *ent;
   const double *zt;
   const double4 *coef;          // eta_bk, deta/dx, deta/dy, deta/dz
   const double *eta_bks, *beta_b;
   const int *bcm;               // prescribed mask per bk point (may be null)
   const double *bcu, *bcv;
 };
+
+__global__ void __launch_bounds__(kBlock) k_bpa_pack(int nnz, const int *__restrict__ row, const int *__restrict__ ind,
+                                                     const int *__restrict__ TriC, const double *__restrict__ hx,
+                                                     const double *__restrict__ hy, const double *__restrict__ hxx,
+                                                     const double *__restrict__ hxy, const double *__restrict__ hyy,
+                                                     BpaEntry *__restrict__ ent) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nnz) return;
+  const int ti = row[e], tj = ind[e];
+  int adj = 0;
+  for (int q = 0; q < 3; ++q) adj |= TriC[3 * ti + q] == tj;
+  ent[e] = BpaEntry{hx[e], hy[e], hxx[e], hxy[e], hyy[e], tj, tj != ti ? adj : 0};
+}
 
 // Row kind of component uv of bk point (ti, k): 0 free, 1 surface, 2 base,
 // 3 identity with a value (prescribed, 'zero', copy, base without sliding),
@@ -371,122 +396,225 @@ __device__ __forceinline__ int bpa_row_kind(const BpaSys &s, const BpaParams &p,
   const int tb = s.TriBI[ti];
   if (tb > 0) {
     const int side = (tb - 1) / 2;
-    const int choice = uv == 0 ? p.bc_u[side] : p.bc_v[side];
-    return choice == UFE_BC_INFINITE ? 4 : 3;
+    return (p.infinite >> (4 * uv + side)) & 1 ? 4 : 3;
   }
   if (k == 0) return 1;
   if (k == s.nz - 1) return p.sl.law == UFE_SLIDING_NO_SLIDING ? 3 : 2;
   return 0;
 }
 
-// One thread per block entry.  The 3-D operator coefficients of the entry
-// (calc_3D_matrix_operators_mesh_bk_bk, :832-1072) are formed from the b->b
-// entry and the zeta stencil, then combined per row kind: free rows
-// (:480-644), surface rows (:646-889), base rows (:891-1163), 'infinite'
-// borders (:1165-1723) and identity rows.
-__global__ void __launch_bounds__(kBlock) k_bpa_assemble(BpaSys s, ZOps z, BpaParams p, long nnzb,
-                                                         double4 *__restrict__ A) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nnzb) return;
-  const int nz = s.nz;
-  const int r = s.crow[e];
-  const int ti = r / nz, k = r % nz;
-  const int pos = (int)(e - s.ptr[r]);
-  const int ii = pos / 3, jz = pos % 3;
-  const int be = s.bb_ptr[ti] + ii;
-  const int tj = s.bb_ind[be];
-  const int kk = zbase(k, nz) + jz;
-  const bool diag = (tj == ti && kk == k);
-  double blk[4];  // (u row: u col, v col), (v row: u col, v col)
-  int kind[2] = {bpa_row_kind(s, p, ti, k, 0), bpa_row_kind(s, p, ti, k, 1)};
-  bool need_ops = false;
-  for (int uv = 0; uv < 2; ++uv) need_ops |= kind[uv] <= 2;
-  double ox = 0, oy = 0, oz = 0, oxx = 0, oxy = 0, oyy = 0, ozz = 0;
-  ZGrad g{};
-  if (need_ops) {
-    const double hx = s.bb_ddx[be], hy = s.bb_ddy[be];
-    const double hxx = s.bb_d2dx2[be], hxy = s.bb_d2dxdy[be], hyy = s.bb_d2dy2[be];
-    const double cz = z.d[3 * k + jz], czz = z.dd[3 * k + jz];
-    g = zgrad_tri(s.zt + (size_t)ti * kZt, z.zeta[k]);
-    if (kk == k) { ox += hx; oy += hy; oxx += hxx; oxy += hxy; oyy += hyy; }
-    if (tj == ti) {
-      ox += g.zx * cz;
-      oy += g.zy * cz;
-      oz += g.zz * cz;
-      oxx += g.zxx * cz + g.zx * g.zx * czz;
-      oxy += g.zxy * cz + g.zx * g.zy * czz;
-      oyy += g.zyy * cz + g.zy * g.zy * czz;
-      ozz += g.zz * g.zz * czz;
-    }
-    oxx += 2.0 * g.zx * hx * cz;
-    oxy += g.zx * hy * cz + g.zy * hx * cz;
-    oyy += 2.0 * g.zy * hy * cz;
+// Coefficients of the momentum row of component uv at (ti, k) on the 3-D
+// derivatives of its own and of the other velocity component (own d/ds, d/do,
+// d2/ds2, d2/do2, d/dz, d2/dz2; other d/do, d/ds, d2/dsdo; s = x for u, y for
+// v, o the other one), plus terms on the own point (c_k) and on the next layer
+// inwards (c_kn): free rows (BPA_main.f90:480-644), surface rows (:646-889)
+// and base rows (:891-1163).
+struct BpaRow {
+  double s, o, ss, oo, z, zz, c_k, c_kn, x_o, x_s, x_so;
+};
+
+template <int UV>
+__device__ __forceinline__ BpaRow bpa_row(const BpaSys &s, const ZOps &z, const ZGrad &g, const double *zt,
+                                          const double4 &c, int kind, int ti) {
+  const double ds = UV == 0 ? c.y : c.z, dox = UV == 0 ? c.z : c.y, dez = c.w;
+  double eta = c.x, hs = 0.0, ho = 0.0, R = dez, c_k = 0.0, c_kn = 0.0;
+  if (kind != 0) {
+    // surface: R = d eta/dz - 2 eta / dz dzeta/dz on the surface slope; base:
+    // R = d eta/dz + 2 eta / dz dzeta/dz on the slope of the ice base, and friction
+    const bool base = kind == 2;
+    const double *slope = zt + (base ? 11 : 1);
+    eta = s.eta_bks[(size_t)ti * (s.nz - 1) + (base ? s.nz - 2 : 0)];
+    const double rd = base ? z.rbase : z.rsurf, q = 2.0 * eta * rd * g.zz;
+    hs = slope[UV];
+    ho = slope[1 - UV];
+    R = base ? dez + q : dez - q;
+    c_kn = q * rd * g.zz;
+    c_k = -c_kn;
+    if (base) c_k += R * s.beta_b[ti] / eta;
   }
-  const double4 c = s.coef[r];
-  for (int uv = 0; uv < 2; ++uv) {
-    double own = 0.0, oth = 0.0;
-    const int kd = kind[uv];
-    if (kd == 3) {
-      own = diag ? 1.0 : 0.0;
-    } else if (kd == 4) {
-      if (kk == k) {
-        if (tj == ti) {
-          int n = 0;
-          for (int q = 0; q < 3; ++q) n += s.TriC[3 * ti + q] >= 0;
-          own = -(double)n;
-        } else {
-          for (int q = 0; q < 3; ++q)
-            if (s.TriC[3 * ti + q] == tj) own = 1.0;
-        }
+  BpaRow r;
+  r.s = 4.0 * ds + 4.0 * R * hs;
+  r.o = dox + R * ho;
+  r.x_o = 2.0 * ds + 2.0 * R * hs;
+  r.x_s = r.o;
+  r.ss = 4.0 * eta;
+  r.oo = eta;
+  r.x_so = 3.0 * eta;
+  r.z = kind == 0 ? dez : 0.0;
+  r.zz = kind == 0 ? eta : 0.0;
+  r.c_k = c_k;
+  r.c_kn = c_kn;
+  return r;
+}
+
+// The blocks of each triangle's own column on the layers k - 1, k, k + 1 (the
+// block tridiagonal part of the system that the column solve factors), in
+// [k][ti] order: L, D and U.  The 3-D operator coefficients on the own column
+// are those of calc_3D_matrix_operators_mesh_bk_bk (:832-1072).
+__global__ void __launch_bounds__(kBlock) k_bpa_column(BpaSys s, ZOps z, BpaParams p, double4 *__restrict__ Lb,
+                                                       double4 *__restrict__ Db, double4 *__restrict__ Ub) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long)s.nT * s.nz) return;
+  const int nz = s.nz, k = (int)(i / s.nT), ti = (int)(i % s.nT);
+  const BpaEntry e = s.ent[s.bb_diag[ti]];
+  const double *zt = s.zt + (size_t)ti * kZt;
+  const ZGrad g = zgrad_tri(zt, z.zeta[k]);
+  const double4 c = s.coef[(size_t)ti * nz + k];
+  const int b0 = zbase(k, nz);
+  const int kind0 = bpa_row_kind(s, p, ti, k, 0), kind1 = bpa_row_kind(s, p, ti, k, 1);
+  BpaRow ru{}, rv{};
+  if (kind0 <= 2) ru = bpa_row<0>(s, z, g, zt, c, kind0, ti);
+  if (kind1 <= 2) rv = bpa_row<1>(s, z, g, zt, c, kind1, ti);
+  int nn = 0;
+  for (int q = 0; q < 3; ++q) nn += s.TriC[3 * ti + q] >= 0;
+  auto block = [&](int kk) {
+    if (kk < 0 || kk >= nz) return make_double4(0.0, 0.0, 0.0, 0.0);
+    const int jz = kk - b0;  // k - 1 .. k + 1 lie in the stencil, except beyond the column
+    const double cz = z.d[3 * k + jz], czz = z.dd[3 * k + jz], at = kk == k ? 1.0 : 0.0;
+    const double ox = at * e.hx + g.zx * cz, oy = at * e.hy + g.zy * cz, oz = g.zz * cz, ozz = g.zz * g.zz * czz;
+    const double oxx = at * e.hxx + g.zxx * cz + g.zx * g.zx * czz + 2.0 * g.zx * e.hx * cz;
+    const double oxy = at * e.hxy + g.zxy * cz + g.zx * g.zy * czz + g.zx * e.hy * cz + g.zy * e.hx * cz;
+    const double oyy = at * e.hyy + g.zyy * cz + g.zy * g.zy * czz + 2.0 * g.zy * e.hy * cz;
+    // free rows have no c_k, c_kn
+    const double own_u = ru.c_k * at + (kk == (kind0 == 1 ? 1 : nz - 2) ? ru.c_kn : 0.0);
+    const double own_v = rv.c_k * at + (kk == (kind1 == 1 ? 1 : nz - 2) ? rv.c_kn : 0.0);
+    double4 o;
+    o.x = ru.s * ox + ru.o * oy + ru.ss * oxx + ru.oo * oyy + ru.z * oz + ru.zz * ozz + own_u;
+    o.y = ru.x_o * oy + ru.x_s * ox + ru.x_so * oxy;
+    o.z = rv.x_o * ox + rv.x_s * oy + rv.x_so * oxy;
+    o.w = rv.s * oy + rv.o * ox + rv.ss * oyy + rv.oo * oxx + rv.z * oz + rv.zz * ozz + own_v;
+    if (kind0 >= 3) { o.x = at * (kind0 == 3 ? 1.0 : -(double)nn); o.y = 0.0; }
+    if (kind1 >= 3) { o.w = at * (kind1 == 3 ? 1.0 : -(double)nn); o.z = 0.0; }
+    return o;
+  };
+  Lb[i] = block(k - 1);
+  Db[i] = block(k);
+  Ub[i] = block(k + 1);
+}
+
+// y = A x (RESID: y = rhs - A x with the partial sums of ||y||^2 and ||rhs||^2),
+// one thread per bk point, layers fastest.  A row needs five sums over its b->b
+// entries (the 2-D operators of f(tj, k) for u and v); the mixed terms, the
+// d/dx and d/dy of the vertical derivative, are the vertical derivative of the
+// d/dx and d/dy sums along the row's own column, so they come from the other
+// threads of the column through LDS.  A workgroup takes whole columns of
+// kBlock / nz consecutive triangles and stages their entries in LDS, so the
+// column indices are at hand and the gathers of several entries are in flight.
+// Bound: the entries (48 B) are read once per triangle and shared by its nz
+// layers, against 3 nz blocks of 36 B each when the matrix is stored; what is
+// left is x, y, the viscosity fields and the gathers of x in the caches.  On
+// ISMIP-HOM A at 2 km (51,838 triangles x 12 layers) the product takes 30.5 us
+// against 128 us (600 MB of blocks at 4.9 TB/s) and the system is no longer
+// assembled; at 8 km 6.1 us against 8.2 us.
+constexpr int kBpaStage = 512;  // entries staged at a time (24 KB): one pass for nz >= 5 at ten entries per row
+
+template <bool RESID>
+__global__ void __launch_bounds__(kBlock) k_bpa_product(BpaSys s, ZOps z, BpaParams p, const double2 *__restrict__ x,
+                                                        double2 *__restrict__ y, const double2 *__restrict__ rhs,
+                                                        RedSlot slot, const KrylovScalars *__restrict__ sc) {
+  if (sc && sc->done) return;
+  __shared__ BpaEntry ent[kBpaStage];
+  __shared__ double2 colx[kBlock], coly[kBlock];
+  __shared__ __align__(16) double tri[kBlock / 3 * kZt];  // the columns' thickness and surface gradients (nz >= 3)
+  const int nz = s.nz, per = kBlock / nz, ngroup = (s.nT + per - 1) / per;
+  const int lt = (int)threadIdx.x / nz, k = (int)threadIdx.x % nz;
+  const int b0 = zbase(k, nz);
+  const double d0 = z.d[3 * k], d1 = z.d[3 * k + 1], d2 = z.d[3 * k + 2];
+  double acc[3] = {0.0, 0.0, 0.0};
+  for (int grp = xcd_block(); grp < ngroup; grp += gridDim.x) {
+    const int t0 = grp * per, t1 = min(t0 + per, s.nT), ti = t0 + lt;
+    const bool live = lt < per && ti < t1;
+    const int g0 = s.bb_ptr[t0], g1 = s.bb_ptr[t1];
+    const int p0 = live ? s.bb_ptr[ti] : 0, p1 = live ? s.bb_ptr[ti + 1] : 0;
+    double2 sx{}, sy{}, sxx{}, sxy{}, syy{}, adj{};
+    int c0 = g0;
+    do {  // at least once: the barrier also ends the previous group's reads of the LDS columns
+      const int c1 = min(c0 + kBpaStage, g1);
+      __syncthreads();
+      const double2 *src = reinterpret_cast<const double2 *>(s.ent + c0);
+      double2 *dst = reinterpret_cast<double2 *>(ent);
+      for (int q = threadIdx.x; q < (c1 - c0) * 3; q += kBlock) dst[q] = src[q];
+      if (c0 == g0)
+        for (int q = threadIdx.x; q < (t1 - t0) * kZt; q += kBlock) tri[q] = s.zt[(size_t)t0 * kZt + q];
+      __syncthreads();
+      const int e1 = min(p1, c1);
+#pragma unroll 4
+      for (int e = max(p0, c0); e < e1; ++e) {
+        const BpaEntry &h = ent[e - c0];
+        const double2 f = x[(size_t)h.tj * nz + k];
+        sx.x += h.hx * f.x; sx.y += h.hx * f.y;
+        sy.x += h.hy * f.x; sy.y += h.hy * f.y;
+        sxx.x += h.hxx * f.x; sxx.y += h.hxx * f.y;
+        sxy.x += h.hxy * f.x; sxy.y += h.hxy * f.y;
+        syy.x += h.hyy * f.x; syy.y += h.hyy * f.y;
+        if (h.adj) { adj.x += f.x; adj.y += f.y; }
       }
-    } else {
-      const double os = uv == 0 ? ox : oy, oo = uv == 0 ? oy : ox;
-      const double oss = uv == 0 ? oxx : oyy, ooo = uv == 0 ? oyy : oxx;
-      const double ds = uv == 0 ? c.y : c.z, dox = uv == 0 ? c.z : c.y, dez = c.w;
-      if (kd == 0) {
-        const double eta = c.x;
-        own = 4.0 * eta * oss + 4.0 * ds * os + eta * ooo + dox * oo + eta * ozz + dez * oz;
-        oth = 3.0 * eta * oxy + 2.0 * ds * oo + dox * os;
-      } else {
-        const double *ztt = s.zt + (size_t)ti * kZt;
-        double eta, c_own_x, c_own_y, c_oth_x, c_oth_y, c_k, c_kn;
-        int kn;
-        if (kd == 1) {
-          eta = s.eta_bks[(size_t)ti * (nz - 1)];
-          const double hs = uv == 0 ? ztt[1] : ztt[2], ho = uv == 0 ? ztt[2] : ztt[1];
-          const double dz = z.zeta[1] - z.zeta[0];
-          const double q = 2.0 * eta / dz * g.zz;
-          c_own_x = 4.0 * ds - q * 4.0 * hs + 4.0 * dez * hs;
-          c_own_y = dox - q * ho + dez * ho;
-          c_oth_y = 2.0 * ds - q * 2.0 * hs + 2.0 * dez * hs;
-          c_oth_x = dox - q * ho + dez * ho;
-          c_k = -2.0 * eta / (dz * dz) * g.zz * g.zz;
-          c_kn = 2.0 * eta / (dz * dz) * g.zz * g.zz;
-          kn = 1;
-        } else {
-          eta = s.eta_bks[(size_t)ti * (nz - 1) + nz - 2];
-          const double bs = uv == 0 ? ztt[11] : ztt[12], bo = uv == 0 ? ztt[12] : ztt[11];
-          const double dz = z.zeta[nz - 1] - z.zeta[nz - 2];
-          const double Q = 2.0 * eta / (dz * dz) * g.zz * g.zz;
-          const double R = 2.0 * eta / dz * g.zz + dez;
-          c_own_x = 4.0 * ds + 4.0 * R * bs;
-          c_own_y = dox + R * bo;
-          c_oth_y = 2.0 * ds + 2.0 * R * bs;
-          c_oth_x = dox + R * bo;
-          c_k = (R * s.beta_b[ti] / eta) - Q;
-          c_kn = Q;
-          kn = nz - 2;
-        }
-        own = c_own_x * os + c_own_y * oo + 4.0 * eta * oss + eta * ooo;
-        if (tj == ti && kk == k) own += c_k;
-        if (tj == ti && kk == kn) own += c_kn;
-        oth = c_oth_y * oo + c_oth_x * os + 3.0 * eta * oxy;
+      c0 = c1;
+    } while (c0 < g1);
+    colx[threadIdx.x] = sx;
+    coly[threadIdx.x] = sy;
+    __syncthreads();
+    if (!live) continue;
+    const double2 *cx = colx + (threadIdx.x - k + b0), *cy = coly + (threadIdx.x - k + b0);
+    const double2 px = make_double2(d0 * cx[0].x + d1 * cx[1].x + d2 * cx[2].x,
+                                    d0 * cx[0].y + d1 * cx[1].y + d2 * cx[2].y);
+    const double2 py = make_double2(d0 * cy[0].x + d1 * cy[1].x + d2 * cy[2].x,
+                                    d0 * cy[0].y + d1 * cy[1].y + d2 * cy[2].y);
+    const size_t i = (size_t)ti * nz + k;
+    const double2 *xi = x + (size_t)ti * nz;
+    const double2 own = xi[k];
+    const int kind0 = bpa_row_kind(s, p, ti, k, 0), kind1 = bpa_row_kind(s, p, ti, k, 1);
+    double2 o = own;  // identity rows
+    if (kind0 == 4 || kind1 == 4) {
+      int nn = 0;
+      for (int q = 0; q < 3; ++q) nn += s.TriC[3 * ti + q] >= 0;
+      if (kind0 == 4) o.x = adj.x - (double)nn * own.x;
+      if (kind1 == 4) o.y = adj.y - (double)nn * own.y;
+    }
+    if (kind0 <= 2 || kind1 <= 2) {
+      const double *zt = tri + lt * kZt;
+      const ZGrad g = zgrad_tri(zt, z.zeta[k]);
+      const double4 c = s.coef[i];
+      const double2 q0 = xi[b0], q1 = xi[b0 + 1], q2 = xi[b0 + 2];
+      const double w0 = z.dd[3 * k], w1 = z.dd[3 * k + 1], w2 = z.dd[3 * k + 2];
+      const double zxx = g.zx * g.zx, zxy = g.zx * g.zy, zyy = g.zy * g.zy, zzz = g.zz * g.zz;
+      const double fzu = d0 * q0.x + d1 * q1.x + d2 * q2.x, fzv = d0 * q0.y + d1 * q1.y + d2 * q2.y;
+      const double gzu = w0 * q0.x + w1 * q1.x + w2 * q2.x, gzv = w0 * q0.y + w1 * q1.y + w2 * q2.y;
+      // 3-D derivatives of u and v at the point
+      const double ux = sx.x + g.zx * fzu, vx = sx.y + g.zx * fzv;
+      const double uy = sy.x + g.zy * fzu, vy = sy.y + g.zy * fzv;
+      const double uxx = sxx.x + g.zxx * fzu + zxx * gzu + 2.0 * g.zx * px.x;
+      const double vxx = sxx.y + g.zxx * fzv + zxx * gzv + 2.0 * g.zx * px.y;
+      const double uxy = sxy.x + g.zxy * fzu + zxy * gzu + g.zx * py.x + g.zy * px.x;
+      const double vxy = sxy.y + g.zxy * fzv + zxy * gzv + g.zx * py.y + g.zy * px.y;
+      const double uyy = syy.x + g.zyy * fzu + zyy * gzu + 2.0 * g.zy * py.x;
+      const double vyy = syy.y + g.zyy * fzv + zyy * gzv + 2.0 * g.zy * py.y;
+      if (kind0 <= 2) {
+        const BpaRow r = bpa_row<0>(s, z, g, zt, c, kind0, ti);
+        const double un = kind0 == 0 ? own.x : xi[kind0 == 1 ? 1 : nz - 2].x;
+        o.x = r.s * ux + r.o * uy + r.ss * uxx + r.oo * uyy + r.z * (g.zz * fzu) + r.zz * (zzz * gzu) +
+              r.c_k * own.x + r.c_kn * un + r.x_o * vy + r.x_s * vx + r.x_so * vxy;
+      }
+      if (kind1 <= 2) {
+        const BpaRow r = bpa_row<1>(s, z, g, zt, c, kind1, ti);
+        const double vn = kind1 == 0 ? own.y : xi[kind1 == 1 ? 1 : nz - 2].y;
+        o.y = r.s * vy + r.o * vx + r.ss * vyy + r.oo * vxx + r.z * (g.zz * fzv) + r.zz * (zzz * gzv) +
+              r.c_k * own.y + r.c_kn * vn + r.x_o * ux + r.x_s * uy + r.x_so * uxy;
       }
     }
-    if (uv == 0) { blk[0] = own; blk[1] = oth; }
-    else { blk[3] = own; blk[2] = oth; }
+    if (RESID) {
+      const double2 b = rhs[i];
+      o.x = b.x - o.x;
+      o.y = b.y - o.y;
+      acc[0] += o.x * o.x + o.y * o.y;
+      acc[1] += b.x * b.x + b.y * b.y;
+    }
+    y[i] = o;
   }
-  A[e] = make_double4(blk[0], blk[1], blk[2], blk[3]);
+  if (!RESID) return;
+  __shared__ double lds[3][kBlock / 64];
+  block_sum<3>(acc, lds);
+  block_partials<3>(slot, acc);
 }
 
 // Load vector per bk point: -tau_d (tau_d = -rho g grad Hs) on the momentum
@@ -545,30 +673,17 @@ __device__ __forceinline__ double2 m2vec(double4 a, double2 v) {
   return make_double2(a.x * v.x + a.y * v.y, a.z * v.x + a.w * v.y);
 }
 
-// Entry of block (ti, k) -> (ti, kk) for |kk - k| <= 1 within the stencil, or -1.
-__device__ __forceinline__ long col_entry(const int *__restrict__ ptr, const int *__restrict__ bb_ptr,
-                                          const int *__restrict__ bb_diag, int nz, int ti, int k, int kk) {
-  const int j = kk - zbase(k, nz);
-  if (kk < 0 || kk >= nz || j < 0 || j > 2) return -1;
-  return (long)ptr[ti * nz + k] + 3L * (bb_diag[ti] - bb_ptr[ti]) + j;
-}
-
-// Factor per triangle: D'_0 = D_0, W_k = L_k D'_{k-1}^-1, D'_k = D_k - W_k U_{k-1};
-// stores D'^-1, W and U per layer in [k][ti] order.
-__global__ void __launch_bounds__(kBlock) k_col_factor(int nT, int nz, const int *__restrict__ ptr,
-                                                       const int *__restrict__ bb_ptr, const int *__restrict__ bb_diag,
-                                                       const double4 *__restrict__ A, double4 *__restrict__ Dinv,
-                                                       double4 *__restrict__ W, double4 *__restrict__ U) {
+// Factor per triangle: D'_0 = D_0, W_k = L_k D'_{k-1}^-1, D'_k = D_k - W_k U_{k-1},
+// in place on the blocks of k_bpa_column ([k][ti] order): W over L, D'^-1 over D.
+__global__ void __launch_bounds__(kBlock) k_col_factor(int nT, int nz, double4 *__restrict__ Dinv,
+                                                       double4 *__restrict__ W, const double4 *__restrict__ U) {
   const int ti = blockIdx.x * blockDim.x + threadIdx.x;
   if (ti >= nT) return;
   double4 dprev_inv = make_double4(1, 0, 0, 1), uprev = make_double4(0, 0, 0, 0);
   for (int k = 0; k < nz; ++k) {
-    const long ed = col_entry(ptr, bb_ptr, bb_diag, nz, ti, k, k);
-    const long el = col_entry(ptr, bb_ptr, bb_diag, nz, ti, k, k - 1);
-    const long eu = col_entry(ptr, bb_ptr, bb_diag, nz, ti, k, k + 1);
-    double4 D = A[ed];
-    const double4 L = el >= 0 ? A[el] : make_double4(0, 0, 0, 0);
-    const double4 Uk = eu >= 0 ? A[eu] : make_double4(0, 0, 0, 0);
+    const size_t o = (size_t)k * nT + ti;
+    double4 D = Dinv[o];
+    const double4 L = W[o], Uk = U[o];
     double4 w = make_double4(0, 0, 0, 0);
     if (k > 0) {
       w = m2mul(L, dprev_inv);
@@ -576,10 +691,8 @@ __global__ void __launch_bounds__(kBlock) k_col_factor(int nT, int nz, const int
     }
     dprev_inv = m2inv(D);
     uprev = Uk;
-    const size_t o = (size_t)k * nT + ti;
     Dinv[o] = dprev_inv;
     W[o] = w;
-    U[o] = Uk;
   }
 }
 
@@ -685,17 +798,17 @@ struct BpaState {
   DBuf aa_ptr, aa_ind, aa_ddx, aa_ddy;
   DBuf zeta, zs, zd, zdd, kkm, kkd, ksc, ksm, ksd;
   std::vector<double> h_zeta;
-  // block pattern (built on the first BPA call)
-  int nb = 0;
-  long nnzb = 0;
-  DBuf ptr, col, crow, bb_diag_copy;
+  // b->b rows as the product reads them (packed on the first BPA call)
+  int nb = 0, bb_nnz = 0;
+  DBuf ent;
   int n_copy = 0;
   DBuf copy_row, copy_ptr, copy_tri, copy_w;
   // inputs and geometry
   DBuf Hi, Hs, A_ak, A_bks, rough, fgr, bcm, bcu, bcv, zv, zt, a2, tribi;
   bool has_bc = false;
   // iteration
-  DBuf x, xprev, rhs, sr4, eta_ak, eta_bks, coef, beta_a, beta_b, A, cDinv, cW, cU, part, out, r;
+  DBuf x, xprev, rhs, sr4, eta_ak, eta_bks, coef, beta_a, beta_b, cDinv, cW, cU, part, out, r;
+  BpaParams par{};  // of the system formed last
   std::unique_ptr<Krylov> kry;
   // stage timings of the last solve (HIP events on the context's stream)
   hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -712,6 +825,8 @@ struct BpaState {
     z.d = zd.as<double>(); z.dd = zdd.as<double>();
     z.kkm = kkm.as<double>(); z.kkd = kkd.as<double>();
     z.ksc = ksc.as<int>(); z.ksm = ksm.as<double>(); z.ksd = ksd.as<double>();
+    z.rsurf = 1.0 / (h_zeta[1] - h_zeta[0]);
+    z.rbase = 1.0 / (h_zeta[nz - 1] - h_zeta[nz - 2]);
     return z;
   }
 };
@@ -801,36 +916,21 @@ void bpa_inputs(ufe_ctx *c, BpaState &b, const ufe_bpa_inputs *in, bool need_bc)
   UFE_HIP(hipStreamSynchronize(s));  // host vectors end here
 }
 
-// Block pattern of the BPA system, once per context.
+void set_operator(ufe_ctx *c, BpaState &b);
+
+// Packed b->b rows and work arrays of the BPA system, once per context.
 void bpa_pattern(ufe_ctx *c, BpaState &b) {
   if (b.nb) return;
   const DevMesh &m = *ctx_mesh(c);
   hipStream_t s = ctx_stream(c);
   const int nT = b.nT, nz = b.nz;
-  std::vector<int> bp(nT + 1), bi(m.bb_nnz);
-  UFE_HIP(hipMemcpy(bp.data(), m.bb_ptr, sizeof(int) * (nT + 1), hipMemcpyDeviceToHost));
-  UFE_HIP(hipMemcpy(bi.data(), m.bb_ind, sizeof(int) * m.bb_nnz, hipMemcpyDeviceToHost));
-  const long nnzb = 3L * nz * m.bb_nnz;
-  if (nnzb >= (1L << 31)) throw std::runtime_error("BPA system too large for 32-bit block indices");
+  if (3L * nz * m.bb_nnz >= (1L << 31)) throw std::runtime_error("BPA system too large for 32-bit block indices");
   b.nb = nT * nz;
-  b.nnzb = nnzb;
-  std::vector<int> ptr((size_t)b.nb + 1), col(nnzb), crow(nnzb);
-  long e = 0;
-  for (int ti = 0; ti < nT; ++ti)
-    for (int k = 0; k < nz; ++k) {
-      const int r = ti * nz + k;
-      ptr[r] = (int)e;
-      const int base = std::min(std::max(k - 1, 0), nz - 3);
-      for (int q = bp[ti]; q < bp[ti + 1]; ++q)
-        for (int j = 0; j < 3; ++j, ++e) {
-          col[e] = bi[q] * nz + base + j;
-          crow[e] = r;
-        }
-    }
-  ptr[b.nb] = (int)e;
-  up(b.ptr, ptr.data(), sizeof(int) * ptr.size(), s);
-  up(b.col, col.data(), sizeof(int) * col.size(), s);
-  up(b.crow, crow.data(), sizeof(int) * crow.size(), s);
+  b.bb_nnz = m.bb_nnz;
+  ensure(b.ent, sizeof(BpaEntry) * (size_t)m.bb_nnz);
+  hipLaunchKernelGGL(k_bpa_pack, dim3(blocks_for(m.bb_nnz)), dim3(kBlock), 0, s, m.bb_nnz, m.bb_row, m.bb_ind, m.TriC,
+                     m.bb_ddx, m.bb_ddy, m.bb_d2dx2, m.bb_d2dxdy, m.bb_d2dy2, b.ent.as<BpaEntry>());
+  UFE_LAUNCH_CHECK();
   // lagged copy rows of the periodic borders
   std::vector<int> crw, cp, ct;
   std::vector<double> cw;
@@ -854,13 +954,13 @@ void bpa_pattern(ufe_ctx *c, BpaState &b) {
   ensure(b.coef, sizeof(double4) * nbk);
   ensure(b.beta_a, sizeof(double) * b.nV);
   ensure(b.beta_b, sizeof(double) * nT);
-  ensure(b.A, sizeof(double4) * (size_t)nnzb);
   ensure(b.cDinv, sizeof(double4) * nbk);
   ensure(b.cW, sizeof(double4) * nbk);
   ensure(b.cU, sizeof(double4) * nbk);
   ensure(b.part, sizeof(double) * kMaxPartials * 2);
   ensure(b.out, sizeof(double) * 2);
   b.kry = std::make_unique<Krylov>(b.nb, s);
+  set_operator(c, b);
   for (hipEvent_t &ev : b.ev) UFE_HIP(hipEventCreate(&ev));
 }
 
@@ -877,7 +977,8 @@ BpaParams bpa_params(const ufe_ctx *c, double eps0_applied) {
   q.subgrid_exp = p.subgrid_friction_exponent;
   q.relax_copy = p.visc_it_relax;
   q.do_subgrid = p.do_gl_subgrid_friction;
-  for (int i = 0; i < 4; ++i) { q.bc_u[i] = p.bc_u[i]; q.bc_v[i] = p.bc_v[i]; }
+  for (int i = 0; i < 4; ++i)
+    q.infinite |= (p.bc_u[i] == UFE_BC_INFINITE) << i | (p.bc_v[i] == UFE_BC_INFINITE) << (4 + i);
   return q;
 }
 
@@ -885,9 +986,8 @@ BpaSys bpa_sys(ufe_ctx *c, const BpaState &b, const int *TriBI_dev) {
   const DevMesh &m = *ctx_mesh(c);
   BpaSys s{};
   s.nT = b.nT; s.nz = b.nz;
-  s.ptr = b.ptr.as<int>(); s.crow = b.crow.as<int>();
-  s.bb_ptr = m.bb_ptr; s.bb_ind = m.bb_ind; s.TriC = m.TriC; s.TriBI = TriBI_dev;
-  s.bb_ddx = m.bb_ddx; s.bb_ddy = m.bb_ddy; s.bb_d2dx2 = m.bb_d2dx2; s.bb_d2dxdy = m.bb_d2dxdy; s.bb_d2dy2 = m.bb_d2dy2;
+  s.bb_ptr = m.bb_ptr; s.bb_diag = m.bb_diag; s.TriC = m.TriC; s.TriBI = TriBI_dev;
+  s.ent = b.ent.as<BpaEntry>();
   s.zt = b.zt.as<double>();
   s.coef = b.coef.as<double4>();
   s.eta_bks = b.eta_bks.as<double>();
@@ -898,17 +998,42 @@ BpaSys bpa_sys(ufe_ctx *c, const BpaState &b, const int *TriBI_dev) {
   return s;
 }
 
+// Size of the system for the Krylov solver; its products go through the
+// operator set by set_operator.
 BsrT<double> bpa_bsr(const BpaState &b) {
   BsrT<double> A;
-  A.nb = b.nb; A.nnzb = (int)b.nnzb; A.ptr = b.ptr.as<int>(); A.col = b.col.as<int>();
-  A.val = b.A.as<double4>(); A.dinv = nullptr;
+  A.nb = b.nb;
   return A;
 }
 
-// The state at the current iterate x and the system assembled there
-// (calc_strain_rates, calc_effective_viscosity,
-// calc_applied_basal_friction_coefficient, solve_BPA_linearised's assembly);
-// the copy rows read xprev.
+// The Krylov solver's product with the system formed last: y = A x, or with
+// rhs the residual y = rhs - A x and its partial sums (their number returned).
+void set_operator(ufe_ctx *c, BpaState &b) {
+  BpaState *bp = &b;
+  b.kry->set_custom_op([c, bp](const double *x, double *y, const double *rhs, const RedSlot &slot,
+                               const KrylovScalars *sc) -> int {
+    const BpaSys sys = bpa_sys(c, *bp, bp->tribi.as<int>());
+    int g = xcd_grid(blocks_for(bp->nT, kBlock / bp->nz));
+    hipStream_t s = ctx_stream(c);
+    if (rhs) {
+      g = std::min(g, kMaxPartials);
+      hipLaunchKernelGGL(k_bpa_product<true>, dim3(g), dim3(kBlock), 0, s, sys, bp->zops(), bp->par,
+                         reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y),
+                         reinterpret_cast<const double2 *>(rhs), slot, sc);
+    } else {
+      hipLaunchKernelGGL(k_bpa_product<false>, dim3(g), dim3(kBlock), 0, s, sys, bp->zops(), bp->par,
+                         reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y),
+                         (const double2 *)nullptr, slot, sc);
+    }
+    UFE_LAUNCH_CHECK();
+    return g;
+  });
+}
+
+// The state at the current iterate x and the system there (calc_strain_rates,
+// calc_effective_viscosity, calc_applied_basal_friction_coefficient; of
+// solve_BPA_linearised's matrix the own-column blocks, the rest lives in
+// k_bpa_product); the copy rows read xprev.
 void bpa_state_and_system(ufe_ctx *c, BpaState &b, const BpaParams &p, const int *TriBI_dev) {
   const DevMesh &m = *ctx_mesh(c);
   hipStream_t s = ctx_stream(c);
@@ -930,8 +1055,9 @@ void bpa_state_and_system(ufe_ctx *c, BpaState &b, const BpaParams &p, const int
   UFE_LAUNCH_CHECK();
   if (b.ev[1]) UFE_HIP(hipEventRecord(b.ev[1], s));
   const BpaSys sys = bpa_sys(c, b, TriBI_dev);
-  hipLaunchKernelGGL(k_bpa_assemble, dim3(blocks_for(b.nnzb)), dim3(kBlock), 0, s, sys, z, p, b.nnzb,
-                     b.A.as<double4>());
+  b.par = p;
+  hipLaunchKernelGGL(k_bpa_column, dim3(blocks_for((long)b.nb)), dim3(kBlock), 0, s, sys, z, p, b.cW.as<double4>(),
+                     b.cDinv.as<double4>(), b.cU.as<double4>());
   UFE_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_bpa_rhs, dim3(blocks_for((long)b.nb)), dim3(kBlock), 0, s, sys, p, b.rhs.as<double2>());
   UFE_LAUNCH_CHECK();
@@ -1004,10 +1130,8 @@ int check_inputs(ufe_ctx *c, const ufe_bpa_inputs *in) {
 }
 
 void col_factor(ufe_ctx *c, BpaState &b) {
-  const DevMesh &m = *ctx_mesh(c);
-  hipLaunchKernelGGL(k_col_factor, dim3(blocks_for(b.nT)), dim3(kBlock), 0, ctx_stream(c), b.nT, b.nz, b.ptr.as<int>(),
-                     m.bb_ptr, m.bb_diag, b.A.as<double4>(), b.cDinv.as<double4>(), b.cW.as<double4>(),
-                     b.cU.as<double4>());
+  hipLaunchKernelGGL(k_col_factor, dim3(blocks_for(b.nT)), dim3(kBlock), 0, ctx_stream(c), b.nT, b.nz,
+                     b.cDinv.as<double4>(), b.cW.as<double4>(), b.cU.as<double4>());
   UFE_LAUNCH_CHECK();
 }
 
@@ -1021,7 +1145,7 @@ void set_column_pc(ufe_ctx *c, BpaState &b) {
   });
 }
 
-// ||b - A x|| / ||b|| of the system assembled last, at x
+// ||b - A x|| / ||b|| of the system formed last, at x
 double bpa_rel_residual(BpaState &b) {
   double rr = 0.0, bb = 0.0;
   b.kry->residual64(bpa_bsr(b), b.x.as<double>(), b.rhs.as<double>(), b.r.as<double>(), &rr, &bb);
@@ -1375,7 +1499,11 @@ extern "C" int ufe_bpa_profile_spmv(ufe_ctx *c, int reps, double *avg_ms, double
   return ctx_guard(c, [&]() -> int {
     BpaState *b = state(c);
     if (!b || !b->nb) return ctx_fail(c, UFE_ERR_ARGUMENT, "no BPA system has been assembled");
-    *avg_ms = b->kry->time_spmv64(bpa_bsr(*b), b->x.as<double>(), b->r.as<double>(), reps, bytes);
+    *avg_ms = b->kry->time_spmv64(bpa_bsr(*b), b->x.as<double>(), b->r.as<double>(), reps, nullptr);
+    // b->b entries and row pointers, per-triangle gradients and border index,
+    // viscosity fields, x and y, once each
+    *bytes = (double)b->bb_nnz * sizeof(BpaEntry) + (double)(b->nT + 1) * sizeof(int) +
+             (double)b->nT * (kZt * sizeof(double) + sizeof(int)) + (double)b->nb * (sizeof(double4) + 2 * sizeof(double2));
     return UFE_OK;
   });
 }

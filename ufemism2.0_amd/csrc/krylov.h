@@ -120,6 +120,14 @@ class Krylov {
   // A preconditioner of the caller's, z = M^-1 r on the FP64 vectors, used by
   // gmres64 in place of the built-in ones while set (empty function: off).
   void set_custom_pc(std::function<void(const double *r, double *z)> f) { custom_pc_ = std::move(f); }
+  // A system of the caller's that is not stored as blocks (A.val null), used by
+  // gmres64, residual64 and time_spmv64: y = A x when b is null, else y = b - A x
+  // with the partial sums of ||y||^2 and ||b||^2 (and a zero third sum) in the
+  // slot; returns the number of partials.  Nothing is launched that reads the
+  // vectors when sc->done is set (sc may be null).
+  using OpFn = std::function<int(const double *x, double *y, const double *b, const RedSlot &slot,
+                                 const KrylovScalars *sc)>;
+  void set_custom_op(OpFn f) { custom_op_ = std::move(f); }
   // Launch BiCGStab iteration chunks as replays of captured HIP graphs
   // (same kernels in the same order: identical results).
   void set_graphs(bool on) { use_graphs_ = on; }
@@ -187,6 +195,9 @@ class Krylov {
   int nb_;
   hipStream_t s_;
   std::function<void(const double *, double *)> custom_pc_;
+  OpFn custom_op_;
+  template <typename T> void product(const BsrT<T> &A, const T *x, T *y, KrylovScalars *sc);
+  template <typename T> void residual(const BsrT<T> &A, const T *x, T *y, const T *b, const RedSlot &slot, double *out);
   int pc_ = UFE_PC_BLOCK_JACOBI;
   const AmgHierarchy *amg_ = nullptr;
   const int *A_diag_ = nullptr;

@@ -198,6 +198,33 @@ static void spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T 
   }
 }
 
+// y = A x through the caller's operator when the system has no stored blocks
+template <typename T>
+void Krylov::product(const BsrT<T> &A, const T *x, T *y, KrylovScalars *sc) {
+  if constexpr (std::is_same<T, double>::value) {
+    if (!A.val && custom_op_) {
+      custom_op_(x, y, nullptr, slot(0), sc);
+      return;
+    }
+  }
+  spmv_launch<T, OP_PLAIN>(A, x, y, nullptr, nullptr, slot(0), nullptr, sc, s_);
+}
+
+// y = b - A x with ||y||^2, ||b||^2 and 0 in out (through slot)
+template <typename T>
+void Krylov::residual(const BsrT<T> &A, const T *x, T *y, const T *b, const RedSlot &sl, double *out) {
+  if constexpr (std::is_same<T, double>::value) {
+    if (!A.val && custom_op_) {
+      const int g = custom_op_(x, y, b, sl, nullptr);
+      hipLaunchKernelGGL((k_spmv_finish<OP_RESID>), dim3(1), dim3(kFinishBlock), 0, s_, sl, g, out,
+                         (KrylovScalars *)nullptr);
+      UFE_LAUNCH_CHECK();
+      return;
+    }
+  }
+  spmv_launch<T, OP_RESID>(A, x, y, b, nullptr, sl, out, nullptr, s_, 0.0);
+}
+
 // ===========================================================================
 // Block-local preconditioners, fused into vector updates
 // ===========================================================================
@@ -975,10 +1002,9 @@ double Krylov::time_spmv64(const BsrT<double> &A, const double *x, double *y, in
   hipEvent_t e0, e1;
   UFE_HIP(hipEventCreateWithFlags(&e0, hipEventDisableSystemFence));
   UFE_HIP(hipEventCreateWithFlags(&e1, hipEventDisableSystemFence));
-  RedSlot sl = slot(3);
-  spmv_launch<double, OP_PLAIN>(A, x, y, nullptr, nullptr, sl, nullptr, nullptr, s_);  // warm caches/clocks
+  product<double>(A, x, y, nullptr);  // warm caches/clocks
   UFE_HIP(hipEventRecord(e0, s_));
-  for (int i = 0; i < reps; ++i) spmv_launch<double, OP_PLAIN>(A, x, y, nullptr, nullptr, sl, nullptr, nullptr, s_);
+  for (int i = 0; i < reps; ++i) product<double>(A, x, y, nullptr);
   UFE_HIP(hipEventRecord(e1, s_));
   UFE_HIP(hipEventSynchronize(e1));
   float ms = 0.0f;
@@ -1014,7 +1040,8 @@ float *Krylov::tmp32(int i) { return vec32_[i].as<float>(); }
 void Krylov::residual64(const BsrT<double> &A, const double *x, const double *b, double *r, double *rr,
                         double *bb, double vmax, int *n_clamped, const double4 *dblk, int write_unscaled) {
   RedSlot sl = slot(3);
-  spmv_launch<double, OP_RESID>(A, x, r, b, nullptr, sl, sl.result, nullptr, s_, vmax, dblk, write_unscaled);
+  if (!A.val) residual<double>(A, x, r, b, sl, sl.result);
+  else spmv_launch<double, OP_RESID>(A, x, r, b, nullptr, sl, sl.result, nullptr, s_, vmax, dblk, write_unscaled);
   double h[3];
   UFE_HIP(hipMemcpyAsync(h, sl.result, sizeof(h), hipMemcpyDeviceToHost, s_));
   UFE_HIP(hipStreamSynchronize(s_));
@@ -1761,7 +1788,7 @@ SolveStats Krylov::gmres(const BsrT<T> &A, const T *b, T *x, double rtol, double
   const int pred0 = last_gmres_its_[sizeof(T) == 4];
   for (int cycle = 0;; ++cycle) {
     // true residual into v0 (the norm of the system given)
-    spmv_launch<T, OP_RESID>(A, x, V, b, nullptr, sl0, sl0.result, nullptr, s_, 0.0);
+    residual<T>(A, x, V, b, sl0, sl0.result);
     double h0[3];
     UFE_HIP(hipMemcpyAsync(h0, sl0.result, sizeof(h0), hipMemcpyDeviceToHost, s_));
     UFE_HIP(hipStreamSynchronize(s_));
@@ -1793,7 +1820,7 @@ SolveStats Krylov::gmres(const BsrT<T> &A, const T *b, T *x, double rtol, double
                              A_diag_, sc);
           UFE_LAUNCH_CHECK();
         }
-        spmv_launch<T, OP_PLAIN>(A, z, w, nullptr, nullptr, sl0, nullptr, sc, s_);
+        product<T>(A, z, w, sc);
         if (R == 4) gmres_dots_update<T, 4>(n, j + 1, V, n, w, part, gs, j, sc, s_);
         else gmres_dots_update<T, 16>(n, j + 1, V, n, w, part, gs, j, sc, s_);
         hipLaunchKernelGGL(k_gmres_scale<T>, dim3(blocks_for(n)), dim3(kBlock), 0, s_, n, w, gs, sc);

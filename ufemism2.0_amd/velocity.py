@@ -432,7 +432,7 @@ class VelocitySolver:
         return dict(zip(("state", "assembly", "column_factor", "gmres", "update"), ms.tolist()))
 
     def bpa_profile_spmv(self, reps=100):
-        """(average ms, algorithmic bytes) of the BPA block product."""
+        """(average ms, algorithmic bytes) of the product with the BPA system."""
         ms, by = C.c_double(0.0), C.c_double(0.0)
         self._check(self.lib.ufe_bpa_profile_spmv(self._ctx, int(reps), C.byref(ms), C.byref(by)))
         return ms.value, by.value
