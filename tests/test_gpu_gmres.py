@@ -41,6 +41,31 @@ def test_gmres_vs_direct(V, OB, L, dome, restart):
     assert max_rel(x, xd) < 1e-8
 
 
+@pytest.mark.parametrize("n,restart", [(2, 1), (3, 2), (514, 9), (4097, 64), (300_001, 17)])
+def test_gmres_basis_passes_at_the_ends_of_their_range(V, L, n, restart):
+    """Fewer unknowns than a wavefront, one more than a workgroup's, more than
+    the basis passes' grid takes at once, every remainder of their column
+    groups; rows scaled over twelve decades (the stored basis vectors are
+    only normalised to a power of two).  The bound on the error is the
+    residual tolerance times a bound on the condition number after the point
+    Jacobi scaling (diagonally dominant by a factor 2: 3)."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n)
+    m = 4 * n
+    A = sp.coo_matrix((rng.uniform(-1, 1, m), (rng.integers(0, n, m), rng.integers(0, n, m))), shape=(n, n)).tocsr()
+    A.setdiag(0.0)
+    A = A + sp.diags(2.0 * np.asarray(abs(A).sum(axis=1)).ravel() + 1.0)
+    x_ex = rng.normal(size=n)
+    s = 10.0 ** rng.uniform(-6, 6, n)
+    A = sp.csr_matrix(sp.diags(s) @ A)
+    d = 1.0 / A.diagonal()
+    As, bs = sp.csr_matrix(sp.diags(d) @ A), d * (A @ x_ex)
+    x, its, rel = V.csr_solve(As, 1e-9 * bs, rtol=1e-13, maxit=5000, krylov=L.KRYLOV_GMRES, restart=restart,
+                              precond=L.PC_NONE)
+    assert rel <= 1e-13
+    assert np.linalg.norm(1e9 * x - x_ex) < 3e-13 * np.linalg.norm(x_ex) + 1e-14 * np.sqrt(n)
+
+
 def test_gmres_argument_errors(V, L, dome):
     import scipy.sparse as sp
     A = sp.identity(10, format="csr")
