@@ -187,6 +187,36 @@ def test_newtonian_slab_closed_form(V, L, sx, sy):
     s.close()
 
 
+@pytest.mark.parametrize("nz,h", [(3, 30e3), (4, 12e3), (5, 12e3), (6, 16e3), (9, 12e3), (32, 20e3)])
+def test_column_solve_at_the_ends_of_its_range(V, L, nz, h):
+    """Layer counts around the column solve's look-ahead and its largest, on
+    partly filled wavefronts: the slab's closed form, which the discretisation
+    holds exactly, and few GMRES steps (the column solve removes the vertical
+    coupling; a wrong factor in one layer leaves it).  With 32 layers the
+    residual cannot fall to 1e-13: the round-off of A u, eta / dz^2 |u| ~ 4e3 *
+    500 against |b| ~ 450, is 4e-13 |b|, so the solve asks for 1e-11 there, and
+    the bound on the velocity, which is proportional to the residual, is 100
+    times the other cases'."""
+    c = Case(h=h, zeta=np.linspace(0.0, 1.0, nz) ** 1.2)
+    H, beta, eta = 1000.0, 500.0, 0.5 / 5e-7
+    rtol, bound = (1e-11, 1e-6) if nz == 32 else (1e-13, 1e-8)
+    inp = _slab_inputs(c, -0.03, 0.04, H=H, beta=beta)
+    kw = dict(glens_n=1.0, sliding_law=1, slid_weertman_m=1.0, visc_it_relax=1.0, visc_it_norm_dUV_tol=1e-24,
+              visc_it_nit=1, rtol=rtol, abstol=0.0, krylov_maxit=20000, do_gl_subgrid_friction=0, vel_max=1e6)
+    s = _solver(V, c, **kw)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", V.ViscosityIterationWarning)
+        u, v, info = s.solve_BPA(inp["Hi"], inp["Hs"], inp["A_flow"], inp["beta_sq"], inp["fgr_b"],
+                                 inp["mask_grounded"])
+    s.close()
+    print(f"column solve nT={c.mesh.nT} nz={nz}: {info.n_Axb_its} steps in {info.n_visc_its} iterations", flush=True)
+    ue, ve = _slab_exact(c, -0.03, 0.04, H, beta, eta, c.zeta)
+    scale = max(np.abs(ue).max(), np.abs(ve).max())
+    assert np.abs(u.reshape(nz, -1) - ue[:, None]).max() < bound * scale
+    assert np.abs(v.reshape(nz, -1) - ve[:, None]).max() < bound * scale
+    assert info.n_Axb_its <= 200  # 92 to 106 with the exact column solve
+
+
 @pytest.mark.parametrize("sliding", [1, 0])
 def test_converged_solve_matches_oracle(V, OB, L, sliding):
     """n = 3 over a bumpy bed, weak linear sliding or none, from the same start."""
