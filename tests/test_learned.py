@@ -56,6 +56,43 @@ def test_gradients_match_reference(graph):
         assert np.linalg.norm(got - ref) <= 2e-2 * np.linalg.norm(ref) + 1e-7, k
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 131, 40_000])
+def test_layer_kernels_at_the_edges_of_their_tiles(n):
+    """Fewer nodes than a tile, one more than a tile, more tiles than
+    workgroups; a chain graph with end nodes of one neighbour and, every
+    seventh node, none.  Bounds of the tests above (BF16 operands; a rounding
+    to BF16 that flips is 2^-8 of one operand)."""
+    from ufemism2_amd import learned as LN
+    rng = np.random.default_rng(n)
+    nb = np.full((n, 3), -1, np.int32)
+    i = np.arange(n - 1)
+    i = i[(i % 7 != 0) & ((i + 1) % 7 != 0)]
+    nb[i, 0] = i + 1
+    nb[i + 1, 2] = i
+    X = rng.normal(size=(n, M.F_IN)).astype(np.float32)
+    T = rng.normal(size=(n, M.N_T)).astype(np.float32)
+    p = params(n % 5)
+    net = LN.Mpnn(0, LN.flatten_params(p))
+    Y = net.forward(X, nb)
+    loss, g = net.loss_grad(X, nb, T)
+    bad = nb.copy()
+    bad[0, 1] = n          # out of range
+    with pytest.raises(LN.MpnnError, match="range and symmetric"):
+        net.forward(X, bad)
+    if n > 2:
+        bad[0, 1] = 2      # not symmetric
+        with pytest.raises(LN.MpnnError, match="range and symmetric"):
+            net.loss_grad(X, bad, T)
+    net.close()
+    lr, gr, Yr = M.loss_and_grad(p, X, nb, T, bf=True)
+    assert np.abs(Y[:, :M.N_T] - Yr[:, :M.N_T]).max() <= 2e-3 * np.abs(Yr[:, :M.N_T]).max()
+    assert abs(loss - lr) <= 1e-3 * lr
+    gd = LN.unflatten_grad(g, p)
+    for k in p:
+        cut = np.s_[..., :M.N_T] if k in ("Wd", "bd") else np.s_[...]
+        assert np.linalg.norm(gd[k][cut] - gr[k][cut]) <= 2e-2 * np.linalg.norm(gr[k][cut]) + 1e-7, k
+
+
 def test_training_reduces_loss(graph):
     """Fit a smooth function of the features (learnable by construction)."""
     from ufemism2_amd import learned as LN

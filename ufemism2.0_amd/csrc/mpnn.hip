@@ -14,16 +14,25 @@
 // minimises sum_i ||y_i[0:3] - t_i||^2 / N with Adam (full batch over the
 // disjoint union of the training graphs).
 //
-// Kernels
-//   k_rowgemm<K, NO, EPI>  C[N,NO] = A[N,K] W[K,NO] (+ bias, epilogue); one
-//       workgroup = 4 wavefronts = a 64-row tile; W^T (bf16) and the A tile
-//       (converted to bf16) are staged in LDS with K contiguous, so each lane
-//       reads its 4 consecutive bf16 operands with one 64-bit LDS load.
-//   k_colgemm<K, NO>       partial sums of A^T B over the rows of each
-//       workgroup (weight gradients) plus column sums of B (bias gradients);
-//       k_reduce_parts adds the partials in a fixed order (deterministic).
-//   gathers: k_concat_mean (forward aggregation), k_dh_update (its adjoint,
-//       as a gather over the symmetric neighbour lists: no atomics).
+// Kernels (one workgroup = 4 wavefronts = 64-row tiles, grid-stride; operands
+// are converted to bf16 in LDS with the reduction index contiguous, so each
+// lane reads its 8 (or 4) consecutive operands with one LDS load):
+//   k_layer_fwd     one message-passing layer: the rows of h and the means over
+//       the neighbours are gathered straight into the LDS tile of [h | mean];
+//       keeps one bit per output for the backward pass (pre-activation > 0)
+//   k_rowgemm       encoder and decoder
+//   k_decoder_back  loss, dY, gradient of Wd and bd, dH of the last layer
+//   k_layer_back    one layer backward: dH (the previous kernel's own part plus
+//       the gather of its neighbour part, the adjoint of the mean), dZ, weight
+//       and bias gradient of the layer and both parts of the next dH, from one
+//       tile; [h | mean] is gathered again instead of being kept
+//   k_encoder_back  the same end for the encoder
+//   k_reduce_parts  adds the workgroups' partial gradients in a fixed order
+// Bound: HBM passes over the [N, 64] fields.  A layer reads and writes two
+// fields forward and reads three and writes two backward (N = 160k: 41 MB each);
+// with a kernel per operation and Cat, Z, dZ and dCat in memory one gradient took
+// 2.66 ms of kernel time at N = 160k, now 0.62 ms (one layer: forward 45 us against
+// 144 us, backward 127 us against 495 us).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -60,22 +69,88 @@ __device__ __forceinline__ f32x4 mfma_tile(const unsigned short *p, const unsign
   }
 }
 
-// float32 -> bfloat16, round to nearest even
-__device__ __forceinline__ unsigned short f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
+// float32 -> bfloat16, round to nearest even (gfx950 converts in hardware)
+__device__ __forceinline__ unsigned short f2bf(float f) { return __builtin_bit_cast(unsigned short, (__bf16)f); }
+
+// Four consecutive rows of 4 columns (one float4 per row) -> bf16, row-major
+// tile of pitch P at (row 4 rg, column 4 c4).
+template <int P>
+__device__ __forceinline__ void put_rows(unsigned short *t, int rg, int c4, const float4 (&v)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const bf16x4 o = {(short)f2bf(v[q].x), (short)f2bf(v[q].y), (short)f2bf(v[q].z), (short)f2bf(v[q].w)};
+    *reinterpret_cast<bf16x4 *>(&t[(4 * rg + q) * P + 4 * c4]) = o;
+  }
 }
 
-enum { EPI_ENC = 0, EPI_MP = 1, EPI_LIN = 2 };
+// The same values transposed: column-major tile of pitch P (rows contiguous).
+template <int P>
+__device__ __forceinline__ void put_cols(unsigned short *t, int rg, int c4, const float4 (&v)[4]) {
+  const bf16x4 o0 = {(short)f2bf(v[0].x), (short)f2bf(v[1].x), (short)f2bf(v[2].x), (short)f2bf(v[3].x)};
+  const bf16x4 o1 = {(short)f2bf(v[0].y), (short)f2bf(v[1].y), (short)f2bf(v[2].y), (short)f2bf(v[3].y)};
+  const bf16x4 o2 = {(short)f2bf(v[0].z), (short)f2bf(v[1].z), (short)f2bf(v[2].z), (short)f2bf(v[3].z)};
+  const bf16x4 o3 = {(short)f2bf(v[0].w), (short)f2bf(v[1].w), (short)f2bf(v[2].w), (short)f2bf(v[3].w)};
+  *reinterpret_cast<bf16x4 *>(&t[(4 * c4 + 0) * P + 4 * rg]) = o0;
+  *reinterpret_cast<bf16x4 *>(&t[(4 * c4 + 1) * P + 4 * rg]) = o1;
+  *reinterpret_cast<bf16x4 *>(&t[(4 * c4 + 2) * P + 4 * rg]) = o2;
+  *reinterpret_cast<bf16x4 *>(&t[(4 * c4 + 3) * P + 4 * rg]) = o3;
+}
+
+__device__ __forceinline__ void add4(float4 &a, const float4 &b) { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
+
+// The rows r0 + 4 rg .. + 3 of h and the means over their valid neighbours
+// (summed in list order), 4 columns each; zero past the last row.
+__device__ __forceinline__ void load_cat(int N, int r0, int rg, int c4, const float4 *__restrict__ H,
+                                         const int *__restrict__ nb, float4 (&h)[4], float4 (&m)[4]) {
+  int j[4][3];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int row = r0 + 4 * rg + q;
+#pragma unroll
+    for (int n = 0; n < 3; ++n) j[q][n] = row < N ? nb[3 * row + n] : -1;
+    h[q] = row < N ? H[(size_t)row * (kHid / 4) + c4] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float4 s{0.0f, 0.0f, 0.0f, 0.0f};
+    int d = 0;
+#pragma unroll
+    for (int n = 0; n < 3; ++n)
+      if (j[q][n] >= 0) {
+        add4(s, H[(size_t)j[q][n] * (kHid / 4) + c4]);
+        ++d;
+      }
+    const float f = (float)d;
+    m[q] = d ? float4{s.x / f, s.y / f, s.z / f, s.w / f} : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+}
+
+// Signs of the pre-activations of one wavefront's 16 rows: bit c of mask[row]
+// is z(row, c) > 0; pos[t][i] belongs to row 4 (lane / 16) + i, column 16 t +
+// lane % 16.  mask is one 64-bit word per row, stored as four 16-bit parts.
+__device__ __forceinline__ void put_mask(int N, int row0, int lane, const bool (&pos)[4][4],
+                                         unsigned short *__restrict__ mask) {
+  const int g = lane >> 4, part = lane & 15;
+  unsigned int mine = 0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned long long b = __ballot(pos[t][i]);
+      if (part == 4 * i + t) mine = (unsigned int)(b >> (16 * g)) & 0xffffu;
+    }
+  const int row = row0 + 4 * g + (part >> 2);
+  if (row < N) mask[4 * (size_t)row + (part & 3)] = (unsigned short)mine;
+}
+
+enum { EPI_ENC = 0, EPI_LIN = 2 };
 
 // Out[N,NO] = epi(A[N,K] W + bias); Wt = W^T in bf16, [NO][K].
 template <int K, int NO, int EPI>
-__global__ void __launch_bounds__(256) k_rowgemm(int N, const float *__restrict__ A,
+__global__ void __launch_bounds__(256) k_rowgemm(int N, const float4 *__restrict__ A,
                                                  const unsigned short *__restrict__ Wt,
-                                                 const float *__restrict__ bias, const float *__restrict__ Hin,
-                                                 float *__restrict__ Zout, float *__restrict__ Out) {
+                                                 const float *__restrict__ bias, unsigned short *__restrict__ mask,
+                                                 float *__restrict__ Out) {
   // K steps of 32 where K allows (gfx950's 16x16x32 shape), else of 16; row
   // pitch K + 8 keeps every lane's 16-byte operand aligned and the 16 rows of
   // a step on distinct LDS banks
@@ -90,9 +165,12 @@ __global__ void __launch_bounds__(256) k_rowgemm(int N, const float *__restrict_
   for (int tile = blockIdx.x; tile * kRows < N; tile += gridDim.x) {
     const int r0 = tile * kRows;
     __syncthreads();
-    for (int e = tid; e < kRows * K; e += 256) {
-      const int r = e / K, k = e % K, row = r0 + r;
-      sA[r * KP + k] = f2bf(row < N ? A[(size_t)row * K + k] : 0.0f);
+#pragma unroll
+    for (int e = tid; e < kRows * K / 4; e += 256) {
+      const int r = e / (K / 4), c4 = e % (K / 4), row = r0 + r;
+      const float4 v = row < N ? A[(size_t)row * (K / 4) + c4] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+      const bf16x4 o = {(short)f2bf(v.x), (short)f2bf(v.y), (short)f2bf(v.z), (short)f2bf(v.w)};
+      *reinterpret_cast<bf16x4 *>(&sA[r * KP + 4 * c4]) = o;
     }
     __syncthreads();
     f32x4 acc[NO / 16];
@@ -105,75 +183,101 @@ __global__ void __launch_bounds__(256) k_rowgemm(int N, const float *__restrict_
         acc[t] = mfma_tile<KS>(&sA[ar * KP + kb + kq], &sW[(t * 16 + (lane & 15)) * KP + kb + kq], acc[t]);
     }
     // lane holds rows 4*(lane/16)+i, column lane%16 of each 16x16 tile
+    [[maybe_unused]] bool pos[4][4];
 #pragma unroll
     for (int t = 0; t < NO / 16; ++t) {
       const int col = t * 16 + (lane & 15);
-      const float bc = bias ? bias[col] : 0.0f;
+      const float bc = bias[col];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int row = r0 + wave * 16 + 4 * (lane >> 4) + i;
-        if (row >= N) continue;
         const float z = acc[t][i] + bc;
-        const size_t o = (size_t)row * NO + col;
-        if (EPI == EPI_ENC) {
-          Zout[o] = z;
-          Out[o] = fmaxf(z, 0.0f);
-        } else if (EPI == EPI_MP) {
-          Zout[o] = z;
-          Out[o] = Hin[o] + fmaxf(z, 0.0f);
-        } else {
-          Out[o] = z;
-        }
+        if constexpr (EPI == EPI_ENC) pos[t][i] = z > 0.0f;
+        if (row < N) Out[(size_t)row * NO + col] = EPI == EPI_ENC ? fmaxf(z, 0.0f) : z;
       }
+    }
+    if constexpr (EPI == EPI_ENC) put_mask(N, r0 + wave * 16, lane, pos, mask);
+  }
+}
+
+// Out = H + relu([H | mean_nb H] W + b), mask = signs of the pre-activations;
+// Wt = W^T in bf16, [64][128].
+__global__ void __launch_bounds__(256) k_layer_fwd(int N, const float4 *__restrict__ H, const int *__restrict__ nb,
+                                                   const unsigned short *__restrict__ Wt,
+                                                   const float *__restrict__ bias, unsigned short *__restrict__ mask,
+                                                   float *__restrict__ Out) {
+  constexpr int K = 2 * kHid, KP = K + 8;
+  __shared__ __align__(16) unsigned short sA[kRows * KP];
+  __shared__ __align__(16) unsigned short sW[kHid * KP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rg = tid >> 4, c4 = tid & 15;
+  for (int e = tid; e < kHid * K / 8; e += 256)
+    *reinterpret_cast<bf16x8 *>(&sW[(e / (K / 8)) * KP + 8 * (e % (K / 8))]) =
+        reinterpret_cast<const bf16x8 *>(Wt)[e];
+  const int ar = wave * 16 + (lane & 15), kq = 8 * (lane >> 4);
+  const float *Hf = reinterpret_cast<const float *>(H);
+  for (int tile = blockIdx.x; tile * kRows < N; tile += gridDim.x) {
+    const int r0 = tile * kRows;
+    float4 h[4], m[4];
+    load_cat(N, r0, rg, c4, H, nb, h, m);
+    __syncthreads();  // the previous tile's operand reads
+    put_rows<KP>(sA, rg, c4, h);
+    put_rows<KP>(sA + kHid, rg, c4, m);
+    __syncthreads();
+    f32x4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kb = 0; kb < K; kb += 32)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        acc[t] = mfma_tile<32>(&sA[ar * KP + kb + kq], &sW[(t * 16 + (lane & 15)) * KP + kb + kq], acc[t]);
+    bool pos[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int col = t * 16 + (lane & 15);
+      const float bc = bias[col];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = r0 + wave * 16 + 4 * (lane >> 4) + i;
+        const float z = acc[t][i] + bc;
+        pos[t][i] = z > 0.0f;
+        const size_t o = (size_t)row * kHid + col;
+        if (row < N) Out[o] = Hf[o] + fmaxf(z, 0.0f);
+      }
+    }
+    put_mask(N, r0 + wave * 16, lane, pos, mask);
+  }
+}
+
+// Accumulates A^T B over a tile's 64 rows into this wavefront's 16x16 tiles of
+// the K x NO product; At [K][RP] and Bt [NO][RP] hold the rows contiguously.
+constexpr int kRP = kRows + 8;
+template <int K, int NO>
+constexpr int col_tiles() { return ((K / 16) * (NO / 16) + 3) / 4; }
+template <int K, int NO>
+__device__ __forceinline__ void col_product(const unsigned short *At, const unsigned short *Bt, int wave, int lane,
+                                            f32x4 (&acc)[col_tiles<K, NO>()]) {
+  constexpr int TN = NO / 16, TT = (K / 16) * TN, PER = col_tiles<K, NO>();
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int t = wave * PER + q;
+    if (t < TT) {
+      const int tm = t / TN, tn = t % TN, kq = 8 * (lane >> 4);
+#pragma unroll
+      for (int rb = 0; rb < kRows; rb += 32)
+        acc[q] = mfma_tile<32>(&At[(tm * 16 + (lane & 15)) * kRP + rb + kq],
+                               &Bt[(tn * 16 + (lane & 15)) * kRP + rb + kq], acc[q]);
     }
   }
 }
 
-// part[block][K*NO + NO]: sum over this block's rows of A[r,:]^T B[r,:], then
-// the column sums of B.
+// This workgroup's partial gradient: [K * NO] weights, then NO column sums
+// (col[c] summed over the workgroup's 16 row groups through LDS).
 template <int K, int NO>
-__global__ void __launch_bounds__(256) k_colgemm(int N, const float *__restrict__ A, const float *__restrict__ B,
-                                                 float *__restrict__ part) {
-  // the reduction runs over the tile's kRows rows in steps of 32 (16x16x32)
-  static_assert(kRows % 32 == 0, "row tile must be a multiple of 32");
-  constexpr int RP = kRows + 8;
-  constexpr int TM = K / 16, TN = NO / 16, TT = TM * TN, PER = (TT + 3) / 4;
-  __shared__ __align__(16) unsigned short sAt[K * RP];
-  __shared__ __align__(16) unsigned short sBt[NO * RP];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int kq = 8 * (lane >> 4);
-  f32x4 acc[PER];
-#pragma unroll
-  for (int q = 0; q < PER; ++q) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  float bsum = 0.0f;
-  for (int tile = blockIdx.x; tile * kRows < N; tile += gridDim.x) {
-    const int r0 = tile * kRows;
-    __syncthreads();
-    for (int e = tid; e < kRows * K; e += 256) {
-      const int r = e / K, k = e % K, row = r0 + r;
-      sAt[k * RP + r] = f2bf(row < N ? A[(size_t)row * K + k] : 0.0f);
-    }
-    for (int e = tid; e < kRows * NO; e += 256) {
-      const int r = e / NO, n = e % NO, row = r0 + r;
-      sBt[n * RP + r] = f2bf(row < N ? B[(size_t)row * NO + n] : 0.0f);
-    }
-    if (tid < NO) {
-      const int rmax = min(kRows, N - r0);
-      for (int r = 0; r < rmax; ++r) bsum += B[(size_t)(r0 + r) * NO + tid];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      const int t = wave * PER + q;
-      if (t < TT) {
-        const int tm = t / TN, tn = t % TN;
-#pragma unroll
-        for (int rb = 0; rb < kRows; rb += 32)
-          acc[q] = mfma_tile<32>(&sAt[(tm * 16 + (lane & 15)) * RP + rb + kq],
-                                 &sBt[(tn * 16 + (lane & 15)) * RP + rb + kq], acc[q]);
-      }
-    }
-  }
+__device__ __forceinline__ void put_partial(int wave, int lane, const f32x4 (&acc)[col_tiles<K, NO>()], float4 bsum,
+                                            float *red /* [16][NO] LDS */, float *__restrict__ part) {
+  constexpr int TN = NO / 16, TT = (K / 16) * TN, PER = col_tiles<K, NO>();
+  const int tid = threadIdx.x, rg = tid / (NO / 4), c4 = tid % (NO / 4);
   float *out = part + (size_t)blockIdx.x * (K * NO + NO);
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
@@ -184,88 +288,259 @@ __global__ void __launch_bounds__(256) k_colgemm(int N, const float *__restrict_
       for (int i = 0; i < 4; ++i) out[(tm * 16 + 4 * (lane >> 4) + i) * NO + tn * 16 + (lane & 15)] = acc[q][i];
     }
   }
-  if (tid < NO) out[K * NO + tid] = bsum;
-}
-
-// out[e] = sum over parts p (in order) of part[p * len + e]
-__global__ void __launch_bounds__(256) k_reduce_parts(int nparts, int len, const float *__restrict__ part,
-                                                      float *__restrict__ out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= len) return;
-  float s = 0.0f;
-  for (int p = 0; p < nparts; ++p) s += part[(size_t)p * len + e];
-  out[e] = s;
-}
-
-// Cat[i] = [H[i] | mean over valid neighbours of H[j]]  (H: [N,64], Cat: [N,128])
-__global__ void __launch_bounds__(256) k_concat_mean(int N, const float *__restrict__ H, const int *__restrict__ nb,
-                                                     float *__restrict__ Cat) {
-  const long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (e >= (long)N * kHid) return;
-  const int i = (int)(e / kHid), c = (int)(e % kHid);
-  float s = 0.0f;
-  int d = 0;
-#pragma unroll
-  for (int n = 0; n < 3; ++n) {
-    const int j = nb[3 * i + n];
-    if (j >= 0) { s += H[(size_t)j * kHid + c]; ++d; }
+  constexpr int RG = 256 / (NO / 4);  // row groups
+  __syncthreads();
+  *reinterpret_cast<float4 *>(&red[rg * NO + 4 * c4]) = bsum;
+  __syncthreads();
+  if (tid < NO) {
+    float t = 0.0f;
+    for (int q = 0; q < RG; ++q) t += red[q * NO + tid];
+    out[K * NO + tid] = t;
   }
-  Cat[(size_t)i * 2 * kHid + c] = H[e];
-  Cat[(size_t)i * 2 * kHid + kHid + c] = d ? s / d : 0.0f;
 }
 
-// dZ = dH * (Z > 0)
-__global__ void __launch_bounds__(256) k_relu_back(long n, const float *__restrict__ dH, const float *__restrict__ Z,
-                                                   float *__restrict__ dZ) {
-  const long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (e < n) dZ[e] = Z[e] > 0.0f ? dH[e] : 0.0f;
-}
-
-// dH[j] += dCat[j, 0:64] + sum_{i in nb(j)} dCat[i, 64:128] / deg(i)
-// (adjoint of k_concat_mean for symmetric neighbour lists)
-__global__ void __launch_bounds__(256) k_dh_update(int N, const float *__restrict__ dCat, const int *__restrict__ nb,
-                                                   float *__restrict__ dH) {
-  const long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (e >= (long)N * kHid) return;
-  const int j = (int)(e / kHid), c = (int)(e % kHid);
-  float s = dH[e] + dCat[(size_t)j * 2 * kHid + c];
-#pragma unroll
-  for (int n = 0; n < 3; ++n) {
-    const int i = nb[3 * j + n];
-    if (i < 0) continue;
-    int d = 0;
-#pragma unroll
-    for (int m = 0; m < 3; ++m) d += nb[3 * i + m] >= 0;
-    s += dCat[(size_t)i * 2 * kHid + kHid + c] / (float)d;
-  }
-  dH[e] = s;
-}
-
-// dY = 2 (Y[:, 0:3] - T) / N (other columns 0); per-block partial sums of the
-// squared error into part[blockIdx]
-__global__ void __launch_bounds__(256) k_loss_dy(int N, const float *__restrict__ Y, const float *__restrict__ T,
-                                                 float *__restrict__ dY, float *__restrict__ part) {
-  __shared__ float red[256];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Loss, decoder gradient and dH of the last layer: dY = 2 (Y[:, 0:3] - T) / N
+// (other columns 0), partial sums of Wd's gradient H^T dY and of the squared
+// error, dH = dY Wd^T.  Wn = Wd in bf16, [64][16].
+__global__ void __launch_bounds__(256) k_decoder_back(int N, const float4 *__restrict__ Y, const float *__restrict__ T,
+                                                      const float4 *__restrict__ H,
+                                                      const unsigned short *__restrict__ Wn, float *__restrict__ dH,
+                                                      float *__restrict__ part, float *__restrict__ lpart) {
+  constexpr int YP = kFout + 8;
+  __shared__ __align__(16) unsigned short sY[kRows * YP], sYt[kFout * kRP], sHt[kHid * kRP], sW[kHid * YP];
+  __shared__ __align__(16) float red[64 * kFout];
+  __shared__ float sl[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rg = tid >> 4, c4 = tid & 15;
+  for (int e = tid; e < kHid * kFout; e += 256) sW[(e / kFout) * YP + (e % kFout)] = Wn[e];
+  const float s = 2.0f / (float)N;
+  f32x4 acc[col_tiles<kHid, kFout>()];
+  acc[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 bsum{0.0f, 0.0f, 0.0f, 0.0f};
   float se = 0.0f;
-  if (i < N) {
-    const float s = 2.0f / (float)N;
+  for (int tile = blockIdx.x; tile * kRows < N; tile += gridDim.x) {
+    const int r0 = tile * kRows;
+    float4 h[4];
 #pragma unroll
-    for (int c = 0; c < kTargets; ++c) {
-      const float d = Y[(size_t)i * kFout + c] - T[(size_t)kTargets * i + c];
-      se += d * d;
-      dY[(size_t)i * kFout + c] = s * d;
+    for (int q = 0; q < 4; ++q) {
+      const int row = r0 + 4 * rg + q;
+      h[q] = row < N ? H[(size_t)row * (kHid / 4) + c4] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    // one thread per (row, four outputs)
+    const int yr = tid >> 2, yc = tid & 3, yrow = r0 + yr;
+    float4 d{0.0f, 0.0f, 0.0f, 0.0f};
+    if (yc == 0 && yrow < N) {
+      const float4 y = Y[(size_t)yrow * (kFout / 4)];
+      const float *t = T + (size_t)kTargets * yrow;
+      const float d0 = y.x - t[0], d1 = y.y - t[1], d2 = y.z - t[2];
+      se += d0 * d0 + d1 * d1 + d2 * d2;
+      d = float4{s * d0, s * d1, s * d2, 0.0f};
+    }
+    add4(bsum, d);
+    __syncthreads();
+    put_cols<kRP>(sHt, rg, c4, h);
+    const unsigned short b0 = f2bf(d.x), b1 = f2bf(d.y), b2 = f2bf(d.z), b3 = f2bf(d.w);
+    const bf16x4 o = {(short)b0, (short)b1, (short)b2, (short)b3};
+    *reinterpret_cast<bf16x4 *>(&sY[yr * YP + 4 * yc]) = o;
+    sYt[(4 * yc + 0) * kRP + yr] = b0;
+    sYt[(4 * yc + 1) * kRP + yr] = b1;
+    sYt[(4 * yc + 2) * kRP + yr] = b2;
+    sYt[(4 * yc + 3) * kRP + yr] = b3;
+    __syncthreads();
+    col_product<kHid, kFout>(sHt, sYt, wave, lane, acc);
+#pragma unroll
+    for (int t = 0; t < kHid / 16; ++t) {
+      const f32x4 z = mfma_tile<16>(&sY[(wave * 16 + (lane & 15)) * YP + 4 * (lane >> 4)],
+                                    &sW[(t * 16 + (lane & 15)) * YP + 4 * (lane >> 4)], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = r0 + wave * 16 + 4 * (lane >> 4) + i;
+        if (row < N) dH[(size_t)row * kHid + t * 16 + (lane & 15)] = z[i];
+      }
+    }
+  }
+  se = wave_sum(se);
+  if (lane == 0) sl[wave] = se;
+  put_partial<kHid, kFout>(wave, lane, acc, bsum, red, part);
+  if (tid == 0) lpart[blockIdx.x] = sl[0] + sl[1] + sl[2] + sl[3];
+}
+
+// dH of the rows r0 + 4 rg .. + 3: the own part plus, from the second layer on,
+// the neighbours' parts G (already divided by their degrees) in list order.
+template <bool HAS_G>
+__device__ __forceinline__ void load_dh(int N, int r0, int rg, int c4, const float4 *__restrict__ dH,
+                                        const float4 *__restrict__ G, const int *__restrict__ nb, float4 (&v)[4]) {
+  int j[4][3];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int row = r0 + 4 * rg + q;
+    v[q] = row < N ? dH[(size_t)row * (kHid / 4) + c4] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (HAS_G)
+#pragma unroll
+      for (int n = 0; n < 3; ++n) j[q][n] = row < N ? nb[3 * row + n] : -1;
+  }
+  if (HAS_G)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int n = 0; n < 3; ++n)
+        if (j[q][n] >= 0) add4(v[q], G[(size_t)j[q][n] * (kHid / 4) + c4]);
+}
+
+// dZ = dH where the pre-activation was positive
+__device__ __forceinline__ void apply_mask(int N, int r0, int rg, int c4, const unsigned short *__restrict__ mask,
+                                           float4 (&v)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int row = r0 + 4 * rg + q;
+    const unsigned int b = row < N ? mask[4 * (size_t)row + (c4 >> 2)] >> (4 * (c4 & 3)) : 0u;
+    v[q].x = b & 1u ? v[q].x : 0.0f;
+    v[q].y = b & 2u ? v[q].y : 0.0f;
+    v[q].z = b & 4u ? v[q].z : 0.0f;
+    v[q].w = b & 8u ? v[q].w : 0.0f;
+  }
+}
+
+// One layer backward (file comment).  Wn = W in bf16, [128][64]; dHout = dH +
+// dCat[:, 0:64], Gout = dCat[:, 64:128] / degree.
+template <bool HAS_G>
+__global__ void __launch_bounds__(256) k_layer_back(int N, const float4 *__restrict__ dH, const float4 *__restrict__ G,
+                                                    const int *__restrict__ nb,
+                                                    const unsigned short *__restrict__ mask,
+                                                    const float4 *__restrict__ H,
+                                                    const unsigned short *__restrict__ Wn, float *__restrict__ dHout,
+                                                    float *__restrict__ Gout, float *__restrict__ part) {
+  constexpr int K = 2 * kHid, ZP = kHid + 8, DP = kHid + 4;
+  __shared__ __align__(16) unsigned short sW[K * ZP], sZ[kRows * ZP], sZt[kHid * kRP], sCt[K * kRP];
+  __shared__ __align__(16) float sD[kRows * DP];
+  __shared__ float sdeg[kRows];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rg = tid >> 4, c4 = tid & 15;
+  for (int e = tid; e < K * kHid / 8; e += 256)
+    *reinterpret_cast<bf16x8 *>(&sW[(e / (kHid / 8)) * ZP + 8 * (e % (kHid / 8))]) =
+        reinterpret_cast<const bf16x8 *>(Wn)[e];
+  f32x4 acc[col_tiles<K, kHid>()];
+#pragma unroll
+  for (int q = 0; q < col_tiles<K, kHid>(); ++q) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 bsum{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int tile = blockIdx.x; tile * kRows < N; tile += gridDim.x) {
+    const int r0 = tile * kRows;
+    float4 v[4], h[4], m[4];
+    load_dh<HAS_G>(N, r0, rg, c4, dH, G, nb, v);
+    load_cat(N, r0, rg, c4, H, nb, h, m);
+    __syncthreads();  // the previous tile's reads
+    if (tid < kRows) {
+      const int row = r0 + tid;
+      int d = 0;
+      if (row < N)
+        for (int n = 0; n < 3; ++n) d += nb[3 * row + n] >= 0;
+      sdeg[tid] = (float)d;
     }
 #pragma unroll
-    for (int c = kTargets; c < kFout; ++c) dY[(size_t)i * kFout + c] = 0.0f;
-  }
-  red[threadIdx.x] = se;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<float4 *>(&sD[(4 * rg + q) * DP + 4 * c4]) = v[q];
+    apply_mask(N, r0, rg, c4, mask, v);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) add4(bsum, v[q]);
+    put_rows<ZP>(sZ, rg, c4, v);
+    put_cols<kRP>(sZt, rg, c4, v);
+    put_cols<kRP>(sCt, rg, c4, h);
+    put_cols<kRP>(sCt + kHid * kRP, rg, c4, m);
     __syncthreads();
+    col_product<K, kHid>(sCt, sZt, wave, lane, acc);
+    const int ar = wave * 16 + (lane & 15), kq = 8 * (lane >> 4);
+#pragma unroll
+    for (int t = 0; t < K / 16; ++t) {
+      f32x4 z = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kb = 0; kb < kHid; kb += 32)
+        z = mfma_tile<32>(&sZ[ar * ZP + kb + kq], &sW[(t * 16 + (lane & 15)) * ZP + kb + kq], z);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = wave * 16 + 4 * (lane >> 4) + i, row = r0 + r;
+        if (row >= N) continue;
+        if (t < kHid / 16) {
+          const int c = t * 16 + (lane & 15);
+          dHout[(size_t)row * kHid + c] = sD[r * DP + c] + z[i];
+        } else {
+          // a node without neighbours is read by none
+          Gout[(size_t)row * kHid + (t - kHid / 16) * 16 + (lane & 15)] = sdeg[r] > 0.0f ? z[i] / sdeg[r] : 0.0f;
+        }
+      }
+    }
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+  put_partial<K, kHid>(wave, lane, acc, bsum, sD, part);
+}
+
+// Encoder gradient: dZ from the first layer's dH, X^T dZ and its column sums.
+__global__ void __launch_bounds__(256) k_encoder_back(int N, const float4 *__restrict__ dH,
+                                                      const float4 *__restrict__ G, const int *__restrict__ nb,
+                                                      const unsigned short *__restrict__ mask,
+                                                      const float4 *__restrict__ X, float *__restrict__ part) {
+  __shared__ __align__(16) unsigned short sXt[kFin * kRP], sZt[kHid * kRP];
+  __shared__ __align__(16) float red[16 * kHid];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rg = tid >> 4, c4 = tid & 15;
+  f32x4 acc[col_tiles<kFin, kHid>()];
+  acc[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 bsum{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int tile = blockIdx.x; tile * kRows < N; tile += gridDim.x) {
+    const int r0 = tile * kRows;
+    float4 v[4];
+    load_dh<true>(N, r0, rg, c4, dH, G, nb, v);
+    apply_mask(N, r0, rg, c4, mask, v);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) add4(bsum, v[q]);
+    const int xr = tid >> 2, xc = tid & 3;
+    const float4 x = r0 + xr < N ? X[(size_t)(r0 + xr) * (kFin / 4) + xc] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+    __syncthreads();
+    put_cols<kRP>(sZt, rg, c4, v);
+    sXt[(4 * xc + 0) * kRP + xr] = f2bf(x.x);
+    sXt[(4 * xc + 1) * kRP + xr] = f2bf(x.y);
+    sXt[(4 * xc + 2) * kRP + xr] = f2bf(x.z);
+    sXt[(4 * xc + 3) * kRP + xr] = f2bf(x.w);
+    __syncthreads();
+    col_product<kFin, kHid>(sXt, sZt, wave, lane, acc);
+  }
+  put_partial<kFin, kHid>(wave, lane, acc, bsum, red, part);
+}
+
+// Sum over the workgroups' partials part[p * len + e]: elements below n go to
+// w[e], the rest to b[e - n].  A wavefront takes 64 elements of every 16th
+// partial, the 16 sums are added in order.
+constexpr int kReduceWaves = 16;
+__global__ void __launch_bounds__(64 * kReduceWaves) k_reduce_parts(int nparts, int len, int n,
+                                                                    const float *__restrict__ part,
+                                                                    float *__restrict__ w, float *__restrict__ b) {
+  __shared__ float red[kReduceWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = blockIdx.x * 64 + lane;
+  float s = 0.0f;
+  if (e < len) {
+#pragma unroll 8
+    for (int p = wave; p < nparts; p += kReduceWaves) s += part[(size_t)p * len + e];
+  }
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && e < len) {
+    float t = 0.0f;
+    for (int q = 0; q < kReduceWaves; ++q) t += red[q][lane];
+    if (e < n) w[e] = t;
+    else b[e - n] = t;
+  }
+}
+
+// Neighbour lists must be symmetric (j in nb(i) <=> i in nb(j)) and in range:
+// the gathers rely on it, so this runs before any of them.
+__global__ void __launch_bounds__(256) k_check_graph(int N, const int *__restrict__ nb, int *__restrict__ bad) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  bool ok = true;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int j = nb[3 * i + a];
+    if (j < -1 || j >= N) {
+      ok = false;
+    } else if (j >= 0) {
+      ok = ok && (nb[3 * j] == i || nb[3 * j + 1] == i || nb[3 * j + 2] == i);
+    }
+  }
+  if (!ok) *bad = 1;
 }
 
 // W [K, NO] fp32 -> Wt [NO][K] bf16 (forward operand) and Wn [K][NO] bf16
@@ -314,7 +589,11 @@ struct Layout {
   }
 };
 
-inline int grid_rows(int N) { return std::max(1, std::min((N + kRows - 1) / kRows, 1024)); }
+// persistent workgroups of the tile kernels: two per CU fit beside k_layer_back's
+// 78 KB of LDS, and each adds one partial gradient to sum
+constexpr int kMaxParts = 512;
+inline int grid_rows(int N) { return std::max(1, std::min((N + kRows - 1) / kRows, 4 * kMaxParts)); }
+inline int grid_parts(int N) { return std::min(grid_rows(N), kMaxParts); }
 inline int grid_elems(long n) { return (int)std::max<long>(1, (n + 255) / 256); }
 
 }  // namespace mp
@@ -331,8 +610,12 @@ struct ufe_mpnn {
   int step = 0;
   // graph buffers (sized for the largest N seen)
   int cap = 0;
-  DBuf X, nb, T, Ze, H[kLayers + 1], Z[kLayers], Cat[kLayers], Y, dY, dH, dZ, dCat, lpart;
+  DBuf X, nb, T, H[kLayers + 1], mask[kLayers + 1], Y, dH[2], G[2], lpart;
+  int *bad = nullptr;  // pinned: set by the graph check
   std::string err;
+  ~ufe_mpnn() {
+    if (bad) (void)hipHostFree(bad);
+  }
 
   size_t wt_off(size_t woff) const { return woff; }  // bf16 copies share the fp32 offsets
 
@@ -343,16 +626,12 @@ struct ufe_mpnn {
     X.alloc(n * kFin * 4);
     nb.alloc(n * 3 * 4);
     T.alloc(n * kTargets * 4);
-    Ze.alloc(n * kHid * 4);
     for (auto &b : H) b.alloc(n * kHid * 4);
-    for (auto &b : Z) b.alloc(n * kHid * 4);
-    for (auto &b : Cat) b.alloc(n * 2 * kHid * 4);
+    for (auto &b : mask) b.alloc(n * kHid / 8);
     Y.alloc(n * kFout * 4);
-    dY.alloc(n * kFout * 4);
-    dH.alloc(n * kHid * 4);
-    dZ.alloc(n * kHid * 4);
-    dCat.alloc(n * 2 * kHid * 4);
-    lpart.alloc(((n + 255) / 256) * 4);
+    for (auto &b : dH) b.alloc(n * kHid * 4);
+    for (auto &b : G) b.alloc(n * kHid * 4);
+    lpart.alloc(kMaxParts * 4);
   }
 
   void refresh_bf16() {
@@ -372,75 +651,62 @@ struct ufe_mpnn {
 
   // forward over N nodes already in X / nb
   void forward(int N) {
-    float *x = X.as<float>();
     const int *n3 = nb.as<int>();
     const int gr = grid_rows(N);
-    hipLaunchKernelGGL((k_rowgemm<kFin, kHid, EPI_ENC>), dim3(gr), dim3(256), 0, s, N, x, wt(L.We), wf(L.be),
-                       (const float *)nullptr, Ze.as<float>(), H[0].as<float>());
+    hipLaunchKernelGGL((k_rowgemm<kFin, kHid, EPI_ENC>), dim3(gr), dim3(256), 0, s, N, X.as<float4>(), wt(L.We),
+                       wf(L.be), mask[0].as<unsigned short>(), H[0].as<float>());
     UFE_LAUNCH_CHECK();
     for (int l = 0; l < kLayers; ++l) {
-      hipLaunchKernelGGL(k_concat_mean, dim3(grid_elems((long)N * kHid)), dim3(256), 0, s, N, H[l].as<float>(), n3,
-                         Cat[l].as<float>());
-      UFE_LAUNCH_CHECK();
-      hipLaunchKernelGGL((k_rowgemm<2 * kHid, kHid, EPI_MP>), dim3(gr), dim3(256), 0, s, N, Cat[l].as<float>(),
-                         wt(L.W[l]), wf(L.b[l]), H[l].as<float>(), Z[l].as<float>(), H[l + 1].as<float>());
+      hipLaunchKernelGGL(k_layer_fwd, dim3(gr), dim3(256), 0, s, N, H[l].as<float4>(), n3, wt(L.W[l]), wf(L.b[l]),
+                         mask[l + 1].as<unsigned short>(), H[l + 1].as<float>());
       UFE_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL((k_rowgemm<kHid, kFout, EPI_LIN>), dim3(gr), dim3(256), 0, s, N, H[kLayers].as<float>(),
-                       wt(L.Wd), wf(L.bd), (const float *)nullptr, (float *)nullptr, Y.as<float>());
+    hipLaunchKernelGGL((k_rowgemm<kHid, kFout, EPI_LIN>), dim3(gr), dim3(256), 0, s, N, H[kLayers].as<float4>(),
+                       wt(L.Wd), wf(L.bd), (unsigned short *)nullptr, Y.as<float>());
     UFE_LAUNCH_CHECK();
   }
 
-  template <int K, int NO>
-  void weight_grad(int N, const float *A, const float *B, size_t woff, size_t boff) {
-    const int gr = grid_rows(N);
+  // gradient of a K x NO weight block and its bias from the workgroups' partials
+  void reduce(int nparts, int K, int NO, size_t woff, size_t boff) {
     const int len = K * NO + NO;
-    hipLaunchKernelGGL((k_colgemm<K, NO>), dim3(gr), dim3(256), 0, s, N, A, B, part.as<float>());
+    hipLaunchKernelGGL(k_reduce_parts, dim3((len + 63) / 64), dim3(64 * kReduceWaves), 0, s, nparts, len, K * NO,
+                       part.as<float>(), g.as<float>() + woff, g.as<float>() + boff);
     UFE_LAUNCH_CHECK();
-    // the weight block and the bias follow each other in the partials; reduce
-    // them into a contiguous scratch then scatter into the gradient layout
-    float *tmp = part.as<float>() + (size_t)1024 * (2 * kHid * kHid + kHid);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(grid_elems(len)), dim3(256), 0, s, gr, len, part.as<float>(), tmp);
-    UFE_LAUNCH_CHECK();
-    UFE_HIP(hipMemcpyAsync(g.as<float>() + woff, tmp, sizeof(float) * K * NO, hipMemcpyDeviceToDevice, s));
-    UFE_HIP(hipMemcpyAsync(g.as<float>() + boff, tmp + K * NO, sizeof(float) * NO, hipMemcpyDeviceToDevice, s));
   }
 
   // loss and gradient for the N nodes in X / nb / T; returns the loss
   float loss_grad(int N) {
     forward(N);
-    const int nbk = grid_elems(N);
-    hipLaunchKernelGGL(k_loss_dy, dim3(nbk), dim3(256), 0, s, N, Y.as<float>(), T.as<float>(), dY.as<float>(),
-                       lpart.as<float>());
+    const int gp = grid_parts(N);
+    const int *n3 = nb.as<int>();
+    float *pt = part.as<float>();
+    hipLaunchKernelGGL(k_decoder_back, dim3(gp), dim3(256), 0, s, N, Y.as<float4>(), T.as<float>(),
+                       H[kLayers].as<float4>(), wn(L.Wd), dH[0].as<float>(), pt, lpart.as<float>());
     UFE_LAUNCH_CHECK();
-    const int gr = grid_rows(N);
-    // decoder
-    weight_grad<kHid, kFout>(N, H[kLayers].as<float>(), dY.as<float>(), L.Wd, L.bd);
-    hipLaunchKernelGGL((k_rowgemm<kFout, kHid, EPI_LIN>), dim3(gr), dim3(256), 0, s, N, dY.as<float>(), wn(L.Wd),
-                       (const float *)nullptr, (const float *)nullptr, (float *)nullptr, dH.as<float>());
-    UFE_LAUNCH_CHECK();
-    for (int l = kLayers - 1; l >= 0; --l) {
-      hipLaunchKernelGGL(k_relu_back, dim3(grid_elems((long)N * kHid)), dim3(256), 0, s, (long)N * kHid,
-                         dH.as<float>(), Z[l].as<float>(), dZ.as<float>());
+    reduce(gp, kHid, kFout, L.Wd, L.bd);
+    int cur = 0;
+    for (int l = kLayers - 1; l >= 0; --l, cur ^= 1) {
+      const unsigned short *mk = mask[l + 1].as<unsigned short>();
+      if (l == kLayers - 1)
+        hipLaunchKernelGGL(k_layer_back<false>, dim3(gp), dim3(256), 0, s, N, dH[cur].as<float4>(),
+                           (const float4 *)nullptr, n3, mk, H[l].as<float4>(), wn(L.W[l]), dH[cur ^ 1].as<float>(),
+                           G[cur ^ 1].as<float>(), pt);
+      else
+        hipLaunchKernelGGL(k_layer_back<true>, dim3(gp), dim3(256), 0, s, N, dH[cur].as<float4>(),
+                           G[cur].as<float4>(), n3, mk, H[l].as<float4>(), wn(L.W[l]), dH[cur ^ 1].as<float>(),
+                           G[cur ^ 1].as<float>(), pt);
       UFE_LAUNCH_CHECK();
-      weight_grad<2 * kHid, kHid>(N, Cat[l].as<float>(), dZ.as<float>(), L.W[l], L.b[l]);
-      hipLaunchKernelGGL((k_rowgemm<kHid, 2 * kHid, EPI_LIN>), dim3(gr), dim3(256), 0, s, N, dZ.as<float>(),
-                         wn(L.W[l]), (const float *)nullptr, (const float *)nullptr, (float *)nullptr,
-                         dCat.as<float>());
-      UFE_LAUNCH_CHECK();
-      hipLaunchKernelGGL(k_dh_update, dim3(grid_elems((long)N * kHid)), dim3(256), 0, s, N, dCat.as<float>(),
-                         nb.as<int>(), dH.as<float>());
-      UFE_LAUNCH_CHECK();
+      reduce(gp, 2 * kHid, kHid, L.W[l], L.b[l]);
     }
-    hipLaunchKernelGGL(k_relu_back, dim3(grid_elems((long)N * kHid)), dim3(256), 0, s, (long)N * kHid,
-                       dH.as<float>(), Ze.as<float>(), dZ.as<float>());
+    hipLaunchKernelGGL(k_encoder_back, dim3(gp), dim3(256), 0, s, N, dH[cur].as<float4>(), G[cur].as<float4>(), n3,
+                       mask[0].as<unsigned short>(), X.as<float4>(), pt);
     UFE_LAUNCH_CHECK();
-    weight_grad<kFin, kHid>(N, X.as<float>(), dZ.as<float>(), L.We, L.be);
-    std::vector<float> lp(nbk);
-    UFE_HIP(hipMemcpyAsync(lp.data(), lpart.p, sizeof(float) * nbk, hipMemcpyDeviceToHost, s));
+    reduce(gp, kFin, kHid, L.We, L.be);
+    float lp[kMaxParts];
+    UFE_HIP(hipMemcpyAsync(lp, lpart.p, sizeof(float) * gp, hipMemcpyDeviceToHost, s));
     UFE_HIP(hipStreamSynchronize(s));
     double tot = 0.0;
-    for (float x : lp) tot += x;
+    for (int i = 0; i < gp; ++i) tot += lp[i];
     return (float)(tot / N);
   }
 
@@ -459,6 +725,15 @@ struct ufe_mpnn {
     UFE_HIP(hipMemcpyAsync(X.p, Xh, sizeof(float) * kFin * (size_t)N, hipMemcpyHostToDevice, s));
     UFE_HIP(hipMemcpyAsync(nb.p, nbh, sizeof(int) * 3 * (size_t)N, hipMemcpyHostToDevice, s));
     if (Th) UFE_HIP(hipMemcpyAsync(T.p, Th, sizeof(float) * kTargets * (size_t)N, hipMemcpyHostToDevice, s));
+  }
+
+  // whether the neighbour lists in nb are in range and symmetric
+  bool graph_ok(int N) {
+    *bad = 0;
+    hipLaunchKernelGGL(k_check_graph, dim3(grid_elems(N)), dim3(256), 0, s, N, nb.as<int>(), bad);
+    UFE_LAUNCH_CHECK();
+    UFE_HIP(hipStreamSynchronize(s));
+    return *bad == 0;
   }
 };
 
@@ -481,20 +756,7 @@ int mp_guard(ufe_mpnn *n, F &&f) {
   }
 }
 
-// Neighbour lists must be symmetric (j in nb(i) <=> i in nb(j)) and in range:
-// the backward gather relies on it.
-bool valid_graph(int N, const int *nb) {
-  for (int i = 0; i < N; ++i)
-    for (int a = 0; a < 3; ++a) {
-      int j = nb[3 * i + a];
-      if (j < -1 || j >= N) return false;
-      if (j < 0) continue;
-      bool back = false;
-      for (int b = 0; b < 3; ++b) back |= nb[3 * j + b] == i;
-      if (!back) return false;
-    }
-  return true;
-}
+constexpr const char *kBadGraph = "neighbour lists must be in range and symmetric";
 
 }  // namespace
 
@@ -514,9 +776,9 @@ extern "C" int ufe_mpnn_create(ufe_mpnn **out, int device, const float *weights)
     n->v.alloc(P * 4);
     n->wt16.alloc(P * 2);
     n->wn16.alloc(P * 2);
-    // partials: up to 1024 workgroups x the largest block (128x64 + 64), plus
-    // a reduction target after them
-    n->part.alloc(sizeof(float) * (size_t)1025 * (2 * kHid * kHid + kHid));
+    // partials: the largest block (128x64 + 64) of every workgroup
+    n->part.alloc(sizeof(float) * (size_t)kMaxParts * (2 * kHid * kHid + kHid));
+    UFE_HIP(hipHostMalloc((void **)&n->bad, sizeof(int), hipHostMallocDefault));
     UFE_HIP(hipMemsetAsync(n->g.p, 0, P * 4, n->s));
     UFE_HIP(hipMemsetAsync(n->m.p, 0, P * 4, n->s));
     UFE_HIP(hipMemsetAsync(n->v.p, 0, P * 4, n->s));
@@ -553,10 +815,10 @@ extern "C" int ufe_mpnn_get_weights(ufe_mpnn *n, float *weights) {
 
 extern "C" int ufe_mpnn_forward(ufe_mpnn *n, int N, const float *X, const int *nb, float *Y) {
   if (!n || N < 1 || !X || !nb || !Y) return mp_fail(n, UFE_ERR_ARGUMENT, "invalid argument");
-  if (!valid_graph(N, nb)) return mp_fail(n, UFE_ERR_ARGUMENT, "neighbour lists must be in range and symmetric");
   return mp_guard(n, [&]() -> int {
     UFE_HIP(hipSetDevice(n->device));
     n->upload_graph(N, X, nb, nullptr);
+    if (!n->graph_ok(N)) return mp_fail(n, UFE_ERR_ARGUMENT, kBadGraph);
     n->forward(N);
     UFE_HIP(hipMemcpyAsync(Y, n->Y.p, sizeof(float) * kFout * (size_t)N, hipMemcpyDeviceToHost, n->s));
     UFE_HIP(hipStreamSynchronize(n->s));
@@ -567,10 +829,10 @@ extern "C" int ufe_mpnn_forward(ufe_mpnn *n, int N, const float *X, const int *n
 extern "C" int ufe_mpnn_loss_grad(ufe_mpnn *n, int N, const float *X, const int *nb, const float *T, float *loss,
                                   float *grad) {
   if (!n || N < 1 || !X || !nb || !T || !loss) return mp_fail(n, UFE_ERR_ARGUMENT, "invalid argument");
-  if (!valid_graph(N, nb)) return mp_fail(n, UFE_ERR_ARGUMENT, "neighbour lists must be in range and symmetric");
   return mp_guard(n, [&]() -> int {
     UFE_HIP(hipSetDevice(n->device));
     n->upload_graph(N, X, nb, T);
+    if (!n->graph_ok(N)) return mp_fail(n, UFE_ERR_ARGUMENT, kBadGraph);
     *loss = n->loss_grad(N);
     if (grad) {
       UFE_HIP(hipMemcpyAsync(grad, n->g.p, n->L.total * 4, hipMemcpyDeviceToHost, n->s));
@@ -584,10 +846,10 @@ extern "C" int ufe_mpnn_train(ufe_mpnn *n, int N, const float *X, const int *nb,
                               float lr, float *loss_history) {
   if (!n || N < 1 || !X || !nb || !T || steps < 0 || !(lr > 0.0f))
     return mp_fail(n, UFE_ERR_ARGUMENT, "invalid argument");
-  if (!valid_graph(N, nb)) return mp_fail(n, UFE_ERR_ARGUMENT, "neighbour lists must be in range and symmetric");
   return mp_guard(n, [&]() -> int {
     UFE_HIP(hipSetDevice(n->device));
     n->upload_graph(N, X, nb, T);
+    if (!n->graph_ok(N)) return mp_fail(n, UFE_ERR_ARGUMENT, kBadGraph);
     for (int it = 0; it < steps; ++it) {
       float l = n->loss_grad(N);
       if (loss_history) loss_history[it] = l;
