@@ -491,6 +491,24 @@ def test_heat_columns_parity(V, OB, W, nV, nz):
     assert np.abs(T - To).max() < 1e-9
 
 
+@pytest.mark.parametrize("nV,nz", [(1, 3), (63, 8), (65, 9), (129, 16), (200, 17), (64, 32), (530_001, 4)])
+def test_heat_columns_at_the_edges_of_their_range(V, OB, W, dome, nV, nz):
+    """Fewer columns than a wavefront, one more, more than the grid takes at
+    once; the layer counts where the unrolled kernel changes; uneven layers
+    (the zeta operators are formed on the device); with and without a context.
+    Bound as above (FP64, same recurrences)."""
+    c = W.heat_columns_inputs(nV, nz, seed=nV % 7, gl=0.2)
+    hin, keep = V.make_heat_inputs(nV, nz, c["zeta"] ** 1.4, c["fields"], c["dt"])
+    T, un, n = V.heat_columns(hin)
+    s = V.VelocitySolver(dome.descriptor())
+    Tc, unc, nc = V.heat_columns(hin, s)
+    s.close()
+    rc, To, uo, no = OB.heat_columns(hin)
+    assert rc == 0 and n == no == nc and np.array_equal(un, uo)
+    assert np.array_equal(T, Tc) and np.array_equal(un, unc)
+    assert np.abs(T - To).max() < 1e-9
+
+
 @pytest.mark.parametrize("nz", [12, 30])
 def test_heat_grounding_line_blend_matches_oracle(V, W, OB, nz):
     """Grounding-line columns blended with fraction_gr ('subgrid') equal the

@@ -139,9 +139,9 @@ struct HeatDev {
   const int *mask;
   const double *fgr;  // [nV] vertex grounded fraction, read where mask = 3 (may be null otherwise)
   double dt, Hi_min;
-  const double *tri;  // [6][nz] d/dzeta and d2/dzeta2 tridiagonals (ldiag, diag, udiag)
 };
-void launch_heat_columns(const HeatDev &h, double *Tout, int *unstable, const RedSlot &slot, double *count,
+// counts (unstable, invalid mask) into slot.result, and into host memory when given
+void launch_heat_columns(const HeatDev &h, double *Tout, int *unstable, const RedSlot &slot, double *host,
                          hipStream_t s);
 
 }  // namespace ufe

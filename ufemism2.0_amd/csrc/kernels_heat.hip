@@ -186,6 +186,39 @@ __device__ __forceinline__ void heat_step(const HeatDev &h, const double *__rest
   }
 }
 
+// Row k of the zeta tridiagonals (tri[6][kHeatMaxNz]: lower, diagonal and upper
+// of d/dzeta, then of d2/dzeta2; the off-diagonal ones at the entry's own
+// layer, lower ones at k - 1): calc_vertical_operators_reg_1D
+// (mesh_zeta.f90:287-365) with 1-D 2nd-order shape functions
+// (shape_functions.f90:17-79), then the tridiagonal extraction of
+// calc_zeta_operators_tridiagonal (:487-605).  Every workgroup forms them
+// itself (one lane per layer), so a call with device arrays copies nothing to
+// the host first; with the counts written to host memory by k_heat_count it
+// makes no copy at all.  ufe_heat_columns_device: 399,156 x 12 columns 154 ->
+// 121 us (the column kernel 98 us: 4.2 TB/s of its 412 MB, against 5.2 TB/s for
+// a plain copy), 3,000 x 12 columns 59 -> 26 us.
+__device__ __forceinline__ void zeta_tridiagonal_row(int nz, int k, const double *__restrict__ z, double *tri,
+                                                     double *zeta) {
+  const int c0 = k == 0 ? 1 : k == nz - 1 ? nz - 3 : k - 1, c1 = k == 0 ? 2 : k == nz - 1 ? nz - 2 : k + 1;
+  const double zk = z[k], d0 = z[c0] - zk, d1 = z[c1] - zk;
+  // squared weights |d|^-3
+  const double w0 = 1.0 / fabs(d0 * d0 * d0), w1 = 1.0 / fabs(d1 * d1 * d1);
+  const double a = w0 * d0 * d0 + w1 * d1 * d1;
+  const double b = 0.5 * (w0 * d0 * d0 * d0 + w1 * d1 * d1 * d1);
+  const double c = 0.25 * (w0 * d0 * d0 * d0 * d0 + w1 * d1 * d1 * d1 * d1);
+  const double det = a * c - b * b;
+  const double m0 = c / det, m1 = -b / det, m3 = a / det;
+  const double x0 = w0 * (m0 * d0 + m1 * 0.5 * d0 * d0), x1 = w1 * (m0 * d1 + m1 * 0.5 * d1 * d1);
+  const double y0 = w0 * (m1 * d0 + m3 * 0.5 * d0 * d0), y1 = w1 * (m1 * d1 + m3 * 0.5 * d1 * d1);
+  zeta[k] = zk;
+  tri[1 * kHeatMaxNz + k] = -(x0 + x1);
+  tri[4 * kHeatMaxNz + k] = -(y0 + y1);
+  const double xl = c0 == k - 1 ? x0 : x1, yl = c0 == k - 1 ? y0 : y1;
+  const double xu = c0 == k + 1 ? x0 : x1, yu = c0 == k + 1 ? y0 : y1;
+  if (k > 0) { tri[0 * kHeatMaxNz + k - 1] = xl; tri[3 * kHeatMaxNz + k - 1] = yl; }
+  if (k < nz - 1) { tri[2 * kHeatMaxNz + k] = xu; tri[5 * kHeatMaxNz + k] = yu; }
+}
+
 // Occupancy target per column height (a minimum: the compiler may fit more):
 // the register budget it leaves lets the scheduler prefetch a few layers
 // ahead without spilling.  Measured on MI355X (399k columns, 100k for
@@ -195,17 +228,16 @@ __device__ __forceinline__ void heat_step(const HeatDev &h, const double *__rest
 template <int NZ>
 constexpr int heat_waves() { return NZ <= 8 ? 4 : 2; }
 
+constexpr int kHeatBlock = 64;  // one wavefront per workgroup: a CU takes the next column set as soon as one is done
+
 template <int NZ>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(heat_waves<NZ>())))
-k_heat_columns(HeatDev h, double *__restrict__ Tout,
-                                                         int *__restrict__ unstable, RedSlot slot,
-                                                         double *__restrict__ count) {
+__global__ void __launch_bounds__(kHeatBlock) __attribute__((amdgpu_waves_per_eu(heat_waves<NZ>())))
+k_heat_columns(HeatDev h, double *__restrict__ Tout, int *__restrict__ unstable, RedSlot slot) {
   __shared__ double tri[6 * kHeatMaxNz];
   __shared__ double zeta[kHeatMaxNz];
-  for (int i = threadIdx.x; i < 6 * kHeatMaxNz; i += blockDim.x) tri[i] = h.tri[i];
-  for (int i = threadIdx.x; i < h.nz; i += blockDim.x) zeta[i] = h.zeta[i];
-  __syncthreads();
   const int nV = h.nV, nz = h.nz;
+  if ((int)threadIdx.x < nz) zeta_tridiagonal_row(nz, threadIdx.x, h.zeta, tri, zeta);
+  __syncthreads();
   const double dzb = zeta[nz - 1] - zeta[nz - 2];
   double nun = 0.0, nbad = 0.0;
 #pragma unroll 1
@@ -248,25 +280,40 @@ k_heat_columns(HeatDev h, double *__restrict__ Tout,
     for (int k = 0; k < NZ; ++k)
       if (k < nz) Tout[(size_t)k * nV + vi] = Tc[k];
   }
-  double acc[2] = {nun, nbad};
-  __shared__ double lds[2][kBlock / 64];
-  block_sum<2>(acc, lds);
+  double acc[2] = {wave_sum(nun), wave_sum(nbad)};
   block_partials<2>(slot, acc);
 }
 
-void launch_heat_columns(const HeatDev &h, double *Tout, int *unstable, const RedSlot &slot, double *count,
+// Columns' totals into the slot's result, and into host memory when the caller
+// has some that the device can write (no copy then).
+constexpr int kHeatCountBlock = 1024;  // up to 8 * 1024 partials in one round trip
+__global__ void __launch_bounds__(kHeatCountBlock) k_heat_count(RedSlot slot, int nparts,
+                                                                double *__restrict__ host) {
+  double tot[2];
+  partials_sum<2, kHeatCountBlock>(slot, nparts, tot);
+  if (threadIdx.x == 0) {
+    slot.result[0] = tot[0];
+    slot.result[1] = tot[1];
+    if (host) {
+      host[0] = tot[0];
+      host[1] = tot[1];
+    }
+  }
+}
+
+void launch_heat_columns(const HeatDev &h, double *Tout, int *unstable, const RedSlot &slot, double *host,
                          hipStream_t s) {
-  int nb = std::min(blocks_for(h.nV), kMaxPartials);
+  int nb = std::min(blocks_for(h.nV, kHeatBlock), kMaxPartials);
   if (h.nz <= 8)
-    hipLaunchKernelGGL(k_heat_columns<8>, dim3(nb), dim3(kBlock), 0, s, h, Tout, unstable, slot, count);
+    hipLaunchKernelGGL(k_heat_columns<8>, dim3(nb), dim3(kHeatBlock), 0, s, h, Tout, unstable, slot);
   else if (h.nz <= 12)
-    hipLaunchKernelGGL(k_heat_columns<12>, dim3(nb), dim3(kBlock), 0, s, h, Tout, unstable, slot, count);
+    hipLaunchKernelGGL(k_heat_columns<12>, dim3(nb), dim3(kHeatBlock), 0, s, h, Tout, unstable, slot);
   else if (h.nz <= 16)
-    hipLaunchKernelGGL(k_heat_columns<16>, dim3(nb), dim3(kBlock), 0, s, h, Tout, unstable, slot, count);
+    hipLaunchKernelGGL(k_heat_columns<16>, dim3(nb), dim3(kHeatBlock), 0, s, h, Tout, unstable, slot);
   else
-    hipLaunchKernelGGL(k_heat_columns<kHeatMaxNz>, dim3(nb), dim3(kBlock), 0, s, h, Tout, unstable, slot, count);
+    hipLaunchKernelGGL(k_heat_columns<kHeatMaxNz>, dim3(nb), dim3(kHeatBlock), 0, s, h, Tout, unstable, slot);
   UFE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_partials_out<2>, dim3(1), dim3(kBlock), 0, s, slot, nb, count);
+  hipLaunchKernelGGL(k_heat_count, dim3(1), dim3(kHeatCountBlock), 0, s, slot, nb, host);
   UFE_LAUNCH_CHECK();
 }
 
@@ -310,42 +357,6 @@ __global__ void __launch_bounds__(kBlock) k_heat_robin(int nV, int nz, const dou
   }
 }
 
-// zeta tridiagonals: calc_vertical_operators_reg_1D (mesh_zeta.f90:287-365)
-// with 1-D 2nd-order shape functions (shape_functions.f90:17-79), then the
-// tridiagonal extraction of calc_zeta_operators_tridiagonal (:487-605).
-void zeta_tridiagonals(int nz, const double *zeta, double *tri /* [6][kHeatMaxNz] */) {
-  for (int i = 0; i < 6 * kHeatMaxNz; ++i) tri[i] = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    int cidx[2];
-    if (k == 0) { cidx[0] = 1; cidx[1] = 2; }
-    else if (k == nz - 1) { cidx[0] = nz - 3; cidx[1] = nz - 2; }
-    else { cidx[0] = k - 1; cidx[1] = k + 1; }
-    double dx[2], w2[2], A[4] = {0, 0, 0, 0};
-    for (int i = 0; i < 2; ++i) {
-      dx[i] = zeta[cidx[i]] - zeta[k];
-      double w = 1.0 / std::pow(std::fabs(dx[i]), 1.5);
-      w2[i] = w * w;
-      A[0] += w2[i] * dx[i] * dx[i];
-      A[1] += w2[i] * dx[i] * 0.5 * dx[i] * dx[i];
-      A[2] += w2[i] * 0.5 * dx[i] * dx[i] * dx[i];
-      A[3] += w2[i] * 0.5 * dx[i] * dx[i] * 0.5 * dx[i] * dx[i];
-    }
-    double det = A[0] * A[3] - A[1] * A[2];
-    double M[4] = {A[3] / det, -A[1] / det, -A[2] / det, A[0] / det};
-    double fx[2], fxx[2];
-    for (int i = 0; i < 2; ++i) {
-      fx[i] = w2[i] * (M[0] * dx[i] + M[1] * 0.5 * dx[i] * dx[i]);
-      fxx[i] = w2[i] * (M[2] * dx[i] + M[3] * 0.5 * dx[i] * dx[i]);
-    }
-    tri[1 * kHeatMaxNz + k] = -(fx[0] + fx[1]);
-    tri[4 * kHeatMaxNz + k] = -(fxx[0] + fxx[1]);
-    for (int i = 0; i < 2; ++i) {
-      if (cidx[i] == k - 1) { tri[0 * kHeatMaxNz + k - 1] = fx[i]; tri[3 * kHeatMaxNz + k - 1] = fxx[i]; }
-      if (cidx[i] == k + 1) { tri[2 * kHeatMaxNz + k] = fx[i]; tri[5 * kHeatMaxNz + k] = fxx[i]; }
-    }
-  }
-}
-
 }  // namespace ufe
 
 using namespace ufe;
@@ -363,6 +374,7 @@ namespace ufe {
 int ctx_device(const ufe_ctx *c);
 hipStream_t ctx_stream(const ufe_ctx *c);
 void *ctx_heat_buffer(ufe_ctx *c, int i, size_t bytes);
+double *ctx_host_scalars(ufe_ctx *c);
 const DevMesh *ctx_mesh(const ufe_ctx *c);
 Krylov *ctx_krylov(const ufe_ctx *c);
 int ctx_fail(ufe_ctx *c, int code, const std::string &msg);
@@ -442,24 +454,22 @@ extern "C" int ufe_heat_robin(ufe_ctx *c, const ufe_heat_robin_inputs *in, const
 
 // ---------------------------------------------------------------------------
 // Scratch memory of the allocation-free heat step
-// (ufe_heat_columns_device_noalloc): the zeta tridiagonals, the per-workgroup
-// partial counts and the two totals live in one file-scope device array.
+// (ufe_heat_columns_device_noalloc): the per-workgroup partial counts and the
+// two totals live in one file-scope device array.
 // Every GPU the library runs on holds its own copy until the process ends.
 // In host code `scratch` only names the symbol: its device address on the
 // current GPU is looked up once per device (hipGetSymbolAddress) and only that
 // address reaches kernels and copies.  Layout, in doubles:
-//   [0, kScratchTri)                       zeta tridiagonals (6 x kHeatMaxNz)
-//   [kScratchPart, kScratchPart + 2 * kMaxPartials)   partials of the two counts
-//   [kScratchCnt, kScratchCnt + 2)         the totals (unstable, invalid mask)
+//   [0, 2 * kMaxPartials)              partials of the two counts
+//   [kScratchCnt, kScratchCnt + 2)     the totals (unstable, invalid mask)
 // Nothing in it has to start at zero: each workgroup writes its partials
 // before the one-workgroup pass reads them, and that pass writes both totals.
 // The array keeps the last call's contents; calls that overlap on one GPU
 // race on it.
 // ---------------------------------------------------------------------------
-constexpr size_t kScratchTri = 6 * (size_t)kHeatMaxNz;
-constexpr size_t kScratchPart = kScratchTri;
+constexpr size_t kScratchPart = 0;
 constexpr size_t kScratchCnt = kScratchPart + 2 * (size_t)kMaxPartials;
-constexpr size_t kScratchDoubles = kScratchCnt + 2;  // 16,578 doubles = 132,624 bytes
+constexpr size_t kScratchDoubles = kScratchCnt + 2;  // 16,386 doubles = 131,088 bytes
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
 constexpr int kScratchMaxDevices = 64;
@@ -541,20 +551,9 @@ int heat_columns_call(ufe_ctx *c, const ufe_heat_inputs *in, double *Tnew, int *
       return d;
     };
     auto in_dev = [&](const void *p, size_t bytes) { return device ? p : (const void *)up(p, bytes); };
-    double zeta_h[kHeatMaxNz];
-    if (device) UFE_HIP(hipMemcpy(zeta_h, in->zeta, sizeof(double) * nz, hipMemcpyDeviceToHost));
-    else std::copy(in->zeta, in->zeta + nz, zeta_h);
-    double tri[6 * kHeatMaxNz];
-    zeta_tridiagonals(nz, zeta_h, tri);
     HeatDev h;
     h.nV = nV; h.nz = nz;
     h.zeta = (const double *)in_dev(in->zeta, sizeof(double) * nz);
-    if (use_scratch) {
-      UFE_HIP(hipMemcpyAsync(scr, tri, sizeof(double) * kScratchTri, hipMemcpyHostToDevice, s));
-      h.tri = scr;
-    } else {
-      h.tri = (const double *)up(tri, sizeof(tri));
-    }
     h.Ti = (const double *)in_dev(in->Ti, n3);
     h.u = (const double *)in_dev(in->u_3D, n3);
     h.v = (const double *)in_dev(in->v_3D, n3);
@@ -578,16 +577,19 @@ int heat_columns_call(ufe_ctx *c, const ufe_heat_inputs *in, double *Tnew, int *
     double *cnt = use_scratch ? scr + kScratchCnt : (double *)buf(sizeof(double) * 2);
     double *part = use_scratch ? scr + kScratchPart : (double *)buf(sizeof(double) * 2 * kMaxPartials);
     RedSlot slot{part, cnt};
-    if (nV > 0) launch_heat_columns(h, Tout, unst, slot, cnt, s);
+    // a context keeps pinned host memory that the device writes the counts to
+    double *host = c ? ctx_host_scalars(c) : nullptr;
+    if (nV > 0) launch_heat_columns(h, Tout, unst, slot, host, s);
     double hc[2] = {0.0, 0.0};
     if (nV > 0) {
       if (!device) {
         UFE_HIP(hipMemcpyAsync(Tnew, Tout, n3, hipMemcpyDeviceToHost, s));
         UFE_HIP(hipMemcpyAsync(is_unstable, unst, sizeof(int) * nV, hipMemcpyDeviceToHost, s));
       }
-      UFE_HIP(hipMemcpyAsync(hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, s));
+      if (!host) UFE_HIP(hipMemcpyAsync(hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, s));
     }
     UFE_HIP(hipStreamSynchronize(s));
+    if (host && nV > 0) std::copy(host, host + 2, hc);
     if (!c && !use_scratch) UFE_HIP(hipStreamDestroy(s));
     if (hc[1] > 0.0)
       return heat_fail(UFE_ERR_ARGUMENT, std::to_string((long)hc[1]) +

@@ -72,6 +72,8 @@ struct ufe_ctx {
   std::shared_ptr<void> heat_mesh;  // vertex-triangle lists of the heat-column inputs (heat_inputs.hip)
   std::shared_ptr<void> bpa;        // zeta operators and BPA solver state (bpa.hip), set up on demand
   hipEvent_t ev[8];
+  // pinned host memory that one-workgroup kernels write their scalar results to
+  double *h_scalars = nullptr;
 };
 
 namespace {
@@ -755,6 +757,7 @@ void *ctx_heat_buffer(ufe_ctx *c, int i, size_t bytes) {
   if (!b || b->bytes < bytes) b = std::make_unique<DBuf>(std::max<size_t>(bytes, 8));
   return b->p;
 }
+double *ctx_host_scalars(ufe_ctx *c) { return c->h_scalars; }
 hipStream_t ctx_stream(const ufe_ctx *c) { return c->s; }
 const DevMesh *ctx_mesh(const ufe_ctx *c) { return &c->m; }
 Krylov *ctx_krylov(const ufe_ctx *c) { return c->kry.get(); }
@@ -922,6 +925,7 @@ extern "C" int ufe_ctx_create(ufe_ctx **out, int device, const ufe_mesh_desc *md
     c->out2.alloc(sizeof(double) * 4);
     UFE_HIP(hipMemset(c->u.p, 0, v2));
     c->kry = std::make_unique<Krylov>(nT, c->s);
+    UFE_HIP(hipHostMalloc((void **)&c->h_scalars, 8 * sizeof(double), hipHostMallocDefault));
     {
       const char *e;
       double om = (e = std::getenv("UFE_AMG_OMEGA")) ? std::atof(e) : 0.85;
@@ -956,6 +960,7 @@ extern "C" int ufe_ctx_destroy(ufe_ctx *c) {
   (void)hipSetDevice(c->device);
   if (c->s) (void)hipStreamSynchronize(c->s);
   for (auto &e : c->ev) (void)hipEventDestroy(e);
+  if (c->h_scalars) (void)hipHostFree(c->h_scalars);
   hipStream_t s = c->s;
   delete c;
   if (s) (void)hipStreamDestroy(s);
