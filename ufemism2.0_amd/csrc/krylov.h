@@ -62,7 +62,13 @@ struct AmgLevelPattern {
   DBuf ptr, col, crow, gptr, glist;
   // levels < last: aggregate of each block row and members of each aggregate
   DBuf agg, mem_ptr, mem_ind;
+  // workgroups of the fused residual + restriction: whole aggregates, at most
+  // kAmgWgRows member rows each; per workgroup its first aggregate, per member
+  // slot (row, first entry, end entry, 0).  n_wg = 0: an aggregate is too large.
+  DBuf wg_agg, slot;
+  int n_wg = 0;
 };
+constexpr int kAmgWgRows = 64;
 
 struct AmgHierarchy {
   std::vector<std::unique_ptr<AmgLevelPattern>> levels;  // levels[0] has nb/nnzb of the system
