@@ -277,6 +277,22 @@ def test_amg_fused_variants_equal_per_level_kernels(V, channel_fixtures, monkeyp
     assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
 
 
+@pytest.mark.parametrize("l1", [0, 1])
+@pytest.mark.parametrize("rows", ["30", "100", "300"])
+def test_amg_tail_in_lds_equals_the_one_in_device_memory(V, channel_fixtures, monkeypatch, rows, l1):
+    """The one-workgroup kernel of the coarse levels with patterns and values in
+    LDS (taken when they fit) against the one that reads them from device
+    memory (4096 rows do not fit): one to three levels in it, bit for bit."""
+    w, _ = channel_fixtures["SSA"]
+    form = dict(CHOSEN, amg_smoother=l1)
+    monkeypatch.setenv("UFE_AMG_TAIL_ROWS", "4096")
+    a, ia = solve(V, w, **TIGHT, **form)
+    monkeypatch.setenv("UFE_AMG_TAIL_ROWS", rows)
+    b, ib = solve(V, w, **TIGHT, **form)
+    assert ia.n_visc_its == ib.n_visc_its and ia.n_Axb_its == ib.n_Axb_its
+    assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
+
+
 @pytest.mark.parametrize("nz", [10, 12])
 def test_diva_column_kernels_equal_per_thread_kernels(V, W, monkeypatch, nz):
     """The DIVA vertex and triangle kernels with 16 lanes per column (the

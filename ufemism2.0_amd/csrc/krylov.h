@@ -19,6 +19,7 @@
 //       iteration).  It is a fixed linear operator, so plain BiCGStab applies.
 #pragma once
 
+#include <array>
 #include <cstdint>
 #include <functional>
 #include <memory>
@@ -72,6 +73,12 @@ constexpr int kAmgWgRows = 64;
 
 struct AmgHierarchy {
   std::vector<std::unique_ptr<AmgLevelPattern>> levels;  // levels[0] has nb/nnzb of the system
+  // the small levels' patterns once more in one piece, level after level, for
+  // the one-workgroup kernel, which copies the end of it into LDS: offsets (in
+  // ints, multiples of 4) of ptr, col, agg, mem_ptr, mem_ind; -1: level not in it
+  DBuf packed;
+  std::vector<std::array<int, 5>> packed_off;
+  int packed_ints = 0;
   int n_levels() const { return (int)levels.size(); }
 };
 
@@ -84,7 +91,12 @@ std::unique_ptr<AmgHierarchy> build_amg_hierarchy(int nT, const int *TriC, const
 
 template <typename T>
 struct AmgValues {
-  std::vector<std::unique_ptr<DBuf>> val, dinv;  // levels >= 1 (level 0 values are the system's)
+  // levels >= 1 (level 0 values are the system's) in one piece, level after
+  // level: blocks, then diagonal inverses; offsets in blocks, and the end
+  DBuf arena;
+  std::vector<size_t> val, dinv;
+  size_t end = 0;
+  DBuf dinv0;  // level 0 with the l1 smoother
   std::vector<std::unique_ptr<DBuf>> r, z, zt;   // per-level vectors (levels >= 1 for r, all for z/zt)
 };
 
@@ -209,6 +221,7 @@ class Krylov {
   const int *A_diag_ = nullptr;
   const float4 *fine32_ = nullptr;
   int amg_tail_rows_ = 300;
+  bool tail_in_lds_ = false;  // the device gives a workgroup kTailLdsAll bytes of LDS
   bool amg_l1_ = false;
   bool unit_diag0_ = false;
   double amg_omega_ = 0.85;

@@ -840,6 +840,8 @@ struct AmgTailLevel {
   // device-memory vectors above (the top level's r and z are the kernel's
   // input and output and always live in device memory)
   int off_r, off_z, off_zt;
+  // k_amg_tail_lds: byte offsets in LDS of the level's pattern and values
+  int o_ptr, o_col, o_agg, o_mem_ptr, o_mem_ind, o_val, o_dinv;
 };
 constexpr int kTailLdsMax = 48 * 1024;  // dynamic LDS of the tail kernel, at most
 struct AmgTailArgs {
@@ -847,7 +849,15 @@ struct AmgTailArgs {
   double omega, scale;
   const double *cinv;  // dense inverse of the coarsest level, column-major
   AmgTailLevel lv[kTailMaxLevels];
+  // k_amg_tail_lds: the pieces copied to LDS, one after another from offset 0,
+  // in 16-byte units: patterns, values, the coarsest inverse, the top level's
+  // r and z
+  const void *src[5];
+  int units[5];
+  int o_cinv;
 };
+// LDS of k_amg_tail_lds, at most (of the CU's 160 KB)
+constexpr int kTailLdsAll = 156 * 1024;
 
 // A tail level's vector: in the kernel's LDS when it has an offset there,
 // else in device memory.  The work-group barriers between the phases order
@@ -903,6 +913,85 @@ __global__ void __launch_bounds__(kTailThreads) k_amg_tail(AmgTailArgs a, const 
     __syncthreads();
     for (int i = threadIdx.x; i < L.nb; i += blockDim.x) Lz[i] = Lzt[i];
     __syncthreads();
+  }
+}
+
+// The same with everything in LDS: patterns, values, the coarsest inverse and
+// all vectors are copied there first, all loads in flight together, so the
+// chains of dependent loads of every pass (ptr -> col -> z, mem_ptr -> mem_ind
+// -> q) cost LDS latency instead of L2 latency.  The sums are the same, bit for
+// bit.  Taken when the levels fit (kTailLdsAll: 18 to 79 KB at the default 300
+// rows on the meshes here); on the 20k-vertex channel 8.0 us against 14.1 us.
+template <typename T>
+__global__ void __launch_bounds__(kTailThreads) k_amg_tail_lds(AmgTailArgs a, const KrylovScalars *__restrict__ sc) {
+  using V2 = typename VecT<T>::V2;
+  using V4 = typename VecT<T>::V4;
+  extern __shared__ __align__(16) unsigned char tail_lds[];
+  if (sc && sc->done) return;
+  {
+    const int e0 = a.units[0], e1 = e0 + a.units[1], e2 = e1 + a.units[2], e3 = e2 + a.units[3],
+              e4 = e3 + a.units[4];
+    const uint4 *s0 = (const uint4 *)a.src[0], *s1 = (const uint4 *)a.src[1] - e0,
+                *s2 = (const uint4 *)a.src[2] - e1, *s3 = (const uint4 *)a.src[3] - e2,
+                *s4 = (const uint4 *)a.src[4] - e3;
+    uint4 *dst = (uint4 *)tail_lds;
+    constexpr int U = 10;  // 10 x 1024 x 16 B: one round of loads for all that fits
+    for (int u0 = threadIdx.x; u0 < e4; u0 += U * kTailThreads) {
+      uint4 v[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int u = min(u0 + q * kTailThreads, e4 - 1);
+        v[q] = (u < e0 ? s0 : u < e1 ? s1 : u < e2 ? s2 : u < e3 ? s3 : s4)[u];
+      }
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+        if (u0 + q * kTailThreads < e4) dst[u0 + q * kTailThreads] = v[q];
+    }
+  }
+  __syncthreads();
+  const int lane = threadIdx.x % kLpr, grp = threadIdx.x / kLpr, ngrp = blockDim.x / kLpr;
+  const T om = (T)a.omega, cs = (T)a.scale;
+  auto ints = [&](int o) { return (const int *)(tail_lds + o); };
+  auto vec = [&](int o) { return (V2 *)(tail_lds + o); };
+  auto blk = [&](int o) { return (const V4 *)(tail_lds + o); };
+  for (int l = 0; l + 1 < a.n; ++l) {
+    const AmgTailLevel &L = a.lv[l];
+    const AmgTailLevel &C = a.lv[l + 1];
+    for (int row = grp; row < L.nb; row += ngrp)
+      row_resid<T, T>(row, lane, ints(L.o_ptr), ints(L.o_col), blk(L.o_val), vec(L.off_r), vec(L.off_z),
+                      vec(L.off_zt));
+    __syncthreads();
+    V2 *zc = l + 2 < a.n ? vec(C.off_z) : nullptr;
+    for (int I = grp; I < C.nb; I += ngrp)
+      agg_restrict<T>(I, lane, ints(L.o_mem_ptr), ints(L.o_mem_ind), vec(L.off_zt), vec(C.off_r), blk(C.o_dinv), om,
+                      zc);
+    __syncthreads();
+  }
+  {
+    const AmgTailLevel &C = a.lv[a.n - 1];
+    const int n = 2 * C.nb, i = threadIdx.x;
+    if (i < n) {
+      const T *rr = (const T *)(tail_lds + C.off_r);
+      const double *ci = (const double *)(tail_lds + a.o_cinv);
+      double s = 0.0;
+      for (int j = 0; j < n; ++j) s += ci[(size_t)j * n + i] * (double)rr[j];
+      ((T *)(tail_lds + C.off_z))[i] = (T)s;
+    }
+    __syncthreads();
+  }
+  int oc = a.lv[a.n - 1].off_z;  // the coarser level's correction
+  for (int l = a.n - 2; l >= 0; --l) {
+    const AmgTailLevel &L = a.lv[l];
+    for (int row = grp; row < L.nb; row += ngrp) {
+      if (l > 0)
+        row_prolong_smooth<T, T>(row, lane, ints(L.o_ptr), ints(L.o_col), blk(L.o_val), blk(L.o_dinv), ints(L.o_agg),
+                                 vec(L.off_r), vec(L.off_z), vec(oc), cs, om, vec(L.off_zt));
+      else
+        row_prolong_smooth<T, T>(row, lane, ints(L.o_ptr), ints(L.o_col), blk(L.o_val), blk(L.o_dinv), ints(L.o_agg),
+                                 vec(L.off_r), vec(L.off_z), vec(oc), cs, om, (V2 *)L.z);
+    }
+    oc = L.off_zt;
+    if (l > 0) __syncthreads();
   }
 }
 
@@ -982,6 +1071,7 @@ std::unique_ptr<AmgHierarchy> build_amg_hierarchy(int nT, const int *TriC, const
   }
   std::vector<int> mptr(ptr0, ptr0 + nT + 1), mcol(col0, col0 + ptr0[nT]);
   std::vector<int> gptr, glist;  // gather lists building the current level
+  std::vector<int> packed;
   int n = nT;
   for (int lev = 0; lev < max_levels; ++lev) {
     auto L = std::make_unique<AmgLevelPattern>();
@@ -996,6 +1086,18 @@ std::unique_ptr<AmgHierarchy> build_amg_hierarchy(int nT, const int *TriC, const
       upload(L->crow, crow);
       upload(L->gptr, gptr);
       upload(L->glist, glist);
+    }
+    // packed patterns of the levels that the one-workgroup kernel may take
+    H->packed_off.push_back({-1, -1, -1, -1, -1});
+    const bool pack = lev > 0 && n <= kTailMaxRows;
+    auto add = [&](int which, const std::vector<int> &v) {
+      H->packed_off[lev][which] = (int)packed.size();
+      packed.insert(packed.end(), v.begin(), v.end());
+      packed.resize((packed.size() + 3) & ~size_t(3), 0);
+    };
+    if (pack) {
+      add(0, mptr);
+      add(1, mcol);
     }
     bool last = (n <= coarse_target) || (lev == max_levels - 1);
     int na = 0;
@@ -1027,6 +1129,11 @@ std::unique_ptr<AmgHierarchy> build_amg_hierarchy(int nT, const int *TriC, const
     upload(L->agg, agg);
     upload(L->mem_ptr, cnt);
     upload(L->mem_ind, mem);
+    if (pack) {
+      add(2, agg);
+      add(3, cnt);
+      add(4, mem);
+    }
     // workgroups of the fused residual + restriction
     int largest = 0;
     for (int I = 0; I < na; ++I) largest = std::max(largest, cnt[I + 1] - cnt[I]);
@@ -1073,6 +1180,8 @@ std::unique_ptr<AmgHierarchy> build_amg_hierarchy(int nT, const int *TriC, const
     mcol.swap(ccol);
     n = na;
   }
+  upload(H->packed, packed);
+  H->packed_ints = (int)packed.size();
   return H;
 }
 
@@ -1084,6 +1193,11 @@ Krylov::Krylov(int nb, hipStream_t s) : nb_(nb), s_(s) {
   red_part_.alloc(sizeof(double) * kMaxPartials * 4 * 4);
   red_res_.alloc(sizeof(double) * 4 * 4);
   UFE_HIP(hipMemset(scal_.p, 0, sizeof(KrylovScalars)));
+  tail_in_lds_ = hipFuncSetAttribute((const void *)k_amg_tail_lds<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     kTailLdsAll) == hipSuccess &&
+                 hipFuncSetAttribute((const void *)k_amg_tail_lds<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     kTailLdsAll) == hipSuccess;
+  if (!tail_in_lds_) (void)hipGetLastError();
   UFE_HIP(hipHostMalloc((void **)&h_scal_, sizeof(KrylovScalars), hipHostMallocDefault));
 }
 
@@ -1158,24 +1272,29 @@ void Krylov::amg_setup(const BsrT<T> &A0) {
                                                              : *reinterpret_cast<std::vector<BsrT<T>> *>(&lev32_);
   int L = amg_->n_levels();
   if ((int)av.val.size() != L) {
-    av.val.clear(); av.dinv.clear(); av.r.clear(); av.z.clear(); av.zt.clear();
+    av.val.assign(L, 0); av.dinv.assign(L, 0); av.r.clear(); av.z.clear(); av.zt.clear();
+    av.end = 0;
     for (int l = 0; l < L; ++l) {
       const AmgLevelPattern &P = *amg_->levels[l];
-      av.val.push_back(std::make_unique<DBuf>(l > 0 ? sizeof(V4) * (size_t)P.nnzb : 0));
-      av.dinv.push_back(std::make_unique<DBuf>(l > 0 ? sizeof(V4) * (size_t)P.nb : 0));
-      av.r.push_back(std::make_unique<DBuf>(sizeof(V2) * (size_t)P.nb));
-      av.z.push_back(std::make_unique<DBuf>(sizeof(V2) * (size_t)P.nb));
-      av.zt.push_back(std::make_unique<DBuf>(sizeof(V2) * (size_t)P.nb));
+      if (l > 0) {
+        av.val[l] = av.end;
+        av.dinv[l] = av.end + P.nnzb;
+        av.end += (size_t)P.nnzb + P.nb;
+      }
+      av.r.push_back(std::make_unique<DBuf>((sizeof(V2) * (size_t)P.nb + 15) & ~size_t(15)));
+      av.z.push_back(std::make_unique<DBuf>((sizeof(V2) * (size_t)P.nb + 15) & ~size_t(15)));
+      av.zt.push_back(std::make_unique<DBuf>((sizeof(V2) * (size_t)P.nb + 15) & ~size_t(15)));
     }
+    av.arena.alloc(sizeof(V4) * std::max<size_t>(av.end, 1));
   }
   lev.assign(L, BsrT<T>());
   lev[0] = A0;
   if (amg_l1_) {
-    if (av.dinv[0]->bytes < sizeof(V4) * (size_t)A0.nb) av.dinv[0]->alloc(sizeof(V4) * (size_t)A0.nb);
+    if (av.dinv0.bytes < sizeof(V4) * (size_t)A0.nb) av.dinv0.alloc(sizeof(V4) * (size_t)A0.nb);
     hipLaunchKernelGGL(k_l1_dinv<T>, dim3(blocks_for(A0.nb)), dim3(kBlock), 0, s_, A0.nb, A0.ptr, A0.col, A0.val,
-                       av.dinv[0]->template as<V4>());
+                       av.dinv0.template as<V4>());
     UFE_LAUNCH_CHECK();
-    lev[0].dinv = av.dinv[0]->template as<V4>();
+    lev[0].dinv = av.dinv0.template as<V4>();
   }
   for (int l = 1; l < L; ++l) {
     const AmgLevelPattern &P = *amg_->levels[l];
@@ -1184,15 +1303,16 @@ void Krylov::amg_setup(const BsrT<T> &A0) {
     B.nnzb = P.nnzb;
     B.ptr = P.ptr.as<int>();
     B.col = P.col.as<int>();
-    B.val = av.val[l]->template as<V4>();
-    B.dinv = av.dinv[l]->template as<V4>();
+    V4 *const val = av.arena.template as<V4>() + av.val[l], *const dinv = av.arena.template as<V4>() + av.dinv[l];
+    B.val = val;
+    B.dinv = dinv;
     hipLaunchKernelGGL(k_galerkin<T>, dim3(blocks_for(P.nnzb)), dim3(kBlock), 0, s_, P.nnzb, P.gptr.as<int>(),
                        P.glist.as<int>(), lev[l - 1].val, P.crow.as<int>(), P.col.as<int>(),
-                       av.val[l]->template as<V4>(), av.dinv[l]->template as<V4>());
+                       val, dinv);
     UFE_LAUNCH_CHECK();
     if (amg_l1_) {
       hipLaunchKernelGGL(k_l1_dinv<T>, dim3(blocks_for(B.nb)), dim3(kBlock), 0, s_, B.nb, B.ptr, B.col, B.val,
-                         av.dinv[l]->template as<V4>());
+                         dinv);
       UFE_LAUNCH_CHECK();
     }
     lev[l] = B;
@@ -1210,6 +1330,7 @@ void Krylov::amg_setup32(const BsrT<float> &A0) { amg_setup<float>(A0); }
 template <typename T>
 void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, hipEvent_t ev1) {
   using V2 = typename VecT<T>::V2;
+  using V4 = typename VecT<T>::V4;
   AmgValues<T> &av = amg_vals<T>();
   std::vector<BsrT<T>> &lev = std::is_same<T, double>::value ? *reinterpret_cast<std::vector<BsrT<T>> *>(&lev64_)
                                                              : *reinterpret_cast<std::vector<BsrT<T>> *>(&lev32_);
@@ -1282,6 +1403,7 @@ void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, h
     UFE_LAUNCH_CHECK();
   } else {
     AmgTailArgs ta{};
+    bool tail_done = false;
     ta.n = L - t;
     ta.omega = amg_omega_;
     ta.scale = amg_coarse_scale_;
@@ -1302,25 +1424,70 @@ void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, h
       d.zt = av.zt[l]->p;
       d.off_r = d.off_z = d.off_zt = -1;
     }
-    // the vectors that stay inside the kernel go to LDS: every level's zt and
-    // the r and z of the levels below the top one
-    int lds = 0;
-    auto take = [&](int nb) {
-      const int o = lds;
-      lds += ((int)(nb * sizeof(V2)) + 15) & ~15;
-      return o;
-    };
-    for (int l = 0; l < ta.n; ++l) {
-      AmgTailLevel &d = ta.lv[l];
-      if (l + 1 < ta.n) d.off_zt = take(d.nb);
-      if (l > 0) { d.off_r = take(d.nb); d.off_z = take(d.nb); }
+    // everything in LDS when it fits: patterns and values of the levels are
+    // contiguous from the top one on
+    if (tail_in_lds_ && amg_->packed_off[t][0] >= 0) {
+      const int p0 = amg_->packed_off[t][0];
+      const size_t v0 = av.val[t];
+      const int n2 = 2 * lev[L - 1].nb;
+      const size_t bytes[5] = {sizeof(int) * (size_t)(amg_->packed_ints - p0), sizeof(V4) * (av.end - v0),
+                               (sizeof(double) * (size_t)n2 * n2 + 15) & ~size_t(15),
+                               (sizeof(V2) * (size_t)lev[t].nb + 15) & ~size_t(15),
+                               (sizeof(V2) * (size_t)lev[t].nb + 15) & ~size_t(15)};
+      size_t o[6] = {0};
+      for (int q = 0; q < 5; ++q) o[q + 1] = o[q] + bytes[q];
+      size_t end = o[5];
+      auto take = [&](int nb) {
+        const size_t at = end;
+        end += (sizeof(V2) * (size_t)nb + 15) & ~size_t(15);
+        return (int)at;
+      };
+      for (int l = t; l < L; ++l) {
+        AmgTailLevel &d = ta.lv[l - t];
+        const std::array<int, 5> &po = amg_->packed_off[l];
+        auto pat = [&](int q) { return po[q] >= 0 ? (int)(sizeof(int) * (size_t)(po[q] - p0)) : -1; };
+        d.o_ptr = pat(0); d.o_col = pat(1); d.o_agg = pat(2); d.o_mem_ptr = pat(3); d.o_mem_ind = pat(4);
+        d.o_val = (int)(o[1] + sizeof(V4) * (av.val[l] - v0));
+        d.o_dinv = (int)(o[1] + sizeof(V4) * (av.dinv[l] - v0));
+        d.off_r = l == t ? (int)o[3] : take(d.nb);
+        d.off_z = l == t ? (int)o[4] : take(d.nb);
+        d.off_zt = l + 1 < L ? take(d.nb) : -1;
+      }
+      const void *src[5] = {amg_->packed.template as<int>() + p0, av.arena.template as<V4>() + v0, coarse_inv_.p,
+                            ta.lv[0].r, ta.lv[0].z};
+      for (int q = 0; q < 5; ++q) {
+        ta.src[q] = src[q];
+        ta.units[q] = (int)(bytes[q] / 16);
+      }
+      ta.o_cinv = (int)o[2];
+      if (end <= (size_t)kTailLdsAll) {
+        hipLaunchKernelGGL(k_amg_tail_lds<T>, dim3(1), dim3(kTailThreads), end, s_, ta, sc);
+        UFE_LAUNCH_CHECK();
+        tail_done = true;
+      }
     }
-    if (lds > kTailLdsMax) {
+    if (!tail_done) {
       for (int l = 0; l < ta.n; ++l) ta.lv[l].off_r = ta.lv[l].off_z = ta.lv[l].off_zt = -1;
-      lds = 0;
+      // the vectors that stay inside the kernel go to LDS: every level's zt and
+      // the r and z of the levels below the top one
+      int lds = 0;
+      auto take = [&](int nb) {
+        const int o = lds;
+        lds += ((int)(nb * sizeof(V2)) + 15) & ~15;
+        return o;
+      };
+      for (int l = 0; l < ta.n; ++l) {
+        AmgTailLevel &d = ta.lv[l];
+        if (l + 1 < ta.n) d.off_zt = take(d.nb);
+        if (l > 0) { d.off_r = take(d.nb); d.off_z = take(d.nb); }
+      }
+      if (lds > kTailLdsMax) {
+        for (int l = 0; l < ta.n; ++l) ta.lv[l].off_r = ta.lv[l].off_z = ta.lv[l].off_zt = -1;
+        lds = 0;
+      }
+      hipLaunchKernelGGL(k_amg_tail<T>, dim3(1), dim3(kTailThreads), lds, s_, ta, sc);
+      UFE_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(k_amg_tail<T>, dim3(1), dim3(kTailThreads), lds, s_, ta, sc);
-    UFE_LAUNCH_CHECK();
   }
   for (int l = t - 1; l >= 0; --l) {
     const AmgLevelPattern &P = *amg_->levels[l];
