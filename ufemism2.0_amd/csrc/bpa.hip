@@ -42,6 +42,7 @@
 struct ufe_ctx;
 namespace ufe {
 int ctx_device(const ufe_ctx *c);
+double *ctx_host_scalars(ufe_ctx *c);
 hipStream_t ctx_stream(const ufe_ctx *c);
 const DevMesh *ctx_mesh(const ufe_ctx *c);
 int ctx_fail(ufe_ctx *c, int code, const std::string &msg);
@@ -867,7 +868,7 @@ struct BpaState {
   DBuf Hi, Hs, A_ak, A_bks, rough, fgr, bcm, bcu, bcv, zv, zt, a2, tribi;
   bool has_bc = false;
   // iteration
-  DBuf x, xprev, rhs, sr4, eta_ak, eta_bks, coef, beta_a, beta_b, cDinv, cW, cU, part, out, r;
+  DBuf x, xprev, rhs, sr4, eta_ak, eta_bks, coef, beta_a, beta_b, cDinv, cW, cU, part, r;
   BpaParams par{};  // of the system formed last
   std::unique_ptr<Krylov> kry;
   // stage timings of the last solve (HIP events on the context's stream)
@@ -1018,7 +1019,6 @@ void bpa_pattern(ufe_ctx *c, BpaState &b) {
   ensure(b.cW, sizeof(double4) * nbk);
   ensure(b.cU, sizeof(double4) * nbk);
   ensure(b.part, sizeof(double) * kMaxPartials * 2);
-  ensure(b.out, sizeof(double) * 2);
   b.kry = std::make_unique<Krylov>(b.nb, s);
   set_operator(c, b);
   for (hipEvent_t &ev : b.ev) UFE_HIP(hipEventCreate(&ev));
@@ -1420,7 +1420,7 @@ extern "C" int ufe_solve_bpa(ufe_ctx *c, const ufe_bpa_inputs *in, double *u_bk,
     double relax = p.visc_it_relax, eps0 = p.epsilon_sq_0;
     bool converged = false;
     rc = UFE_OK;
-    RedSlot slot{b.part.as<double>(), b.out.as<double>()};
+    RedSlot slot{b.part.as<double>(), nullptr};
     for (double &t : b.t_ms) t = 0.0;
     while (!converged) {
       ++it;
@@ -1442,11 +1442,10 @@ extern "C" int ufe_solve_bpa(ufe_ctx *c, const ufe_bpa_inputs *in, double *u_bk,
         hipLaunchKernelGGL(k_bpa_update, dim3(g), dim3(kBlock), 0, s, n, p.vel_max, relax,
                            b.x.as<double2>() + off, b.xprev.as<double2>() + off, slot);
         UFE_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_partials_out<2>, dim3(1), dim3(kBlock), 0, s, slot, g, b.out.as<double>());
+        hipLaunchKernelGGL(k_partials_out<2>, dim3(2), dim3(kBlock), 0, s, slot, g, ctx_host_scalars(c));
         UFE_LAUNCH_CHECK();
-        double h2[2];
-        UFE_HIP(hipMemcpyAsync(h2, b.out.p, sizeof(h2), hipMemcpyDeviceToHost, s));
         UFE_HIP(hipStreamSynchronize(s));
+        const double *h2 = ctx_host_scalars(c);
         r1 += h2[0];
         r2 += h2[1];
       }

@@ -83,13 +83,13 @@ __global__ void __launch_bounds__(kBlock) k_aa_mix(int n, double *__restrict__ x
 void launch_aa_columns(int nT, double *x, const double *u, double *fprev, double *gprev, double *dF, double *dG,
                        long stride, int p, int have_prev, int ncols, double vel_max, const RedSlot &slot,
                        double *out, hipStream_t s) {
-  // grid-stride over at most 1,024 workgroups: the one-workgroup second phase
-  // then sums 17 x 1,024 partials instead of 17 x nT / 256
+  // grid-stride over at most 1,024 workgroups: the second phase then sums 17 x
+  // 1,024 partials instead of 17 x nT / 256
   int nb = std::min(blocks_for(nT), 1024);
   hipLaunchKernelGGL(k_aa_columns, dim3(nb), dim3(kBlock), 0, s, nT, x, u, fprev, gprev, dF, dG, stride, p,
                      have_prev, ncols, vel_max, slot, out);
   UFE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_partials_out<kAAW>, dim3(1), dim3(kBlock), 0, s, slot, nb, out);
+  hipLaunchKernelGGL(k_partials_out<kAAW>, dim3(kAAW), dim3(kBlock), 0, s, slot, nb, out);
   UFE_LAUNCH_CHECK();
 }
 
@@ -151,8 +151,7 @@ void anderson_step(AndersonState &aa, const AndersonBuffers &buf, int depth, dou
   sl.result = buf.out;
   launch_aa_columns((int)n2, x, u, buf.fprev, buf.gprev, buf.dF, buf.dG, stride, p < 0 ? 0 : p,
                     aa.have_prev ? 1 : 0, aa.cols, vel_max, sl, buf.out, s);
-  double h[2 * kAAMaxDepth + 1];
-  UFE_HIP(hipMemcpyAsync(h, buf.out, sizeof(h), hipMemcpyDeviceToHost, s));
+  const double *h = buf.out;  // pinned host memory
   UFE_HIP(hipStreamSynchronize(s));
   aa.have_prev = true;
   AAGamma gam{};

@@ -314,7 +314,7 @@ void launch_update(int nT, const double *x, double *u, double *uprev, double vel
   hipLaunchKernelGGL(k_update, dim3(nb), dim3(kBlock), 0, s, nT, x, u, uprev, vel_max, relax, slot, out2,
                      beta_basal_b, tri_coef, F2b0, no_sliding, ubase, taub);
   UFE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_partials_out<2>, dim3(1), dim3(kBlock), 0, s, slot, nb, out2);
+  hipLaunchKernelGGL(k_partials_out<2>, dim3(2), dim3(kBlock), 0, s, slot, nb, out2);
   UFE_LAUNCH_CHECK();
 }
 

@@ -235,7 +235,8 @@ class Krylov {
   DBuf coarse_inv_;      // dense inverse of the coarsest level (column-major)
   DBuf scal_;            // KrylovScalars
   DBuf red_part_, red_res_;
-  KrylovScalars *h_scal_ = nullptr;  // pinned host mirror
+  KrylovScalars *h_scal_ = nullptr;  // pinned host mirror, written by the device
+  double *h_red_ = nullptr;          // pinned: the three sums of a residual product
   bool time_spmv_ = false;
   std::vector<hipEvent_t> tev_;
   long long tn_[2] = {0, 0};

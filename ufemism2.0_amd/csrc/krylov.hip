@@ -144,16 +144,17 @@ template <int OP>
 __global__ void __launch_bounds__(kFinishBlock) k_spmv_finish(RedSlot slot, int nparts, double *__restrict__ out,
                                                               KrylovScalars *__restrict__ sc) {
   if (sc && sc->done) return;
-  double tot[3];
-  partials_sum<3, kFinishBlock>(slot, nparts, tot);
+  constexpr int W = OP == OP_RESID ? 3 : OP == OP_DOT2 ? 2 : 1;
+  double tot[W];
+  partials_sum<W, kFinishBlock>(slot, nparts, tot);
   if (threadIdx.x != 0) return;
-  if (OP == OP_RESID) {
+  if constexpr (OP == OP_RESID) {
     out[0] = tot[0];
     out[1] = tot[1];
     out[2] = tot[2];
-  } else if (OP == OP_DOT1) {
+  } else if constexpr (OP == OP_DOT1) {
     // alpha = rho / (rhat, v)
-    if (tot[0] == 0.0 || !std::isfinite(tot[0])) sc->done = 2;
+    if (tot[0] == 0.0 || !std::isfinite(tot[0])) sc->done = sc->host->done = 2;
     else sc->alpha = sc->rho / tot[0];
   } else {
     // omega = (t, s) / (t, t)
@@ -318,6 +319,17 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x(int nb, typename VecT<T>::V2 
   block_partials<2>(slot, acc);
 }
 
+// What the host polls, into the pinned mirror.
+__device__ __forceinline__ void publish(const KrylovScalars *sc) {
+  KrylovScalars *h = sc->host;
+  h->rr = sc->rr;
+  h->rho = sc->rho;
+  h->omega = sc->omega;
+  h->tol2 = sc->tol2;
+  h->its = sc->its;
+  h->done = sc->done;
+}
+
 // Second phase of k_bicg_x (one workgroup): rho, ||r||^2 and the stop test.
 __global__ void __launch_bounds__(kBlock) k_bicg_x_finish(RedSlot slot, int nparts, KrylovScalars *__restrict__ sc) {
   if (sc->done) return;
@@ -332,15 +344,16 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x_finish(RedSlot slot, int npar
   else if (tot[1] <= sc->tol2) sc->done = 1;
   else if (sc->omega == 0.0 || tot[0] == 0.0) sc->done = 2;
   else if (sc->its >= sc->maxit) sc->done = 3;
+  publish(sc);
 }
 
-// rhat = r, p = v = 0, scalars from ||r0||^2 (rr_in)
+// rhat = r, p = v = 0, scalars from ||r0||^2 and ||b||^2 (rr, bb)
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_bicg_init(int nb, const typename VecT<T>::V2 *__restrict__ r,
                                                       typename VecT<T>::V2 *__restrict__ rhat,
                                                       typename VecT<T>::V2 *__restrict__ p,
                                                       typename VecT<T>::V2 *__restrict__ v,
-                                                      const double *__restrict__ rr_in, double rtol, double abstol,
+                                                      double rr, double bb, double rtol, double abstol,
                                                       int maxit, KrylovScalars *__restrict__ sc) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nb) {
@@ -351,18 +364,18 @@ __global__ void __launch_bounds__(kBlock) k_bicg_init(int nb, const typename Vec
     v[i] = z;
   }
   if (i == 0) {
-    double rr = rr_in[0];
     sc->rho = rr;
     sc->rho_old = 1.0;
     sc->alpha = 1.0;
     sc->omega = 1.0;
     sc->rr = rr;
-    sc->bb = rr_in[1];
+    sc->bb = bb;
     double tol = fmax(rtol * sqrt(rr), abstol);
     sc->tol2 = tol * tol;
     sc->its = 0;
     sc->maxit = maxit;
     sc->done = (rr <= sc->tol2) ? 1 : 0;
+    publish(sc);
   }
 }
 
@@ -1192,18 +1205,23 @@ Krylov::Krylov(int nb, hipStream_t s) : nb_(nb), s_(s) {
   scal_.alloc(sizeof(KrylovScalars));
   red_part_.alloc(sizeof(double) * kMaxPartials * 4 * 4);
   red_res_.alloc(sizeof(double) * 4 * 4);
-  UFE_HIP(hipMemset(scal_.p, 0, sizeof(KrylovScalars)));
   tail_in_lds_ = hipFuncSetAttribute((const void *)k_amg_tail_lds<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      kTailLdsAll) == hipSuccess &&
                  hipFuncSetAttribute((const void *)k_amg_tail_lds<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      kTailLdsAll) == hipSuccess;
   if (!tail_in_lds_) (void)hipGetLastError();
   UFE_HIP(hipHostMalloc((void **)&h_scal_, sizeof(KrylovScalars), hipHostMallocDefault));
+  UFE_HIP(hipHostMalloc((void **)&h_red_, 4 * sizeof(double), hipHostMallocDefault));
+  *h_scal_ = KrylovScalars{};
+  KrylovScalars sc0{};
+  sc0.host = h_scal_;
+  UFE_HIP(hipMemcpy(scal_.p, &sc0, sizeof(sc0), hipMemcpyHostToDevice));
 }
 
 Krylov::~Krylov() {
   for (GraphCache &g : graphs_) g.clear();
   if (h_scal_) (void)hipHostFree(h_scal_);
+  if (h_red_) (void)hipHostFree(h_red_);
   for (hipEvent_t e : tev_) (void)hipEventDestroy(e);
 }
 
@@ -1249,11 +1267,10 @@ float *Krylov::tmp32(int i) { return vec32_[i].as<float>(); }
 void Krylov::residual64(const BsrT<double> &A, const double *x, const double *b, double *r, double *rr,
                         double *bb, double vmax, int *n_clamped, const double4 *dblk, int write_unscaled) {
   RedSlot sl = slot(3);
-  if (!A.val) residual<double>(A, x, r, b, sl, sl.result);
-  else spmv_launch<double, OP_RESID>(A, x, r, b, nullptr, sl, sl.result, nullptr, s_, vmax, dblk, write_unscaled);
-  double h[3];
-  UFE_HIP(hipMemcpyAsync(h, sl.result, sizeof(h), hipMemcpyDeviceToHost, s_));
+  if (!A.val) residual<double>(A, x, r, b, sl, h_red_);
+  else spmv_launch<double, OP_RESID>(A, x, r, b, nullptr, sl, h_red_, nullptr, s_, vmax, dblk, write_unscaled);
   UFE_HIP(hipStreamSynchronize(s_));
+  const double *h = h_red_;
   *rr = h[0];
   *bb = h[1];
   if (n_clamped) *n_clamped = (int)h[2];
@@ -1610,10 +1627,9 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
     }
     // r and its norm (the norm of the system given: for the block-scaled
     // system, the block-Jacobi-scaled residual) for the stopping test
-    spmv_launch<T, OP_RESID>(A, x, r, b, nullptr, sl0, sl0.result, nullptr, s_, 0.0);
-    double h0[3];
-    UFE_HIP(hipMemcpyAsync(h0, sl0.result, sizeof(h0), hipMemcpyDeviceToHost, s_));
+    spmv_launch<T, OP_RESID>(A, x, r, b, nullptr, sl0, h_red_, nullptr, s_, 0.0);
     UFE_HIP(hipStreamSynchronize(s_));
+    const double h0[2] = {h_red_[0], h_red_[1]};
     double rn = std::sqrt(h0[0]);
     if (restart == 0) {
       st.r0 = rn;
@@ -1626,7 +1642,7 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
     }
     hipLaunchKernelGGL(k_bicg_init<T>, dim3(blocks_for(nb)), dim3(kBlock), 0, s_, nb, reinterpret_cast<V2 *>(r),
                        reinterpret_cast<V2 *>(rhat), reinterpret_cast<V2 *>(p), reinterpret_cast<V2 *>(v),
-                       sl0.result, 0.0, tol_abs, maxit - total_its, sc);
+                       h0[0], h0[1], 0.0, tol_abs, maxit - total_its, sc);
     UFE_LAUNCH_CHECK();
     bool finished = false;
     const bool timing = time_spmv_ && std::is_same<T, double>::value;
@@ -1686,7 +1702,6 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
       } else {
         for (int k = 0; k < chunk; ++k) launch_iter(k);
       }
-      UFE_HIP(hipMemcpyAsync(h_scal_, sc, sizeof(KrylovScalars), hipMemcpyDeviceToHost, s_));
       UFE_HIP(hipStreamSynchronize(s_));
       if (verbose_ > 1)
         std::fprintf(stderr, "[ufe:krylov%s] its %d |r| %.3e tol %.3e rho %.3e omega %.3e done %d\n",
@@ -1726,11 +1741,9 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
     st.status = h_scal_->done;
     // verify the true residual (recurrence drift, breakdown) and restart if needed
     RedSlot sl3 = slot(3);
-    spmv_launch<T, OP_RESID>(A, x, t, b, nullptr, sl3, sl3.result, nullptr, s_, 0.0);
-    double hr[3];
-    UFE_HIP(hipMemcpyAsync(hr, sl3.result, sizeof(hr), hipMemcpyDeviceToHost, s_));
+    spmv_launch<T, OP_RESID>(A, x, t, b, nullptr, sl3, h_red_, nullptr, s_, 0.0);
     UFE_HIP(hipStreamSynchronize(s_));
-    st.rel = std::sqrt(hr[0]);
+    st.rel = std::sqrt(h_red_[0]);
     if (st.rel <= tol_abs * 1.0001) { st.status = 1; break; }
     if (total_its >= maxit) { st.status = 3; break; }
     zero_guess = false;
@@ -1793,10 +1806,9 @@ constexpr int kGmresGrid = 512;
 
 // v0 = r / ||r||, g = (||r||, 0, ...), cycle counters reset
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_gmres_init(long n, T *__restrict__ v0, const double *__restrict__ rr,
-                                                       double tol_abs, int maxit, KrylovScalars *__restrict__ sc,
+__global__ void __launch_bounds__(kBlock) k_gmres_init(long n, T *__restrict__ v0, double beta, double tol_abs,
+                                                       int maxit, KrylovScalars *__restrict__ sc,
                                                        GmresScalars *__restrict__ gs) {
-  const double beta = sqrt(rr[0]);
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (i < n) v0[i] = (T)((double)v0[i] / beta);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -1809,6 +1821,7 @@ __global__ void __launch_bounds__(kBlock) k_gmres_init(long n, T *__restrict__ v
     sc->maxit = maxit;
     sc->tol2 = tol_abs * tol_abs;
     sc->rr = beta * beta;
+    publish(sc);
   }
 }
 
@@ -2019,6 +2032,7 @@ __global__ void __launch_bounds__(kBlock) k_gmres_norm_finish(int nparts, const 
     else if (res * res <= sc->tol2 || hn == 0.0) sc->done = 1;  // converged, or the Krylov space is invariant
     else if (r == 0.0) sc->done = 2;
     else if (sc->its >= sc->maxit) sc->done = 3;
+    publish(sc);
   }
   __syncthreads();
   if ((int)threadIdx.x <= j) Hj[threadIdx.x] = H[threadIdx.x];
@@ -2102,11 +2116,9 @@ SolveStats Krylov::gmres(const BsrT<T> &A, const T *b, T *x, double rtol, double
   const int pred0 = last_gmres_its_[sizeof(T) == 4];
   for (int cycle = 0;; ++cycle) {
     // true residual into v0 (the norm of the system given)
-    residual<T>(A, x, V, b, sl0, sl0.result);
-    double h0[3];
-    UFE_HIP(hipMemcpyAsync(h0, sl0.result, sizeof(h0), hipMemcpyDeviceToHost, s_));
+    residual<T>(A, x, V, b, sl0, h_red_);
     UFE_HIP(hipStreamSynchronize(s_));
-    const double rn = std::sqrt(h0[0]);
+    const double rn = std::sqrt(h_red_[0]);
     if (cycle == 0) {
       st.r0 = rn;
       tol_abs = std::max(rtol * rn, abstol);
@@ -2115,7 +2127,7 @@ SolveStats Krylov::gmres(const BsrT<T> &A, const T *b, T *x, double rtol, double
     if (!std::isfinite(rn)) { st.status = 2; break; }
     if (rn <= tol_abs * (cycle ? 1.0001 : 1.0)) { st.status = 1; break; }
     if (total >= maxit) { st.status = 3; break; }
-    hipLaunchKernelGGL(k_gmres_init<T>, dim3(blocks_for(n)), dim3(kBlock), 0, s_, n, V, sl0.result, tol_abs,
+    hipLaunchKernelGGL(k_gmres_init<T>, dim3(blocks_for(n)), dim3(kBlock), 0, s_, n, V, rn, tol_abs,
                        maxit - total, sc, gs);
     UFE_LAUNCH_CHECK();
     int j = 0, seen = 0;
@@ -2145,7 +2157,6 @@ SolveStats Krylov::gmres(const BsrT<T> &A, const T *b, T *x, double rtol, double
         hipLaunchKernelGGL(k_gmres_norm_finish, dim3(1), dim3(kBlock), 0, s_, grid, npart, gs, j, sc);
         UFE_LAUNCH_CHECK();
       }
-      UFE_HIP(hipMemcpyAsync(h_scal_, sc, sizeof(KrylovScalars), hipMemcpyDeviceToHost, s_));
       UFE_HIP(hipStreamSynchronize(s_));
       if (verbose_ > 1)
         std::fprintf(stderr, "[ufe:gmres%s] cycle %d its %d |r| %.3e tol %.3e done %d\n", sizeof(T) == 4 ? "32" : "64",

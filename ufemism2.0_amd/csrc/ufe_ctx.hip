@@ -51,14 +51,14 @@ struct ufe_ctx {
   bool grounded_exists = true;
   bool inputs_ready = false;
   // iterate and work arrays
-  DBuf u, uprev, x, rhs, r64, tdx, tdy, N_a, beta_a, beta_eff_a, tri_coef, beta_basal_b, out2;
+  DBuf u, uprev, x, rhs, r64, tdx, tdy, N_a, beta_a, beta_eff_a, tri_coef, beta_basal_b;
   // DIVA
   DBuf eta3b, eta3a, F1a, F2a, F1b, F2b0, ubase, taub, tmp3;
   DBuf beta_save;  // beta_b kept aside while the diagnostic residual is evaluated
   bool diva_state_ready = false;
   // Anderson mixing: ring of m difference columns (dF, dG), previous f and G,
   // reduction slot of width 2 kAAMaxDepth + 1
-  DBuf aa_dF, aa_dG, aa_fprev, aa_gprev, aa_part, aa_out;
+  DBuf aa_dF, aa_dG, aa_fprev, aa_gprev, aa_part;
   std::unique_ptr<Krylov> kry;
   std::unique_ptr<AmgHierarchy> amg;
   std::string err;
@@ -424,11 +424,10 @@ static double unscaled_rel_residual(ufe_ctx *c) {
   hipLaunchKernelGGL(k_unscaled_norms, dim3(nb), dim3(kBlock), 0, c->s, nT, c->r64.as<double2>(),
                      c->rhs.as<double2>(), c->u.as<double2>(), c->prm.vel_max, sl);
   UFE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_partials_out<2>, dim3(1), dim3(kBlock), 0, c->s, sl, nb, sl.result);
+  hipLaunchKernelGGL(k_partials_out<2>, dim3(2), dim3(kBlock), 0, c->s, sl, nb, c->h_scalars);
   UFE_LAUNCH_CHECK();
-  double h[2];
-  UFE_HIP(hipMemcpyAsync(h, sl.result, sizeof(h), hipMemcpyDeviceToHost, c->s));
   UFE_HIP(hipStreamSynchronize(c->s));
+  const double *h = c->h_scalars;
   return h[1] > 0 ? std::sqrt(h[0] / h[1]) : std::sqrt(h[0]);
 }
 
@@ -483,14 +482,13 @@ static void aa_prepare(ufe_ctx *c) {
     c->aa_fprev.alloc(n * sizeof(double));
     c->aa_gprev.alloc(n * sizeof(double));
     c->aa_part.alloc(sizeof(double) * kMaxPartials * (2 * kAAMaxDepth + 1));
-    c->aa_out.alloc(sizeof(double) * (2 * kAAMaxDepth + 1));
   }
 }
 
 static void aa_step(ufe_ctx *c, AndersonState &aa, double resid) {
   const ufe_params &q = c->prm;
   const AndersonBuffers buf{c->aa_dF.as<double>(), c->aa_dG.as<double>(), c->aa_fprev.as<double>(),
-                            c->aa_gprev.as<double>(), c->aa_part.as<double>(), c->aa_out.as<double>()};
+                            c->aa_gprev.as<double>(), c->aa_part.as<double>(), c->h_scalars + 8};
   anderson_step(aa, buf, q.accel_depth, q.accel_mixing, q.accel_restart, q.vel_max, c->m.nT, c->x.as<double>(),
                 c->u.as<double>(), resid, c->s);
 }
@@ -557,12 +555,11 @@ static int run_picard(ufe_ctx *c, bool diva, ufe_solve_info *info) {
     RedSlot sl = c->kry->slot(3);
     launch_update(nT, c->x.as<double>(), c->u.as<double>(), c->uprev.as<double>(), q.vel_max,
                   q.accel_depth > 0 ? 1.0 : relax, sl,
-                  c->out2.as<double>(), c->beta_basal_b.as<double>(), c->tri_coef.as<double4>(),
+                  c->h_scalars, c->beta_basal_b.as<double>(), c->tri_coef.as<double4>(),
                   diva ? c->F2b0.as<double>() : nullptr, q.sliding_law == UFE_SLIDING_NO_SLIDING,
                   diva ? c->ubase.as<double>() : nullptr, diva ? c->taub.as<double>() : nullptr, s);
-    double h2[2];
-    UFE_HIP(hipMemcpyAsync(h2, c->out2.p, sizeof(h2), hipMemcpyDeviceToHost, s));
     UFE_HIP(hipStreamSynchronize(s));
+    const double h2[2] = {c->h_scalars[0], c->h_scalars[1]};
     float ms;
     for (int k = 0; k < 3; ++k) {
       UFE_HIP(hipEventElapsedTime(&ms, c->ev[k], c->ev[k + 1]));
@@ -922,10 +919,10 @@ extern "C" int ufe_ctx_create(ufe_ctx **out, int device, const ufe_mesh_desc *md
     for (DBuf *b : {&c->eta3a, &c->F1a, &c->F2a, &c->A_vk_vf, &c->A_vk_lf, &c->Apow_lf})
       b->alloc(sizeof(double) * (size_t)nV * nz);
     for (DBuf *b : {&c->eta3b, &c->F1b, &c->tmp3}) b->alloc(sizeof(double) * (size_t)nT * nz);
-    c->out2.alloc(sizeof(double) * 4);
     UFE_HIP(hipMemset(c->u.p, 0, v2));
     c->kry = std::make_unique<Krylov>(nT, c->s);
-    UFE_HIP(hipHostMalloc((void **)&c->h_scalars, 8 * sizeof(double), hipHostMallocDefault));
+    // [0, 8) two- and three-value results, [8, 8 + 2 kAAMaxDepth + 1) the Anderson products
+    UFE_HIP(hipHostMalloc((void **)&c->h_scalars, (8 + 2 * kAAMaxDepth + 1) * sizeof(double), hipHostMallocDefault));
     {
       const char *e;
       double om = (e = std::getenv("UFE_AMG_OMEGA")) ? std::atof(e) : 0.85;

@@ -61,6 +61,9 @@ struct KrylovScalars {
   int its;
   int maxit;
   int pad;
+  // pinned host memory that the kernels which change rr, its or done write them
+  // to as well: the host reads it after waiting for the stream, without a copy
+  KrylovScalars *host;
 };
 
 // Wavefront-wide sum with cross-lane shuffles (wave64).
@@ -109,10 +112,9 @@ __device__ __forceinline__ void block_partials(const RedSlot &slot, const double
 // one-workgroup launch of BS threads.  The loads of all W values are issued
 // together, U per thread and value in flight (U = 8 for W <= 4), so that up to
 // U * BS partials cost one memory round trip.
-template <int W, int BS = kBlock>
+template <int W, int BS = kBlock, int U = (W > 4 ? 2 : 8)>
 __device__ __forceinline__ void partials_sum(const RedSlot &slot, int nparts, double (&out)[W]) {
   __shared__ double lds[W][BS / 64];
-  constexpr int U = W > 4 ? 2 : 8;
   double s[W][U];
 #pragma unroll
   for (int i = 0; i < W; ++i)
@@ -137,15 +139,16 @@ __device__ __forceinline__ void partials_sum(const RedSlot &slot, int nparts, do
   block_sum<W, BS>(out, lds);
 }
 
-// Second phase writing the W totals to out[0..W).
+// Second phase writing the W totals to out[0..W), one workgroup per value (17
+// values in one workgroup took 23 us, 2 took 3 us as they do now).  out may be
+// pinned host memory: the host then needs no copy.
 template <int W>
 __global__ void __launch_bounds__(kBlock) k_partials_out(RedSlot slot, int nparts, double *__restrict__ out) {
-  double tot[W];
-  partials_sum<W>(slot, nparts, tot);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int i = 0; i < W; ++i) out[i] = tot[i];
-  }
+  RedSlot one = slot;
+  one.partials = slot.partials + (size_t)blockIdx.x * kMaxPartials;
+  double tot[1];
+  partials_sum<1, kBlock, (W > 4 ? 2 : 8)>(one, nparts, tot);
+  if (threadIdx.x == 0) out[blockIdx.x] = tot[0];
 }
 
 }  // namespace ufe
