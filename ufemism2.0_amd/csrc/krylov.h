@@ -206,7 +206,7 @@ class Krylov {
   template <typename T> SolveStats gmres(const BsrT<T> &A, const T *b, T *x, double rtol, double abstol, int maxit,
                                          bool zero_guess, int restart, int check_every);
   template <typename T> void precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0 = nullptr,
-                                           hipEvent_t ev1 = nullptr);
+                                           hipEvent_t ev1 = nullptr, bool presmoothed = false);
   template <typename T> void amg_setup(const BsrT<T> &A0);
   template <typename T> AmgValues<T> &amg_vals();
 

@@ -165,11 +165,21 @@ __global__ void __launch_bounds__(kFinishBlock) k_spmv_finish(RedSlot slot, int 
 // lanes per block row: 8 for rows averaging 20 blocks or more, else kSpmvLpr
 inline int spmv_lanes(int nb, long nnzb) { return nnzb >= 20L * nb ? 8 : kSpmvLpr; }
 
+// Partial sums up to which the kernel after a dot product adds them itself
+// (fold_sums) instead of a one-workgroup launch in between (3.7 to 4.1 us, twice
+// per BiCGStab iteration).  Every workgroup reads them all, so the reads grow
+// with the square of the system: 2 MB per kernel at 1,024 partials (65k block
+// rows), 76 MB at the 200k-vertex channel's 6,168, more than its finish kernel
+// takes (8 us).
+constexpr int kFoldParts = 1024;
+
+// Returns the number of partial sums left in the slot for the next kernel to
+// add (fold, with a dot epilogue and few workgroups), else 0.
 template <typename T, int OP>
-static void spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T *w, const RedSlot &slot,
+static int spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T *w, const RedSlot &slot,
                         double *out, KrylovScalars *sc, hipStream_t s, double vmax = 0.0,
                         const typename VecT<T>::V4 *dblk = nullptr, int write_unscaled = 0,
-                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
+                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr, bool fold = false) {
   using V2 = typename VecT<T>::V2;
   const int lpr = spmv_lanes(A.nb, A.nnzb);
   long threads = (long)A.nb * lpr;
@@ -193,10 +203,12 @@ static void spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T 
                        write_unscaled);
   UFE_LAUNCH_CHECK();
   if (ev1) UFE_HIP(hipEventRecord(ev1, s));
+  if (fold && nblk <= kFoldParts) return nblk;
   if (OP != OP_PLAIN) {
     hipLaunchKernelGGL((k_spmv_finish<OP>), dim3(1), dim3(kFinishBlock), 0, s, slot, nblk, out, sc);
     UFE_LAUNCH_CHECK();
   }
+  return 0;
 }
 
 // y = A x through the caller's operator when the system has no stored blocks
@@ -249,6 +261,63 @@ __device__ __forceinline__ typename VecT<T>::V2 pc_local(int pc, const typename 
   return z;
 }
 
+// The V-cycle's per-row arithmetic is written with explicit fused multiply-adds
+// and separately rounded products, so every kernel that inlines it (the
+// per-level kernels, the one-workgroup coarse kernel, with or without the
+// folded pre-smoothing) rounds identically whatever the compiler contracts.
+__device__ __forceinline__ double mul_rn(double a, double b) { return __dmul_rn(a, b); }
+__device__ __forceinline__ float mul_rn(float a, float b) { return __fmul_rn(a, b); }
+
+// The totals of k_spmv_finish (1,024 threads) for up to kFoldParts partials,
+// the same additions in the same order, valid in every thread of a kBlock
+// workgroup.
+template <int W>
+__device__ __forceinline__ void fold_sums(const RedSlot &slot, int nparts, double (&tot)[W]) {
+  constexpr int G = kFoldParts / kBlock, NW = kFoldParts / 64;
+  static_assert(kFoldParts == kFinishBlock, "the finish kernel's wavefronts");
+  __shared__ double lds[W][NW];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  double v[W][G];
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      const int b = q * kBlock + (int)threadIdx.x;
+      v[i][q] = b < nparts ? slot.partials[(size_t)i * kMaxPartials + b] : 0.0;
+    }
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      const double t = wave_sum(v[i][q]);
+      if (lane == 0) lds[i][q * (kBlock / 64) + wid] = t;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    double t = 0.0;
+    for (int q = 0; q < NW; ++q) t += lds[i][q];
+    tot[i] = t;
+  }
+}
+
+// The V-cycle's pre-smoothing from zero of the vector that an update writes,
+// z = omega D^-1 q, in the update (k_amg_presmooth's arithmetic, bit for bit).
+template <typename T>
+struct Presmooth {
+  typename VecT<T>::V2 *z;  // null: none
+  const typename VecT<T>::V4 *dinv;
+  T omega;
+};
+template <typename T>
+__device__ __forceinline__ typename VecT<T>::V2 presmoothed(const typename VecT<T>::V4 &d, T omega,
+                                                            const typename VecT<T>::V2 &q) {
+  typename VecT<T>::V2 o;
+  o.x = mul_rn(omega, fma(d.x, q.x, mul_rn(d.y, q.y)));
+  o.y = mul_rn(omega, fma(d.w, q.y, mul_rn(d.z, q.x)));
+  return o;
+}
+
 // p = r + beta (p - omega v); phat = M p   (beta from the device scalars)
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_bicg_p(int nb, const typename VecT<T>::V2 *__restrict__ r,
@@ -257,7 +326,8 @@ __global__ void __launch_bounds__(kBlock) k_bicg_p(int nb, const typename VecT<T
                                                    typename VecT<T>::V2 *__restrict__ phat, int pc,
                                                    const typename VecT<T>::V4 *__restrict__ dinv,
                                                    const typename VecT<T>::V4 *__restrict__ aval,
-                                                   const int *__restrict__ diag, const KrylovScalars *__restrict__ sc) {
+                                                   const int *__restrict__ diag, Presmooth<T> pre,
+                                                   const KrylovScalars *__restrict__ sc) {
   if (sc->done) return;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nb) return;
@@ -268,9 +338,12 @@ __global__ void __launch_bounds__(kBlock) k_bicg_p(int nb, const typename VecT<T
   pp.y = rr.y + beta * (pp.y - om * vv.y);
   p[i] = pp;
   if (phat) phat[i] = pc_local<T>(pc, dinv, aval, diag, i, pp);
+  if (pre.z) pre.z[i] = presmoothed<T>(pre.dinv[i], pre.omega, pp);
 }
 
-// s = r - alpha v; shat = M s
+// s = r - alpha v; shat = M s.  nparts > 0: the partials of (rhat, v) are added
+// here (every workgroup), alpha = rho / (rhat, v), and the first workgroup
+// stores it; on a breakdown no workgroup goes on.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_bicg_s(int nb, const typename VecT<T>::V2 *__restrict__ r,
                                                    const typename VecT<T>::V2 *__restrict__ v,
@@ -278,19 +351,36 @@ __global__ void __launch_bounds__(kBlock) k_bicg_s(int nb, const typename VecT<T
                                                    typename VecT<T>::V2 *__restrict__ shat, int pc,
                                                    const typename VecT<T>::V4 *__restrict__ dinv,
                                                    const typename VecT<T>::V4 *__restrict__ aval,
-                                                   const int *__restrict__ diag, const KrylovScalars *__restrict__ sc) {
+                                                   const int *__restrict__ diag, Presmooth<T> pre, RedSlot slot,
+                                                   int nparts, KrylovScalars *__restrict__ sc) {
   if (sc->done) return;
+  double alpha;
+  if (nparts > 0) {
+    double tot[1];
+    fold_sums<1>(slot, nparts, tot);
+    const bool bad = tot[0] == 0.0 || !std::isfinite(tot[0]);
+    alpha = sc->rho / tot[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      if (bad) sc->done = sc->host->done = 2;
+      else sc->alpha = alpha;
+    }
+    if (bad) return;
+  } else {
+    alpha = sc->alpha;
+  }
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nb) return;
-  T al = (T)sc->alpha;
+  T al = (T)alpha;
   typename VecT<T>::V2 rr = r[i], vv = v[i], ss;
   ss.x = rr.x - al * vv.x;
   ss.y = rr.y - al * vv.y;
   s[i] = ss;
   if (shat) shat[i] = pc_local<T>(pc, dinv, aval, diag, i, ss);
+  if (pre.z) pre.z[i] = presmoothed<T>(pre.dinv[i], pre.omega, ss);
 }
 
-// x += alpha phat + omega shat; r = s - omega t; rho_new = (rhat, r); ||r||^2
+// x += alpha phat + omega shat; r = s - omega t; rho_new = (rhat, r); ||r||^2.
+// nparts > 0: omega = (t, s) / (t, t) from the partials, as in k_bicg_s.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_bicg_x(int nb, typename VecT<T>::V2 *__restrict__ x,
                                                    const typename VecT<T>::V2 *__restrict__ phat,
@@ -299,9 +389,18 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x(int nb, typename VecT<T>::V2 
                                                    const typename VecT<T>::V2 *__restrict__ t,
                                                    typename VecT<T>::V2 *__restrict__ r,
                                                    const typename VecT<T>::V2 *__restrict__ rhat, RedSlot slot,
-                                                   KrylovScalars *__restrict__ sc) {
+                                                   RedSlot dots, int nparts, KrylovScalars *__restrict__ sc) {
   if (sc->done) return;
-  T al = (T)sc->alpha, om = (T)sc->omega;
+  double omega;
+  if (nparts > 0) {
+    double tot[2];
+    fold_sums<2>(dots, nparts, tot);
+    omega = tot[1] > 0.0 ? tot[0] / tot[1] : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc->omega = omega;
+  } else {
+    omega = sc->omega;
+  }
+  T al = (T)sc->alpha, om = (T)omega;
   double acc[2] = {0.0, 0.0};
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += gridDim.x * blockDim.x) {
     typename VecT<T>::V2 xx = x[i], ph = phat[i], sh = shat[i], ss = s[i], tt = t[i], rh = rhat[i], rr;
@@ -463,12 +562,6 @@ __global__ void __launch_bounds__(kBlock) k_l1_dinv(int nb, const int *__restric
 }
 
 // z0 = omega D0^-1 r0  (pre-smoothing from a zero guess on the finest level)
-// The V-cycle's per-row arithmetic is written with explicit fused multiply-adds
-// and separately rounded products, so every kernel that inlines it (the
-// per-level kernels, the one-workgroup coarse kernel, with or without the
-// folded pre-smoothing) rounds identically whatever the compiler contracts.
-__device__ __forceinline__ double mul_rn(double a, double b) { return __dmul_rn(a, b); }
-__device__ __forceinline__ float mul_rn(float a, float b) { return __fmul_rn(a, b); }
 
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_amg_presmooth(int nb, const typename VecT<T>::V2 *__restrict__ r,
@@ -478,11 +571,7 @@ __global__ void __launch_bounds__(kBlock) k_amg_presmooth(int nb, const typename
   if (sc && sc->done) return;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nb) return;
-  typename VecT<T>::V2 q = r[i], o;
-  typename VecT<T>::V4 d = dinv[i];
-  o.x = mul_rn(omega, fma(d.x, q.x, mul_rn(d.y, q.y)));
-  o.y = mul_rn(omega, fma(d.w, q.y, mul_rn(d.z, q.x)));
-  z[i] = o;
+  z[i] = presmoothed<T>(dinv[i], omega, r[i]);
 }
 
 // Per-row bodies of the V-cycle passes, shared by the grid-wide kernels (fine
@@ -1345,7 +1434,7 @@ void Krylov::amg_setup64(const BsrT<double> &A0) { amg_setup<double>(A0); }
 void Krylov::amg_setup32(const BsrT<float> &A0) { amg_setup<float>(A0); }
 
 template <typename T>
-void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, hipEvent_t ev1) {
+void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, hipEvent_t ev1, bool presmoothed) {
   using V2 = typename VecT<T>::V2;
   using V4 = typename VecT<T>::V4;
   AmgValues<T> &av = amg_vals<T>();
@@ -1369,7 +1458,7 @@ void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, h
   const bool fold = unit_diag0_ && !amg_l1_;
   const V2 *zl0 = fold ? rl : z0;
   const T zs0 = fold ? om : T(1);
-  if (!fold) {
+  if (!fold && !presmoothed) {
     hipLaunchKernelGGL(k_amg_presmooth<T>, dim3(blocks_for(lev[0].nb)), dim3(kBlock), 0, s_, lev[0].nb, rl,
                        lev[0].dinv, om, z0, sc);
     UFE_LAUNCH_CHECK();
@@ -1663,27 +1752,39 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
     // device, so the chunking does not change the result.
     // One BiCGStab iteration: every kernel returns at once after convergence
     // (device flag), so a chunk may run past it.  k picks the timing events.
+    // with a V-cycle whose finest pre-smoothing is a pass of its own, the
+    // updates of p and s write it
+    Presmooth<T> pre{nullptr, nullptr, T(0)};
+    if (amg && amg_->n_levels() > 1 && !(unit_diag0_ && !amg_l1_)) {
+      std::vector<BsrT<T>> &lev = std::is_same<T, double>::value ? *reinterpret_cast<std::vector<BsrT<T>> *>(&lev64_)
+                                                                 : *reinterpret_cast<std::vector<BsrT<T>> *>(&lev32_);
+      pre = Presmooth<T>{amg_vals<T>().z[0]->template as<V2>(), lev[0].dinv, (T)amg_omega_};
+    }
     auto launch_iter = [&](int k) {
       hipLaunchKernelGGL(k_bicg_p<T>, dim3(blocks_for(nb)), dim3(kBlock), 0, s_, nb,
                          reinterpret_cast<const V2 *>(r), reinterpret_cast<V2 *>(p), reinterpret_cast<const V2 *>(v),
-                         reinterpret_cast<V2 *>(amg ? (T *)nullptr : phat), pcl, A.dinv, A.val, A_diag_, sc);
+                         reinterpret_cast<V2 *>(amg ? (T *)nullptr : phat), pcl, A.dinv, A.val, A_diag_, pre, sc);
       UFE_LAUNCH_CHECK();
       if (amg)
-        precond_apply<T>(A, p, phat, timing ? tev_[8 * k + 4] : nullptr, timing ? tev_[8 * k + 5] : nullptr);
-      spmv_launch<T, OP_DOT1>(A, phat, v, nullptr, rhat, sl1, nullptr, sc, s_, 0.0, nullptr, 0,
-                              timing ? tev_[8 * k] : nullptr, timing ? tev_[8 * k + 1] : nullptr);
+        precond_apply<T>(A, p, phat, timing ? tev_[8 * k + 4] : nullptr, timing ? tev_[8 * k + 5] : nullptr,
+                         pre.z != nullptr);
+      const int n1 = spmv_launch<T, OP_DOT1>(A, phat, v, nullptr, rhat, sl1, nullptr, sc, s_, 0.0, nullptr, 0,
+                                             timing ? tev_[8 * k] : nullptr, timing ? tev_[8 * k + 1] : nullptr, true);
       hipLaunchKernelGGL(k_bicg_s<T>, dim3(blocks_for(nb)), dim3(kBlock), 0, s_, nb,
                          reinterpret_cast<const V2 *>(r), reinterpret_cast<const V2 *>(v), reinterpret_cast<V2 *>(s),
-                         reinterpret_cast<V2 *>(amg ? (T *)nullptr : shat), pcl, A.dinv, A.val, A_diag_, sc);
+                         reinterpret_cast<V2 *>(amg ? (T *)nullptr : shat), pcl, A.dinv, A.val, A_diag_, pre, sl1, n1,
+                         sc);
       UFE_LAUNCH_CHECK();
       if (amg)
-        precond_apply<T>(A, s, shat, timing ? tev_[8 * k + 6] : nullptr, timing ? tev_[8 * k + 7] : nullptr);
-      spmv_launch<T, OP_DOT2>(A, shat, t, nullptr, s, sl2, nullptr, sc, s_, 0.0, nullptr, 0,
-                              timing ? tev_[8 * k + 2] : nullptr, timing ? tev_[8 * k + 3] : nullptr);
+        precond_apply<T>(A, s, shat, timing ? tev_[8 * k + 6] : nullptr, timing ? tev_[8 * k + 7] : nullptr,
+                         pre.z != nullptr);
+      const int n2 = spmv_launch<T, OP_DOT2>(A, shat, t, nullptr, s, sl2, nullptr, sc, s_, 0.0, nullptr, 0,
+                                             timing ? tev_[8 * k + 2] : nullptr, timing ? tev_[8 * k + 3] : nullptr,
+                                             true);
       hipLaunchKernelGGL(k_bicg_x<T>, dim3(nbx), dim3(kBlock), 0, s_, nb, reinterpret_cast<V2 *>(x),
                          reinterpret_cast<const V2 *>(phat), reinterpret_cast<const V2 *>(shat),
                          reinterpret_cast<const V2 *>(s), reinterpret_cast<const V2 *>(t), reinterpret_cast<V2 *>(r),
-                         reinterpret_cast<const V2 *>(rhat), sl0, sc);
+                         reinterpret_cast<const V2 *>(rhat), sl0, sl2, n2, sc);
       UFE_LAUNCH_CHECK();
       hipLaunchKernelGGL(k_bicg_x_finish, dim3(1), dim3(kBlock), 0, s_, sl0, nbx, sc);
       UFE_LAUNCH_CHECK();
