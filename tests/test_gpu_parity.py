@@ -293,6 +293,31 @@ def test_amg_tail_in_lds_equals_the_one_in_device_memory(V, channel_fixtures, mo
     assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
 
 
+@pytest.mark.parametrize("h", [9e3, 6e3, 4.5e3])
+def test_coarse_inverse_at_the_ends_of_its_range(V, W, L, OB, h):
+    """Linear ice (n = m = 1) on 14, 28 and 46 triangles.  14 is a hierarchy of
+    one level, where the dense inverse, whose elimination swaps rows here, is
+    the preconditioner: good to epsilon times the condition, 5e6, or 1e-9, so
+    one iteration reaches 1e-6; the others restrict to a coarse level.  The
+    residual 1e-12 leaves at most 5e-6 in the velocities."""
+    from ufemism2_amd.mesh import uniform_mesh
+    mesh = uniform_mesh(-9e3, 9e3, -9e3, 9e3, h, seed=1)
+    nV = mesh.nV
+    w = W.Workload("slab", mesh, W.build_operators(mesh), W.zeta_regular(10),
+                   np.random.default_rng(2).uniform(1500.0, 2500.0, nV), np.zeros(nV), np.zeros(nV),
+                   np.full(10 * nV, 1e-16), np.full(nV, 1e7), 1, "SSA")
+    kw = dict(glens_n=1.0, sliding_law=1, slid_weertman_m=1.0, visc_it_norm_dUV_tol=1e-8, abstol=0.0, rtol=1e-12,
+              visc_it_nit=100)
+    st, info = solve(V, w, precision=0, precond=L.PC_AMG, **kw)
+    rc, uo, vo, io = OB.Oracle(w.descriptor()).solve_ssa(params(L, **kw), w.inputs())
+    print(f"{mesh.nT} triangles: picard {info.n_visc_its} krylov {info.n_Axb_its}", flush=True)
+    assert rc == 0 and info.n_visc_its == io.n_visc_its
+    assert max_rel(st["u_vav_b"], uo) < 5e-6 and max_rel(st["v_vav_b"], vo) < 5e-6
+    if mesh.nT <= 24:
+        _, info = solve(V, w, precision=0, precond=L.PC_AMG, **dict(kw, rtol=1e-6))
+        assert info.n_Axb_its == info.n_visc_its
+
+
 @pytest.mark.parametrize("nz", [10, 12])
 def test_diva_column_kernels_equal_per_thread_kernels(V, W, monkeypatch, nz):
     """The DIVA vertex and triangle kernels with 16 lanes per column (the

