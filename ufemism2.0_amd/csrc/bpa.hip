@@ -1021,7 +1021,7 @@ void bpa_pattern(ufe_ctx *c, BpaState &b) {
   ensure(b.part, sizeof(double) * kMaxPartials * 2);
   b.kry = std::make_unique<Krylov>(b.nb, s);
   set_operator(c, b);
-  for (hipEvent_t &ev : b.ev) UFE_HIP(hipEventCreate(&ev));
+  for (hipEvent_t &ev : b.ev) UFE_HIP(hipEventCreateWithFlags(&ev, hipEventDisableSystemFence));
 }
 
 BpaParams bpa_params(const ufe_ctx *c, double eps0_applied) {

@@ -151,9 +151,11 @@ class Krylov {
   void set_graphs(bool on) { use_graphs_ = on; }
 
   // BiCGStab: x in (initial guess unless zero_guess) / out.  Stops when
-  // ||r|| <= max(rtol*||r0||, abstol).
+  // ||r|| <= max(rtol*||r0||, abstol).  r0 (with zero_guess false): tmp64(0) already
+  // holds b - A x of this A, b and x, and r0 its ||b - A x||^2 and ||b||^2 (residual64
+  // over all rows): they are not formed again.
   SolveStats bicgstab64(const BsrT<double> &A, const double *b, double *x, double rtol, double abstol, int maxit,
-                        bool zero_guess, int check_every);
+                        bool zero_guess, int check_every, const double *r0 = nullptr);
   SolveStats bicgstab32(const BsrT<float> &A, const float *b, float *x, double rtol, double abstol, int maxit,
                         bool zero_guess, int check_every);
 
@@ -199,7 +201,7 @@ class Krylov {
 
  private:
   template <typename T> SolveStats bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, double abstol,
-                                            int maxit, bool zero_guess, int check_every);
+                                            int maxit, bool zero_guess, int check_every, const double *r0);
   template <typename T> std::vector<uintptr_t> graph_key(const BsrT<T> &A, const T *b, const T *x, int nbx);
   template <typename T> hipGraphExec_t iteration_graph(int n, const std::function<void(int)> &launch_iter,
                                                        const BsrT<T> &A, const T *b, T *x, int nbx);

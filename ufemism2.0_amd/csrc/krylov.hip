@@ -1735,7 +1735,7 @@ void Krylov::GraphCache::clear() {
 
 template <typename T>
 SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, double abstol, int maxit,
-                            bool zero_guess, int check_every) {
+                            bool zero_guess, int check_every, const double *r0) {
   using V2 = typename VecT<T>::V2;
   T *r, *rhat, *p, *v, *phat, *s, *shat, *t;
   if (std::is_same<T, double>::value) {
@@ -1761,9 +1761,12 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
     }
     // r and its norm (the norm of the system given: for the block-scaled
     // system, the block-Jacobi-scaled residual) for the stopping test
-    spmv_launch<T, OP_RESID>(A, x, r, b, nullptr, sl0, h_red_, nullptr, s_, 0.0);
-    UFE_HIP(hipStreamSynchronize(s_));
-    const double h0[2] = {h_red_[0], h_red_[1]};
+    const bool known = r0 && restart == 0;
+    if (!known) {
+      spmv_launch<T, OP_RESID>(A, x, r, b, nullptr, sl0, h_red_, nullptr, s_, 0.0);
+      UFE_HIP(hipStreamSynchronize(s_));
+    }
+    const double h0[2] = {known ? r0[0] : h_red_[0], known ? r0[1] : h_red_[1]};
     double rn = std::sqrt(h0[0]);
     if (restart == 0) {
       st.r0 = rn;
@@ -1900,13 +1903,13 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
 }
 
 SolveStats Krylov::bicgstab64(const BsrT<double> &A, const double *b, double *x, double rtol, double abstol,
-                              int maxit, bool zero_guess, int check_every) {
-  return bicgstab<double>(A, b, x, rtol, abstol, maxit, zero_guess, check_every);
+                              int maxit, bool zero_guess, int check_every, const double *r0) {
+  return bicgstab<double>(A, b, x, rtol, abstol, maxit, zero_guess, check_every, r0);
 }
 
 SolveStats Krylov::bicgstab32(const BsrT<float> &A, const float *b, float *x, double rtol, double abstol,
                               int maxit, bool zero_guess, int check_every) {
-  return bicgstab<float>(A, b, x, rtol, abstol, maxit, zero_guess, check_every);
+  return bicgstab<float>(A, b, x, rtol, abstol, maxit, zero_guess, check_every, nullptr);
 }
 
 // ===========================================================================

@@ -306,19 +306,21 @@ void launch_f64_to_f32(int n, const double *a, float *b, hipStream_t s);
 
 // FP64 Krylov solve of the assembled system into c->x with the chosen method
 // (the reference's PETSc default is GMRES(30), petsc_basic.f90:106-119).
-static SolveStats krylov64(ufe_ctx *c, const BsrT<double> &A, double rtol, bool zero_guess) {
+static SolveStats krylov64(ufe_ctx *c, const BsrT<double> &A, double rtol, bool zero_guess,
+                           const double *r0 = nullptr) {
   const ufe_params &q = c->prm;
   if (q.krylov == UFE_KRYLOV_GMRES)
     return c->kry->gmres64(A, c->rhs_s.as<double>(), c->x.as<double>(), rtol, q.abstol, q.krylov_maxit, zero_guess,
                            q.gmres_restart, q.check_every);
   return c->kry->bicgstab64(A, c->rhs_s.as<double>(), c->x.as<double>(), rtol, q.abstol, q.krylov_maxit, zero_guess,
-                            q.check_every);
+                            q.check_every, r0);
 }
 
 // ---------------------------------------------------------------------------
-// Linear solve of one Picard iteration: x := solution of A x = rhs.
+// Linear solve of one Picard iteration: x := solution of A x = rhs.  norms0: the
+// residual at the iterate and its norms are at hand (loop_residual).
 // ---------------------------------------------------------------------------
-static void linear_solve(ufe_ctx *c, int *its, int *nref) {
+static void linear_solve(ufe_ctx *c, int *its, int *nref, const double *norms0) {
   const ufe_params &q = c->prm;
   int n = 2 * c->m.nT;
   Krylov &K = *c->kry;
@@ -338,7 +340,7 @@ static void linear_solve(ufe_ctx *c, int *its, int *nref) {
     BsrT<double> A = sys64(c);
     K.set_amg_fine32(q.precond_fp32 && q.precond == UFE_PC_AMG ? c->A32.as<float4>() : nullptr);
     if (q.precond == UFE_PC_AMG) K.amg_setup64(A);
-    SolveStats st = krylov64(c, A, q.rtol, !warm);
+    SolveStats st = krylov64(c, A, q.rtol, !warm, warm ? norms0 : nullptr);
     *its = st.its;
     return;
   }
@@ -395,6 +397,15 @@ static double rel_residual(ufe_ctx *c, int *n_clamped = nullptr) {
   c->kry->residual64(sys64(c), c->u.as<double>(), c->rhs_s.as<double>(), c->r64.as<double>(), &rr, &bb,
                      c->prm.vel_max, n_clamped, c->Dblk.as<double4>(), 1);
   return bb > 0 ? std::sqrt(rr / bb) : std::sqrt(rr);
+}
+
+// The same inside the viscosity loop, with the scaled residual left where a
+// warm-started BiCGStab starts from (that solve begins at the same velocity, so
+// it would form the same residual again).  norms: ||r||^2, ||b||^2 of it.
+static double loop_residual(ufe_ctx *c, int *n_clamped, double (&norms)[2]) {
+  c->kry->residual64(sys64(c), c->u.as<double>(), c->rhs_s.as<double>(), c->kry->tmp64(0), &norms[0], &norms[1],
+                     c->prm.vel_max, n_clamped);
+  return norms[1] > 0 ? std::sqrt(norms[0] / norms[1]) : std::sqrt(norms[0]);
 }
 
 // ||r|| and ||b|| of the unscaled system over rows whose velocity is below
@@ -543,12 +554,20 @@ static int run_picard(ufe_ctx *c, bool diva, ufe_solve_info *info) {
     const double eps_it = in_cont ? eps0 * std::pow(10.0, n_cont - it + 1) : eps0;
     if (q.accel_depth > 0 && it == n_cont + 1 && n_cont > 0) aa = AndersonState();
     picard_state(c, diva, eps_it, false);
+    double norms[2];
+    bool r_known = false;
     if (q.stop_rule == UFE_STOP_RESIDUAL) {
-      resid = rel_residual(c, &n_clamped);
-      if (!in_cont && resid <= q.nonlinear_rtol) { --it; converged = true; break; }
+      resid = loop_residual(c, &n_clamped, norms);
+      if (!in_cont && resid <= q.nonlinear_rtol) {
+        resid = rel_residual(c, &n_clamped);  // leaves the unscaled residual for the diagnostics below
+        --it;
+        converged = true;
+        break;
+      }
+      r_known = n_clamped == 0;  // else the norms leave rows out
     }
     int its = 0, nref = 0;
-    linear_solve(c, &its, &nref);
+    linear_solve(c, &its, &nref, r_known ? norms : nullptr);
     n_axb += its;
     n_ref += nref;
     if (q.accel_depth > 0) aa_step(c, aa, resid);
@@ -809,7 +828,8 @@ extern "C" int ufe_ctx_create(ufe_ctx **out, int device, const ufe_mesh_desc *md
     c->device = device;
     UFE_HIP(hipSetDevice(device));
     UFE_HIP(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking));
-    for (auto &e : c->ev) UFE_HIP(hipEventCreate(&e));
+    // timing-only events: no system-scope fence (no L2 writeback) when recorded
+    for (auto &e : c->ev) UFE_HIP(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
     ufe_params_default(&c->prm);
     DevMesh &m = c->m;
     m.nV = md->nV; m.nT = md->nT; m.nz = md->nz;
