@@ -423,6 +423,20 @@ def test_krylov_poll_chunks_do_not_change_the_solve(V, channel_fixtures, stress)
         assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
 
 
+@pytest.mark.parametrize("nit", [0, 3, 800])
+def test_update_sums_read_late_equal_those_read_at_once(V, dome, monkeypatch, nit):
+    """Under Anderson mixing with the residual rule an update's sums are read
+    after the next residual; with UFE_VERBOSE they are read at once.  Same
+    iteration, change norm and velocities, converged and at the iteration
+    limit."""
+    kw = dict(TIGHT, **dict(CHOSEN, visc_it_nit=nit))
+    a, ia = solve(V, dome, **kw)
+    monkeypatch.setenv("UFE_VERBOSE", "1")
+    b, ib = solve(V, dome, **kw)
+    assert ia.n_visc_its == ib.n_visc_its and ia.L2_uv == ib.L2_uv and ia.rel_residual == ib.rel_residual
+    assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
+
+
 def test_mixed_precision_matches_fp64(V, dome):
     kw = dict(stop_rule=1, nonlinear_rtol=1e-8, visc_it_nit=300, abstol=0.0, rtol=1e-10)
     a, _ = solve(V, dome, precision=0, **kw)
