@@ -138,20 +138,21 @@ __global__ void __launch_bounds__(kSpmvBlock) k_bsr_spmv(
   block_partials<3>(slot, acc);
 }
 
-// Second phase of the product's reduction (one workgroup).
+// Second phase of the product's reduction: one workgroup, for the residual one
+// per sum (a sum is one round trip to memory and the tree; three in a row took
+// 4.5 us on the domes, side by side 2.9).
 constexpr int kFinishBlock = 1024;  // the block product's partials: up to 8 * 1024 in one round trip
 template <int OP>
 __global__ void __launch_bounds__(kFinishBlock) k_spmv_finish(RedSlot slot, int nparts, double *__restrict__ out,
                                                               KrylovScalars *__restrict__ sc) {
   if (sc && sc->done) return;
-  constexpr int W = OP == OP_RESID ? 3 : OP == OP_DOT2 ? 2 : 1;
+  constexpr int W = OP == OP_DOT2 ? 2 : 1;
+  if constexpr (OP == OP_RESID) slot.partials += (size_t)blockIdx.x * kMaxPartials;
   double tot[W];
   partials_sum<W, kFinishBlock>(slot, nparts, tot);
   if (threadIdx.x != 0) return;
   if constexpr (OP == OP_RESID) {
-    out[0] = tot[0];
-    out[1] = tot[1];
-    out[2] = tot[2];
+    out[blockIdx.x] = tot[0];
   } else if constexpr (OP == OP_DOT1) {
     // alpha = rho / (rhat, v)
     if (tot[0] == 0.0 || !std::isfinite(tot[0])) sc->done = sc->host->done = 2;
@@ -205,7 +206,7 @@ static int spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T *
   if (ev1) UFE_HIP(hipEventRecord(ev1, s));
   if (fold && nblk <= kFoldParts) return nblk;
   if (OP != OP_PLAIN) {
-    hipLaunchKernelGGL((k_spmv_finish<OP>), dim3(1), dim3(kFinishBlock), 0, s, slot, nblk, out, sc);
+    hipLaunchKernelGGL((k_spmv_finish<OP>), dim3(OP == OP_RESID ? 3 : 1), dim3(kFinishBlock), 0, s, slot, nblk, out, sc);
     UFE_LAUNCH_CHECK();
   }
   return 0;
@@ -229,7 +230,7 @@ void Krylov::residual(const BsrT<T> &A, const T *x, T *y, const T *b, const RedS
   if constexpr (std::is_same<T, double>::value) {
     if (!A.val && custom_op_) {
       const int g = custom_op_(x, y, b, sl, nullptr);
-      hipLaunchKernelGGL((k_spmv_finish<OP_RESID>), dim3(1), dim3(kFinishBlock), 0, s_, sl, g, out,
+      hipLaunchKernelGGL((k_spmv_finish<OP_RESID>), dim3(3), dim3(kFinishBlock), 0, s_, sl, g, out,
                          (KrylovScalars *)nullptr);
       UFE_LAUNCH_CHECK();
       return;
