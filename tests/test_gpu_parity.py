@@ -423,6 +423,16 @@ def test_krylov_poll_chunks_do_not_change_the_solve(V, channel_fixtures, stress)
         assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
 
 
+@pytest.mark.parametrize("depth", [1, 3, 8])
+def test_anderson_columns_at_the_ends_of_their_range(V, dome, depth):
+    """One column, some, and all that the sums hold: the mixed iteration stops
+    at the same residual, so at the same velocities to the converged-solve bar."""
+    a, ia = solve(V, dome, **TIGHT, **CHOSEN)
+    b, ib = solve(V, dome, **TIGHT, **dict(CHOSEN, accel_depth=depth))
+    assert ia.rel_residual <= 1e-8 and ib.rel_residual <= 1e-8
+    assert max_rel(b["u_vav_b"], a["u_vav_b"]) < 1e-5 and max_rel(b["v_vav_b"], a["v_vav_b"]) < 1e-5
+
+
 @pytest.mark.parametrize("nit", [0, 3, 800])
 def test_update_sums_read_late_equal_those_read_at_once(V, dome, monkeypatch, nit):
     """Under Anderson mixing with the residual rule an update's sums are read
