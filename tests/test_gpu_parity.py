@@ -82,6 +82,65 @@ def test_csr_solve_vs_direct(V, OB, L, dome):
     assert its > 0 and max_rel(x, xd) < 1e-8
 
 
+def _bicgstab(A, b, rtol, restarts=4):
+    """Unpreconditioned BiCGStab from zero with the engine's rules: a breakdown
+    (rhat, A p) = 0 ends the cycle before its update, the next one starts from
+    the residual.  Returns x, the iterations and the breakdowns."""
+    x, its, broken = np.zeros_like(b), 0, 0
+    tol = rtol * np.linalg.norm(b)
+    for _ in range(restarts):
+        r = b - A @ x
+        if np.linalg.norm(r) <= tol:
+            break
+        rh, p, v, rho, rho_old, al, om = r.copy(), 0 * r, 0 * r, r @ r, 1.0, 1.0, 1.0
+        while np.linalg.norm(r) > tol:
+            p = r + (rho / rho_old) * (al / om) * (p - om * v)
+            v = A @ p
+            if rh @ v == 0.0:
+                broken += 1
+                break
+            al = rho / (rh @ v)
+            s = r - al * v
+            t = A @ s
+            om = (t @ s) / (t @ t)
+            x, r = x + al * p + om * s, s - om * t
+            rho_old, rho = rho, rh @ r
+            its += 1
+    return x, its, broken
+
+
+@pytest.mark.parametrize("copies", [1, 33, 4096, 20_000, 40_000])
+def test_bicgstab_restarts_after_a_breakdown(V, L, copies):
+    """Copies of a 4x4 system on which every scalar of the first two iterations
+    is a small dyadic number, so (rhat, A p) of the second is exactly zero in
+    any order of summation: the solve breaks down there, restarts and reaches
+    the solution in the iterations of the plain restatement (the last one takes
+    the residual from 5 to some 1e-12, so rounding decides nothing at 1e-9).
+    8 to 1,256 workgroups of the product, so both ways of adding its sums (in
+    the update up to 1,024 partials, a kernel of their own above).  The residual
+    and the condition number 4.3 bound the error."""
+    import scipy.sparse as sp
+    B = np.array([[-1.0, -1, -1, 0], [2, 0, 0, 1], [0, -1, -2, -1], [0, 2, 1, 1]])
+    bb = np.array([0.0, 0, 0, -1])
+    _, its, broken = _bicgstab(B, bb, 1e-9)
+    assert broken == 1 and its > 1
+    x, n, rel = V.csr_solve(sp.kron(sp.identity(copies), B, format="csr"), np.tile(bb, copies), rtol=1e-9, maxit=50,
+                            precond=L.PC_NONE)
+    assert n == its and rel <= 1e-9
+    assert np.linalg.norm(x - np.tile(np.linalg.solve(B, bb), copies)) <= 1e-8 * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("copies", [1, 20_000, 80_000])
+def test_bicgstab_that_breaks_down_at_once_leaves_the_guess(V, L, copies):
+    """A skew system: (r, A r) = 0 at the start of every cycle, so no iteration
+    ever runs and the guess comes back as it was."""
+    import scipy.sparse as sp
+    A = sp.kron(sp.identity(copies), np.array([[0.0, 2], [-2, 0]]), format="csr")
+    x0 = np.tile([3.0, -1.0], copies)
+    x, n, rel = V.csr_solve(A, np.tile([1.0, 5.0], copies), x0=x0, rtol=1e-12, maxit=50, precond=L.PC_NONE)
+    assert n == 0 and rel == 1.0 and np.array_equal(x, x0)
+
+
 @pytest.mark.parametrize("cross", [1, 0])
 @pytest.mark.parametrize("case", ["dome", "chan"])
 def test_ssa_residual_parity(V, OB, L, request, case, cross):

@@ -344,7 +344,9 @@ __global__ void __launch_bounds__(kBlock) k_bicg_p(int nb, const typename VecT<T
 
 // s = r - alpha v; shat = M s.  nparts > 0: the partials of (rhat, v) are added
 // here (every workgroup), alpha = rho / (rhat, v), and the first workgroup
-// stores it; on a breakdown no workgroup goes on.
+// stores it.  A breakdown goes into a word of its own, which only later launches
+// read: done is read at the entry of this one, and a wavefront that found it
+// set there would leave the others of its workgroup at the sums' barrier.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_bicg_s(int nb, const typename VecT<T>::V2 *__restrict__ r,
                                                    const typename VecT<T>::V2 *__restrict__ v,
@@ -362,10 +364,10 @@ __global__ void __launch_bounds__(kBlock) k_bicg_s(int nb, const typename VecT<T
     const bool bad = tot[0] == 0.0 || !std::isfinite(tot[0]);
     alpha = sc->rho / tot[0];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-      if (bad) sc->done = sc->host->done = 2;
+      if (bad) sc->broken = 1;
       else sc->alpha = alpha;
     }
-    if (bad) return;
+    if (bad) return;  // every workgroup alike: the same sums
   } else {
     alpha = sc->alpha;
   }
@@ -391,7 +393,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x(int nb, typename VecT<T>::V2 
                                                    typename VecT<T>::V2 *__restrict__ r,
                                                    const typename VecT<T>::V2 *__restrict__ rhat, RedSlot slot,
                                                    RedSlot dots, int nparts, KrylovScalars *__restrict__ sc) {
-  if (sc->done) return;
+  if (sc->done || sc->broken) return;
   double omega;
   if (nparts > 0) {
     double tot[2];
@@ -436,6 +438,11 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x_finish(RedSlot slot, int npar
   double tot[2];
   partials_sum<2>(slot, nparts, tot);
   if (threadIdx.x != 0) return;
+  if (sc->broken) {  // k_bicg_x left x, r and the partials as they were
+    sc->done = 2;
+    publish(sc);
+    return;
+  }
   sc->its += 1;
   sc->rho_old = sc->rho;
   sc->rho = tot[0];
@@ -474,6 +481,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_init(int nb, const typename Vec
     sc->tol2 = tol * tol;
     sc->its = 0;
     sc->maxit = maxit;
+    sc->broken = 0;
     sc->done = (rr <= sc->tol2) ? 1 : 0;
     publish(sc);
   }

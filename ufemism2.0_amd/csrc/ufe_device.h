@@ -60,7 +60,7 @@ struct KrylovScalars {
   int done;              // 0 running, 1 converged, 2 breakdown, 3 max iterations
   int its;
   int maxit;
-  int pad;
+  int broken;            // this iteration found (rhat, v) = 0 or not finite (k_bicg_s); k_bicg_x_finish ends the solve
   // pinned host memory that the kernels which change rr, its or done write them
   // to as well: the host reads it after waiting for the stream, without a copy
   KrylovScalars *host;
