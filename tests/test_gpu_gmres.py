@@ -66,6 +66,21 @@ def test_gmres_basis_passes_at_the_ends_of_their_range(V, L, n, restart):
     assert np.linalg.norm(1e9 * x - x_ex) < 3e-13 * np.linalg.norm(x_ex) + 1e-14 * np.sqrt(n)
 
 
+def test_gmres_beyond_one_partial_sum_per_4096_unknowns(V, L):
+    """8,192 workgroups of 256 x 16 unknowns and three more: the basis passes
+    take any number.  Two distinct diagonal values: solved in two steps, to the
+    rounding of a few sums of 3e7 terms."""
+    import scipy.sparse as sp
+    n = 8192 * 256 * 16 + 3
+    d = np.where(np.arange(n) % 3 == 0, 2.0, 1.0)
+    b = 1.0 + (np.arange(n) % 7)
+    A = sp.csr_matrix((d, np.arange(n, dtype=np.int32), np.arange(n + 1, dtype=np.int32)), shape=(n, n))
+    print(f"GMRES n={n}", flush=True)
+    x, its, rel = V.csr_solve(A, b, rtol=1e-12, maxit=20, krylov=L.KRYLOV_GMRES, restart=3, precond=L.PC_NONE)
+    assert its == 2 and rel <= 1e-12
+    assert np.abs(x * d - b).max() < 1e-10
+
+
 def test_gmres_argument_errors(V, L, dome):
     import scipy.sparse as sp
     A = sp.identity(10, format="csr")

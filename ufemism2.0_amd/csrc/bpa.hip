@@ -985,7 +985,8 @@ void bpa_pattern(ufe_ctx *c, BpaState &b) {
   const DevMesh &m = *ctx_mesh(c);
   hipStream_t s = ctx_stream(c);
   const int nT = b.nT, nz = b.nz;
-  if (3L * nz * m.bb_nnz >= (1L << 31)) throw std::runtime_error("BPA system too large for 32-bit block indices");
+  // points and unknowns are counted in 32 bits (the b->b entries as the mesh counts them)
+  if (2L * nT * nz >= (1L << 31)) throw std::runtime_error("BPA system too large: 2^31 unknowns or more");
   b.nb = nT * nz;
   b.bb_nnz = m.bb_nnz;
   ensure(b.ent, sizeof(BpaEntry) * (size_t)m.bb_nnz);

@@ -2259,7 +2259,6 @@ SolveStats Krylov::gmres(const BsrT<T> &A, const T *b, T *x, double rtol, double
   m = std::max(1, std::min(m, kGmresMaxRestart));
   const int nb = A.nb;
   const long n = 2L * nb;
-  if (n > (long)kMaxPartials * kBlock * 16) throw std::runtime_error("GMRES: system too large for the reduction slots");
   const int grid = std::min(blocks_for(nb), kGmresGrid);
   const size_t vbytes = sizeof(T) * (size_t)n;
   if (gm_V_.bytes < vbytes * (m + 1)) gm_V_.alloc(vbytes * (m + 1));
