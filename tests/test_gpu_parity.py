@@ -493,17 +493,41 @@ def test_anderson_columns_at_the_ends_of_their_range(V, dome, depth):
 
 
 @pytest.mark.parametrize("nit", [0, 3, 800])
-def test_update_sums_read_late_equal_those_read_at_once(V, dome, monkeypatch, nit):
+def test_update_sums_are_those_of_the_last_update(V, dome, nit):
     """Under Anderson mixing with the residual rule an update's sums are read
-    after the next residual; with UFE_VERBOSE they are read at once.  Same
-    iteration, change norm and velocities, converged and at the iteration
-    limit."""
-    kw = dict(TIGHT, **dict(CHOSEN, visc_it_nit=nit))
-    a, ia = solve(V, dome, **kw)
-    monkeypatch.setenv("UFE_VERBOSE", "1")
-    b, ib = solve(V, dome, **kw)
-    assert ia.n_visc_its == ib.n_visc_its and ia.L2_uv == ib.L2_uv and ia.rel_residual == ib.rel_residual
-    assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
+    only after the next residual.  The change norm reported, at the iteration
+    limit and converged, is that of the last update: 2 |u - u'|^2 / |u + u'|^2
+    of the returned velocities and of those one update earlier (the same solve
+    stopped there), to the rounding of the sums."""
+    kw = dict(TIGHT, **CHOSEN)
+    a, ia = solve(V, dome, **dict(kw, visc_it_nit=nit))
+    n = ia.n_visc_its  # updates made; a limit of m stops after m + 1
+    assert n == nit + 1 if nit < 800 else ia.rel_residual <= 1e-8
+    u, v = a["u_vav_b"], a["v_vav_b"]
+    pu, pv = np.zeros_like(u), np.zeros_like(v)
+    if n > 1:
+        b, ib = solve(V, dome, **dict(kw, visc_it_nit=n - 2))
+        assert ib.n_visc_its == n - 1
+        pu, pv = b["u_vav_b"], b["v_vav_b"]
+    L2 = 2.0 * (((u - pu) ** 2 + (v - pv) ** 2).sum() / ((u + pu) ** 2 + (v + pv) ** 2).sum())
+    assert abs(ia.L2_uv - L2) <= 1e-9 * L2
+
+
+def test_verbose_only_prints(V, dome, monkeypatch, capfd):
+    """UFE_VERBOSE prints a line per iteration, each with its own change norm
+    (the last one is the returned one), and leaves the solve as it is, with
+    sums read late and at once."""
+    for kw in (dict(TIGHT, **CHOSEN), dict(visc_it_norm_dUV_tol=1e-6, rtol=1e-11, abstol=0.0, visc_it_nit=300)):
+        monkeypatch.delenv("UFE_VERBOSE", raising=False)
+        a, ia = solve(V, dome, **kw)
+        monkeypatch.setenv("UFE_VERBOSE", "1")
+        capfd.readouterr()
+        b, ib = solve(V, dome, **kw)
+        lines = [ln.split() for ln in capfd.readouterr().err.splitlines() if ln.startswith("[ufe] it ")]
+        assert [int(ln[2]) for ln in lines] == list(range(1, ia.n_visc_its + 1))
+        assert lines[-1][6] == "%.3e" % ia.L2_uv
+        assert ia.n_visc_its == ib.n_visc_its and ia.L2_uv == ib.L2_uv and ia.rel_residual == ib.rel_residual
+        assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
 
 
 def test_mixed_precision_matches_fp64(V, dome):

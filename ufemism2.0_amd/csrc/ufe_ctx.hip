@@ -563,6 +563,14 @@ static int run_picard(ufe_ctx *c, bool diva, ufe_solve_info *info) {
     L2_prev = L2;
     L2 = 2.0 * c->h_scalars[0] / std::max(c->h_scalars[1], 1e-8);
   };
+  const bool late = q.stop_rule == UFE_STOP_RESIDUAL && q.accel_depth > 0;
+  // UFE_VERBOSE: an iteration's line, once its change norm is there
+  struct { int it, its, nref, clamped; double resid; } line{};
+  auto report = [&] {
+    if (verbose)
+      std::fprintf(stderr, "[ufe] it %d resid %.3e L2 %.3e relax %.3f eps0 %.2e krylov %d refs %d clamped %d\n", line.it,
+                   line.resid, L2, relax, eps0, line.its, line.nref, line.clamped);
+  };
   while (!converged) {
     ++it;
     // regularisation continuation: epsilon_sq_0 * 10^(n_cont - it + 1) for it <= n_cont
@@ -575,7 +583,7 @@ static int run_picard(ufe_ctx *c, bool diva, ufe_solve_info *info) {
     bool r_known = false;
     if (q.stop_rule == UFE_STOP_RESIDUAL) {
       resid = loop_residual(c, &n_clamped, norms);
-      if (pending >= 0) collect();
+      if (pending >= 0) { collect(); report(); }
       if (!in_cont && resid <= q.nonlinear_rtol) {
         resid = rel_residual(c, &n_clamped);  // leaves the unscaled residual for the diagnostics below
         --it;
@@ -596,7 +604,8 @@ static int run_picard(ufe_ctx *c, bool diva, ufe_solve_info *info) {
                   diva ? c->F2b0.as<double>() : nullptr, q.sliding_law == UFE_SLIDING_NO_SLIDING,
                   diva ? c->ubase.as<double>() : nullptr, diva ? c->taub.as<double>() : nullptr, s);
     pending = ev0;
-    if (!(q.stop_rule == UFE_STOP_RESIDUAL && q.accel_depth > 0) || verbose) {
+    line = {it, its, nref, n_clamped, resid};
+    if (!late) {
       UFE_HIP(hipStreamSynchronize(s));
       collect();
     }
@@ -609,15 +618,14 @@ static int run_picard(ufe_ctx *c, bool diva, ufe_solve_info *info) {
         break;
       }
     }
-    if (verbose)
-      std::fprintf(stderr, "[ufe] it %d resid %.3e L2 %.3e relax %.3f eps0 %.2e krylov %d refs %d clamped %d\n", it,
-                   resid, L2, relax, eps0, its, nref, n_clamped);
+    if (!late) report();
     if (q.stop_rule == UFE_STOP_L2UV && L2 < q.visc_it_norm_dUV_tol) converged = true;
     if (it > q.visc_it_nit) { rc = UFE_WARN_NOT_CONVERGED; break; }
   }
   if (pending >= 0) {
     UFE_HIP(hipStreamSynchronize(s));
     collect();
+    report();
   }
   if (diva && rc >= 0) {
     // F1_3D_b of the last state the loop evaluated: calc_3D_velocities
