@@ -132,6 +132,28 @@ def test_product_matches_oracle_at_the_ends_of_its_range(V, OB, L, nz, h):
     assert abs(gpu["rel_residual"] - ora["rel_residual"]) < 1e-9 * ora["rel_residual"]
 
 
+def test_product_is_timed_only_on_a_formed_system(V, L):
+    """The measurement hook reads the viscosity fields and the geometry of the
+    system formed last: refused on a fresh set-up and after a solve that ended
+    before one was formed (no grounded ice), taken after an evaluation."""
+    c = Case(h=30e3, zeta=np.linspace(0.0, 1.0, 4))
+    inp = _slab_inputs(c, -0.01, 0.0)
+    kw = dict(glens_n=3.0, sliding_law=1, slid_weertman_m=1.0)
+    s = _solver(V, c, **kw)
+    with pytest.raises(V.VelocitySolverError, match="no BPA system"):
+        s.bpa_profile_spmv(2)
+    s.solve_BPA(inp["Hi"], inp["Hs"], inp["A_flow"], inp["beta_sq"], inp["fgr_b"], np.zeros(c.mesh.nV, np.int32))
+    with pytest.raises(V.VelocitySolverError, match="no BPA system"):
+        s.bpa_profile_spmv(2)
+    s.bpa_residual(*_field(c, 1), **_bpa_kw(inp))
+    ms, nbytes = s.bpa_profile_spmv(2)
+    assert ms > 0.0 and nbytes > c.mesh.nT * c.nz * 64
+    s.zeta_setup(c.aa, c.zs)
+    with pytest.raises(V.VelocitySolverError, match="no BPA system"):
+        s.bpa_profile_spmv(2)
+    s.close()
+
+
 def test_periodic_borders_match_oracle(V, OB, L):
     """'periodic_ISMIP-HOM' borders on a square centred on the origin: the
     lagged copy rows per layer."""

@@ -870,6 +870,7 @@ struct BpaState {
   // iteration
   DBuf x, xprev, rhs, sr4, eta_ak, eta_bks, coef, beta_a, beta_b, cDinv, cW, cU, part, r;
   BpaParams par{};  // of the system formed last
+  bool formed = false;
   std::unique_ptr<Krylov> kry;
   // stage timings of the last solve (HIP events on the context's stream)
   hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -987,7 +988,6 @@ void bpa_pattern(ufe_ctx *c, BpaState &b) {
   const int nT = b.nT, nz = b.nz;
   // points and unknowns are counted in 32 bits (the b->b entries as the mesh counts them)
   if (2L * nT * nz >= (1L << 31)) throw std::runtime_error("BPA system too large: 2^31 unknowns or more");
-  b.nb = nT * nz;
   b.bb_nnz = m.bb_nnz;
   ensure(b.ent, sizeof(BpaEntry) * (size_t)m.bb_nnz);
   hipLaunchKernelGGL(k_bpa_pack, dim3(blocks_for(m.bb_nnz)), dim3(kBlock), 0, s, m.bb_nnz, m.bb_row, m.bb_ind, m.TriC,
@@ -1005,7 +1005,7 @@ void bpa_pattern(ufe_ctx *c, BpaState &b) {
     up(b.copy_w, cw.data(), sizeof(double) * cw.size(), s);
   }
   UFE_HIP(hipStreamSynchronize(s));  // host vectors end here
-  const size_t nbk = (size_t)b.nb;
+  const size_t nbk = (size_t)nT * nz;
   ensure(b.x, sizeof(double2) * nbk);
   ensure(b.xprev, sizeof(double2) * nbk);
   ensure(b.rhs, sizeof(double2) * nbk);
@@ -1020,9 +1020,11 @@ void bpa_pattern(ufe_ctx *c, BpaState &b) {
   ensure(b.cW, sizeof(double4) * nbk);
   ensure(b.cU, sizeof(double4) * nbk);
   ensure(b.part, sizeof(double) * kMaxPartials * 2);
-  b.kry = std::make_unique<Krylov>(b.nb, s);
+  b.kry = std::make_unique<Krylov>(nT * nz, s);
   set_operator(c, b);
-  for (hipEvent_t &ev : b.ev) UFE_HIP(hipEventCreateWithFlags(&ev, hipEventDisableSystemFence));
+  for (hipEvent_t &ev : b.ev)
+    if (!ev) UFE_HIP(hipEventCreateWithFlags(&ev, hipEventDisableSystemFence));
+  b.nb = nT * nz;  // last: after a failed allocation the next call starts over
 }
 
 BpaParams bpa_params(const ufe_ctx *c, double eps0_applied) {
@@ -1128,6 +1130,7 @@ void bpa_state_and_system(ufe_ctx *c, BpaState &b, const BpaParams &p, const int
                        sys.bcm, p.relax_copy, b.xprev.as<double>(), b.rhs.as<double>());
     UFE_LAUNCH_CHECK();
   }
+  b.formed = true;
 }
 
 void velocity_up(ufe_ctx *c, BpaState &b, const double *u, const double *v) {
@@ -1558,7 +1561,8 @@ extern "C" int ufe_bpa_profile_spmv(ufe_ctx *c, int reps, double *avg_ms, double
   if (!c || !avg_ms || !bytes || reps < 1) return ctx_fail(c, UFE_ERR_ARGUMENT, "bad argument");
   return ctx_guard(c, [&]() -> int {
     BpaState *b = state(c);
-    if (!b || !b->nb) return ctx_fail(c, UFE_ERR_ARGUMENT, "no BPA system has been assembled");
+    // the product reads the viscosity fields and the geometry, not a stored matrix
+    if (!b || !b->formed) return ctx_fail(c, UFE_ERR_ARGUMENT, "no BPA system has been formed");
     *avg_ms = b->kry->time_spmv64(bpa_bsr(*b), b->x.as<double>(), b->r.as<double>(), reps, nullptr);
     // b->b entries and row pointers, per-triangle gradients and border index,
     // viscosity fields, x and y, once each
