@@ -109,6 +109,32 @@ def _bicgstab(A, b, rtol, restarts=4):
     return x, its, broken
 
 
+@pytest.mark.parametrize("krylov", ["bicgstab", "gmres"])
+@pytest.mark.parametrize("n,k", [(2000, 19), (2000, 20), (2001, 21), (130_001, 24), (513, 131), (40, 20)])
+def test_csr_solve_on_long_rows(V, L, n, k, krylov):
+    """Block rows around the 20 blocks from which the product takes eight lanes
+    a row, and far longer ones, neighbours and scattered, an odd number of
+    unknowns.  Off-diagonal rows sum to at most 1/2 of the diagonal, so the
+    condition after the Jacobi scaling is at most 3."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n + k)
+    nb = (n + 1) // 2
+    row = np.repeat(np.arange(nb), k)
+    col = (row + np.tile(np.arange(k) - k // 2, nb)) % nb
+    far = rng.random(row.size) < 0.2
+    col[far] = rng.integers(0, nb, far.sum())
+    A = sp.kron(sp.csr_matrix((rng.uniform(-1, 1, row.size), (row, col)), shape=(nb, nb)), np.ones((2, 2)))
+    A = sp.csr_matrix(A)[:n, :n].multiply(rng.uniform(0.5, 1.0, (n, 1))).tocsr()
+    A.setdiag(0.0)
+    A = sp.csr_matrix(A + sp.diags(2.0 * np.asarray(abs(A).sum(axis=1)).ravel() + 1.0))
+    A = sp.csr_matrix(sp.diags(1.0 / A.diagonal()) @ A)
+    x_ex = rng.normal(size=n)
+    x, its, rel = V.csr_solve(A, A @ x_ex, rtol=1e-13, maxit=500, precond=L.PC_JACOBI,
+                              krylov=L.KRYLOV_GMRES if krylov == "gmres" else L.KRYLOV_BICGSTAB)
+    assert its > 0 and rel <= 1.0001e-13
+    assert np.linalg.norm(x - x_ex) < 1e-12 * np.linalg.norm(x_ex)
+
+
 @pytest.mark.parametrize("copies", [1, 33, 4096, 20_000, 40_000])
 def test_bicgstab_restarts_after_a_breakdown(V, L, copies):
     """Copies of a 4x4 system on which every scalar of the first two iterations

@@ -110,23 +110,7 @@ void launch_velocities_3d(int nT, int nz, const double *ubase, const double *bet
 void launch_transpose(int rows, int cols, const double *in, double *out, hipStream_t s);
 void launch_flow_factor_pow(long n, const double *A, double glen_n, double *out, hipStream_t s);
 
-// linear algebra (kernels_linalg.hip)
-struct Bsr64 {
-  int nb = 0, nnzb = 0;
-  const int *ptr = nullptr, *col = nullptr;
-  const double4 *val = nullptr;
-};
-struct Bsr32 {
-  int nb = 0, nnzb = 0;
-  const int *ptr = nullptr, *col = nullptr;
-  const float4 *val = nullptr;
-};
-
-// y = A x (FP64) and, if slot != null, the grid sums ||b - y||^2 and ||b||^2 into out2
-void launch_bsr_residual64(const Bsr64 &A, const double *x, const double *b, double *r, const RedSlot *slot,
-                           double *out2, hipStream_t s);
-void launch_bsr_spmv64(const Bsr64 &A, const double *x, double *y, hipStream_t s);
-void launch_bsr_spmv32(const Bsr32 &A, const float *x, float *y, hipStream_t s);
+// linear algebra (krylov.hip)
 void launch_csr_spmv64(int m, const int *ptr, const int *ind, const double *val, const double *x, double *y,
                        hipStream_t s);
 

@@ -15,7 +15,7 @@
 //       recomputed on the device, as atomic-free gather sums of fine blocks
 //       into coarse blocks.  One V-cycle: damped block-Jacobi pre/post
 //       smoothing, piecewise-constant prolongation, exact solve on the
-//       coarsest level (dense inverse formed in LDS once per Picard
+//       coarsest level (dense inverse formed once per Picard
 //       iteration).  It is a fixed linear operator, so plain BiCGStab applies.
 #pragma once
 
@@ -236,7 +236,7 @@ class Krylov {
   DBuf vec64_[10], vec32_[10];
   DBuf coarse_inv_;      // dense inverse of the coarsest level (column-major)
   DBuf scal_;            // KrylovScalars
-  DBuf red_part_, red_res_;
+  DBuf red_part_;
   KrylovScalars *h_scal_ = nullptr;  // pinned host mirror, written by the device
   double *h_red_ = nullptr;          // pinned: the three sums of a residual product
   bool time_spmv_ = false;

@@ -46,9 +46,12 @@ constexpr int kSpmvLpr = 4;      // lanes per block row in the block product (st
 constexpr int kSpmvBlock = 256;  // workgroup size of the block product
 constexpr int kSpmvRedGrid = kMaxPartials;  // grid cap of the block product with a reduction epilogue
 
-// Rows far longer than the 2-D stencil's (the BPA's block rows hold three
-// layers of a b->b row, ~30-40 blocks) take more lanes per row
-// (spmv_lanes): 8 lanes read 256 contiguous bytes of a row per pass.
+// Rows far longer than the 2-D stencil's, which a caller's own matrix can have
+// (ufe_csr_solve), take 8 lanes, 256 contiguous bytes of a row per pass
+// (spmv_lanes).  Measured with 8 against 4 lanes (us): 50,000 rows of 20
+// neighbouring blocks 7.5 and 7.4, of 24 8.5 and 10.0, of 40 13.0 and 13.6, of
+// 100 29.4 and 31.7; 20,000 rows of 40 scattered blocks 9.4 and 11.2; 1,000 rows
+// of 200 9.2 and 14.8.
 template <typename T, int OP, int LPR = kSpmvLpr>
 __global__ void __launch_bounds__(kSpmvBlock) k_bsr_spmv(
     int nb, const int *__restrict__ ptr, const int *__restrict__ col,
@@ -206,7 +209,8 @@ static int spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T *
   if (ev1) UFE_HIP(hipEventRecord(ev1, s));
   if (fold && nblk <= kFoldParts) return nblk;
   if (OP != OP_PLAIN) {
-    hipLaunchKernelGGL((k_spmv_finish<OP>), dim3(OP == OP_RESID ? 3 : 1), dim3(kFinishBlock), 0, s, slot, nblk, out, sc);
+    hipLaunchKernelGGL((k_spmv_finish<OP>), dim3(OP == OP_RESID ? 3 : 1), dim3(kFinishBlock), 0, s, slot, nblk, out,
+                       sc);
     UFE_LAUNCH_CHECK();
   }
   return 0;
@@ -582,7 +586,6 @@ __global__ void __launch_bounds__(kBlock) k_l1_dinv(int nb, const int *__restric
 }
 
 // z0 = omega D0^-1 r0  (pre-smoothing from a zero guess on the finest level)
-
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_amg_presmooth(int nb, const typename VecT<T>::V2 *__restrict__ r,
                                                           const typename VecT<T>::V4 *__restrict__ dinv, T omega,
@@ -866,10 +869,9 @@ __global__ void __launch_bounds__(kBlock) k_amg_prolong_smooth(
 
 // Coarsest level: an exact solve with the dense inverse of the coarsest
 // Galerkin matrix (nb <= kCoarseMax blocks), formed once per Picard iteration
-// by Gauss-Jordan elimination with partial pivoting in LDS.
+// by Gauss-Jordan elimination with partial pivoting in registers.
 constexpr int kCoarseMax = 24;
 constexpr int kCoarseN = 2 * kCoarseMax;
-constexpr int kCoarseThreads = 1024;
 
 // The augmented matrix lives in registers: lane = row, wavefront w holds the
 // columns w, w + 16, ... .  A step is a serial chain, which is what bounds the
@@ -1358,7 +1360,6 @@ Krylov::Krylov(int nb, hipStream_t s) : nb_(nb), s_(s) {
   for (auto &v : vec32_) v.alloc(sizeof(float) * 2 * (size_t)nb);
   scal_.alloc(sizeof(KrylovScalars));
   red_part_.alloc(sizeof(double) * kMaxPartials * 4 * 4);
-  red_res_.alloc(sizeof(double) * 4 * 4);
   tail_in_lds_ = hipFuncSetAttribute((const void *)k_amg_tail_lds<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      kTailLdsAll) == hipSuccess &&
                  hipFuncSetAttribute((const void *)k_amg_tail_lds<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1411,7 +1412,7 @@ void Krylov::set_spmv_timing(bool on) {
 RedSlot Krylov::slot(int i) const {
   RedSlot r;
   r.partials = red_part_.as<double>() + (size_t)i * kMaxPartials * 4;
-  r.result = red_res_.as<double>() + 4 * i;
+  r.result = nullptr;  // the sums go where the finishing kernel is told
   return r;
 }
 
@@ -1477,8 +1478,8 @@ void Krylov::amg_setup(const BsrT<T> &A0) {
     V4 *const val = av.arena.template as<V4>() + av.val[l], *const dinv = av.arena.template as<V4>() + av.dinv[l];
     B.val = val;
     B.dinv = dinv;
-    hipLaunchKernelGGL(k_galerkin<T>, dim3(blocks_for((long)P.nnzb * kGalLanes)), dim3(kBlock), 0, s_, P.nnzb, P.gptr.as<int>(),
-                       P.glist.as<int>(), lev[l - 1].val, P.crow.as<int>(), P.col.as<int>(),
+    hipLaunchKernelGGL(k_galerkin<T>, dim3(blocks_for((long)P.nnzb * kGalLanes)), dim3(kBlock), 0, s_, P.nnzb,
+                       P.gptr.as<int>(), P.glist.as<int>(), lev[l - 1].val, P.crow.as<int>(), P.col.as<int>(),
                        val, dinv);
     UFE_LAUNCH_CHECK();
     if (amg_l1_) {
@@ -1818,16 +1819,16 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
     // (consecutive Picard systems need similar counts), then grow 1, 2, 4, ...
     // up to check_every past it.  Which iterations run is decided on the
     // device, so the chunking does not change the result.
-    // One BiCGStab iteration: every kernel returns at once after convergence
-    // (device flag), so a chunk may run past it.  k picks the timing events.
-    // with a V-cycle whose finest pre-smoothing is a pass of its own, the
-    // updates of p and s write it
+    // With a V-cycle whose finest pre-smoothing is a pass of its own, the
+    // updates of p and s write it.
     Presmooth<T> pre{nullptr, nullptr, T(0)};
     if (amg && amg_->n_levels() > 1 && !(unit_diag0_ && !amg_l1_)) {
       std::vector<BsrT<T>> &lev = std::is_same<T, double>::value ? *reinterpret_cast<std::vector<BsrT<T>> *>(&lev64_)
                                                                  : *reinterpret_cast<std::vector<BsrT<T>> *>(&lev32_);
       pre = Presmooth<T>{amg_vals<T>().z[0]->template as<V2>(), lev[0].dinv, (T)amg_omega_};
     }
+    // One BiCGStab iteration: every kernel returns at once after convergence
+    // (device flag), so a chunk may run past it.  k picks the timing events.
     auto launch_iter = [&](int k) {
       hipLaunchKernelGGL(k_bicg_p<T>, dim3(blocks_for(nb)), dim3(kBlock), 0, s_, nb,
                          reinterpret_cast<const V2 *>(r), reinterpret_cast<V2 *>(p), reinterpret_cast<const V2 *>(v),
@@ -2369,28 +2370,6 @@ SolveStats Krylov::gmres64(const BsrT<double> &A, const double *b, double *x, do
 SolveStats Krylov::gmres32(const BsrT<float> &A, const float *b, float *x, double rtol, double abstol, int maxit,
                            bool zero_guess, int restart, int check_every) {
   return gmres<float>(A, b, x, rtol, abstol, maxit, zero_guess, restart, check_every);
-}
-
-// Generic wrappers declared in kernels.h
-void launch_bsr_spmv64(const Bsr64 &A, const double *x, double *y, hipStream_t s) {
-  BsrT<double> B;
-  B.nb = A.nb; B.nnzb = A.nnzb; B.ptr = A.ptr; B.col = A.col; B.val = A.val;
-  RedSlot dummy{};
-  spmv_launch<double, OP_PLAIN>(B, x, y, nullptr, nullptr, dummy, nullptr, nullptr, s);
-}
-
-void launch_bsr_spmv32(const Bsr32 &A, const float *x, float *y, hipStream_t s) {
-  BsrT<float> B;
-  B.nb = A.nb; B.nnzb = A.nnzb; B.ptr = A.ptr; B.col = A.col; B.val = A.val;
-  RedSlot dummy{};
-  spmv_launch<float, OP_PLAIN>(B, x, y, nullptr, nullptr, dummy, nullptr, nullptr, s);
-}
-
-void launch_bsr_residual64(const Bsr64 &A, const double *x, const double *b, double *r, const RedSlot *slot,
-                           double *out2, hipStream_t s) {
-  BsrT<double> B;
-  B.nb = A.nb; B.nnzb = A.nnzb; B.ptr = A.ptr; B.col = A.col; B.val = A.val;
-  spmv_launch<double, OP_RESID>(B, x, r, b, nullptr, *slot, out2, nullptr, s);
 }
 
 void launch_f64_to_f32(int n, const double *a, float *b, hipStream_t s) {

@@ -589,8 +589,9 @@ struct Layout {
   }
 };
 
-// persistent workgroups of the tile kernels: two per CU fit beside k_layer_back's
-// 78 KB of LDS, and each adds one partial gradient to sum
+// persistent workgroups of the tile kernels: k_layer_back's 71 KB of LDS
+// (72,960 bytes) leave room for two per CU, and each adds one partial gradient
+// to sum
 constexpr int kMaxParts = 512;
 inline int grid_rows(int N) { return std::max(1, std::min((N + kRows - 1) / kRows, 4 * kMaxParts)); }
 inline int grid_parts(int N) { return std::min(grid_rows(N), kMaxParts); }
