@@ -212,6 +212,14 @@ int  ufe_set_sliding_cap(ufe_ctx *ctx, const double *alpha_sq, const double *eff
  * block rows, run in one workgroup (0..4096, default 300).  Takes effect from
  * the next solve. */
 int  ufe_set_amg_options(ufe_ctx *ctx, double omega, double coarse_scale, int tail_rows);
+/* Measurement hook (no reference counterpart): the multigrid hierarchy and
+ * where the last V-cycle of the context's solves ran its levels.  rows: block
+ * rows of the first max_levels levels, finest first.  route4: [0] number of
+ * levels (0: no hierarchy), [1] first level of those that one workgroup took
+ * (the last level, or -1 before any V-cycle: none), [2] the kernel that took
+ * them (0 none, 1 from device memory, 2 from LDS), [3] levels whose residual
+ * and restriction ran in one pass. */
+int  ufe_amg_levels(const ufe_ctx *ctx, int max_levels, int *rows, int *route4);
 /* Launch mode of the Krylov iterations (no reference counterpart): enable != 0
  * replays chunks of BiCGStab iterations from HIP graphs captured once per
  * context (one hipGraphLaunch instead of ~50 kernel launches per iteration;

@@ -132,6 +132,30 @@ def test_product_matches_oracle_at_the_ends_of_its_range(V, OB, L, nz, h):
     assert abs(gpu["rel_residual"] - ora["rel_residual"]) < 1e-9 * ora["rel_residual"]
 
 
+@pytest.mark.parametrize("nz,h", [(3, 5e3), (9, 9e3), (32, 9e3)])
+def test_residual_with_several_groups_per_workgroup(V, L, monkeypatch, nz, h):
+    """A residual takes at most 8,192 workgroups, so from 65,000 triangles of 32
+    layers on they take several groups of columns each, reusing their LDS;
+    UFE_BPA_GRID lowers that number.  Eight workgroups against one per group: the
+    same rows bit for bit, the norms in another order of addition."""
+    c = Case(h=h, zeta=np.linspace(0.0, 1.0, nz))
+    nT = c.mesh.nT
+    print(f"BPA groups nT={nT} nz={nz}", flush=True)
+    assert nT > 8 * (256 // nz)  # several groups each
+    kw = dict(glens_n=3.0, sliding_law=1, slid_weertman_m=3.0, bc_u=[0, 1, 0, 1], bc_v=[1, 0, 0, 1])
+    u, v = _field(c, 11)
+    out = []
+    for grid in (None, "8"):
+        if grid:
+            monkeypatch.setenv("UFE_BPA_GRID", grid)
+        s = _solver(V, c, **kw)
+        out.append(s.bpa_residual(u, v, **_bpa_kw(_bumpy(c))))
+        s.close()
+    a, b = out
+    assert np.array_equal(a["r"], b["r"]) and np.array_equal(a["b"], b["b"])
+    assert abs(a["rel_residual"] - b["rel_residual"]) <= 1e-12 * a["rel_residual"]
+
+
 def test_product_is_timed_only_on_a_formed_system(V, L):
     """The measurement hook reads the viscosity fields and the geometry of the
     system formed last: refused on a fresh set-up and after a solve that ended

@@ -343,39 +343,140 @@ def test_chosen_form_reaches_the_oracle_solution_on_other_seeds(V, W, sb):
         assert err < 1e-5, (seed, err)
 
 
-@pytest.mark.parametrize("variant", [{"UFE_AMG_TAIL_ROWS": "0"}, {"UFE_AMG_FOLD": "0"}], ids=["no-tail", "no-fold"])
+def solve_levels(V, w, **kw):
+    """solve() with the hierarchy and where its levels ran."""
+    s = V.VelocitySolver(w.descriptor(), **kw)
+    inp = w.inputs()
+    args = (inp["Hi"], inp["Hs"], inp["A_flow"], inp["beta_sq"], inp["fgr_b"], inp["mask_grounded"])
+    try:
+        if w.stress_balance == "DIVA":
+            st, _, _, info = s.solve_DIVA(*args)
+            u, v = st["u_vav_b"], st["v_vav_b"]
+        else:
+            u, v, _, _, info = s.solve_SSA(*args)
+        return u, v, info, s.amg_levels()
+    finally:
+        s.close()
+
+
+def assert_same_solve(a, b):
+    assert a[2].n_visc_its == b[2].n_visc_its and a[2].n_Axb_its == b[2].n_Axb_its
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+PER_LEVEL = {"UFE_AMG_TAIL_ROWS": "0", "UFE_AMG_FUSED": "0"}
+VARIANTS = {"per-level": PER_LEVEL, "no-tail": {"UFE_AMG_TAIL_ROWS": "0"}, "no-fused-pass": {"UFE_AMG_FUSED": "0"},
+            "no-fold": {"UFE_AMG_FOLD": "0"}}
+
+
+@pytest.mark.parametrize("variant", list(VARIANTS))
 @pytest.mark.parametrize("sb", ["SSA", "DIVA"])
 def test_amg_fused_variants_equal_per_level_kernels(V, channel_fixtures, monkeypatch, sb, variant):
-    """The one-workgroup kernel for the coarse V-cycle levels and the finest
-    level's pre-smoothing folded into its passes run the same arithmetic as
-    the separate kernels: identical iterations and bit-identical velocities.
-    UFE_AMG_TAIL_ROWS (largest level given to the one-workgroup kernel, 0 =
-    none) and UFE_AMG_FOLD (0 = separate pre-smoothing kernel) apply to the
-    contexts created afterwards."""
+    """The one-workgroup kernel for the coarse V-cycle levels, residual and
+    restriction of a level in one pass and the finest level's pre-smoothing
+    folded into its passes run the same arithmetic as the separate kernels:
+    identical iterations and bit-identical velocities.  UFE_AMG_TAIL_ROWS
+    (largest level given to the one-workgroup kernel, 0 = none), UFE_AMG_FUSED
+    (0 = residual and restriction as two kernels) and UFE_AMG_FOLD (0 = separate
+    pre-smoothing kernel) apply to the contexts created afterwards."""
     w, _ = channel_fixtures[sb]
     monkeypatch.setenv("UFE_AMG_TAIL_ROWS", "4096")
-    a, ia = solve(V, w, **TIGHT, **CHOSEN)
-    for k, v in variant.items():
+    a = solve_levels(V, w, **TIGHT, **CHOSEN)
+    assert len(a[3]["tail"]) >= 3 and a[3]["fused"] >= 1
+    for k, v in VARIANTS[variant].items():
         monkeypatch.setenv(k, v)
-    b, ib = solve(V, w, **TIGHT, **CHOSEN)
-    assert ia.n_visc_its == ib.n_visc_its and ia.n_Axb_its == ib.n_Axb_its
-    assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
+    b = solve_levels(V, w, **TIGHT, **CHOSEN)
+    if "UFE_AMG_TAIL_ROWS" in VARIANTS[variant]:
+        assert b[3]["tail"] == [] and b[3]["fused"] in (0, len(b[3]["rows"]) - 1)
+    if "UFE_AMG_FUSED" in VARIANTS[variant]:
+        assert b[3]["fused"] == 0
+    assert_same_solve(a, b)
+
+
+@pytest.mark.parametrize("form", ["chosen-l1-smoother", "chosen-fp32-precond", "mixed-amg"])
+def test_amg_fused_pass_equals_two_kernels_in_every_form(V, channel_fixtures, monkeypatch, form):
+    """Residual and restriction in one pass against the two kernels with the l1
+    smoother (the pre-smoothed vector is read, not scaled from r), the FP32
+    finest matrix and the FP32 V-cycle, on every level, bit for bit."""
+    w, _ = channel_fixtures["SSA"]
+    kw = dict(TIGHT, **FORMS[form])
+    monkeypatch.setenv("UFE_AMG_TAIL_ROWS", "0")
+    a = solve_levels(V, w, **kw)
+    monkeypatch.setenv("UFE_AMG_FUSED", "0")
+    b = solve_levels(V, w, **kw)
+    assert a[3]["fused"] == len(a[3]["rows"]) - 1 >= 3 and b[3]["fused"] == 0
+    assert_same_solve(a, b)
 
 
 @pytest.mark.parametrize("l1", [0, 1])
-@pytest.mark.parametrize("rows", ["30", "100", "300"])
-def test_amg_tail_in_lds_equals_the_one_in_device_memory(V, channel_fixtures, monkeypatch, rows, l1):
-    """The one-workgroup kernel of the coarse levels with patterns and values in
-    LDS (taken when they fit) against the one that reads them from device
-    memory (4096 rows do not fit): one to three levels in it, bit for bit."""
-    w, _ = channel_fixtures["SSA"]
-    form = dict(CHOSEN, amg_smoother=l1)
-    monkeypatch.setenv("UFE_AMG_TAIL_ROWS", "4096")
-    a, ia = solve(V, w, **TIGHT, **form)
+@pytest.mark.parametrize("case,rows,kernel,levels", [("dome", "300", "lds", 3), ("dome", "100", "lds", 2),
+                                                     ("channel", "300", "lds", 2), ("channel", "4096", "device", 3)])
+def test_amg_tail_kernels_equal_the_per_level_kernels(V, W, channel_fixtures, monkeypatch, case, rows, kernel, levels,
+                                                      l1):
+    """The one-workgroup kernels of the coarse levels, the one with everything
+    in LDS and the one that reads patterns and values from device memory (taken
+    where they do not fit), with two and three levels in them, against a launch
+    per pass and level, bit for bit.  The 90 km dome's hierarchy ends in levels
+    of 189, 30 and 5 rows, the channel's in 940, 145 and 24."""
+    w = W.dome(h=90e3) if case == "dome" else channel_fixtures["SSA"][0]
+    kw = dict(TIGHT, **dict(CHOSEN, amg_smoother=l1))
     monkeypatch.setenv("UFE_AMG_TAIL_ROWS", rows)
-    b, ib = solve(V, w, **TIGHT, **form)
+    a = solve_levels(V, w, **kw)
+    assert a[3]["tail_kernel"] == kernel and len(a[3]["tail"]) == levels, a[3]
+    for k, v in PER_LEVEL.items():
+        monkeypatch.setenv(k, v)
+    b = solve_levels(V, w, **kw)
+    assert b[3]["tail_kernel"] == "none" and b[3]["fused"] == 0
+    assert_same_solve(a, b)
+
+
+def test_amg_aggregates_too_large_for_the_fused_pass(V, OB, L, dome, monkeypatch):
+    """Three aggregation passes per level: aggregates of more than 64 rows keep
+    the residual and the restriction as two kernels.  The reference's iteration
+    with near-exact linear solves, so the oracle's velocities."""
+    monkeypatch.setenv("UFE_AMG_PASSES", "3")
+    kw = dict(visc_it_norm_dUV_tol=1e-6, rtol=1e-11, abstol=0.0, visc_it_nit=300)
+    u, v, info, lev = solve_levels(V, dome, precond=L.PC_AMG, **kw)
+    assert len(lev["rows"]) >= 2 and lev["rows"][0] > 64 * lev["rows"][1] and lev["fused"] == 0, lev
+    rc, uo, vo, io = OB.Oracle(dome.descriptor()).solve_ssa(params(L, **kw), dome.inputs())
+    assert rc == 0 and info.n_visc_its == io.n_visc_its
+    assert max_rel(u, uo) < 1e-6 and max_rel(v, vo) < 1e-6
+
+
+@pytest.mark.parametrize("form", list(FORMS) + ["reference"])
+def test_dot_sums_in_the_updates_equal_the_finishing_kernels(V, dome, monkeypatch, form):
+    """Up to 1,024 partial sums BiCGStab's updates add a dot product's partials
+    themselves; above (systems of more than 65,536 block rows) kernels of their
+    own do, which UFE_KRYLOV_FOLD=0 takes at any size: the same additions in the
+    same order, bit for bit."""
+    kw = dict(TIGHT, **FORMS[form]) if form != "reference" else dict(rtol=1e-10, abstol=0.0, visc_it_nit=20)
+    a, ia = solve(V, dome, **kw)
+    monkeypatch.setenv("UFE_KRYLOV_FOLD", "0")
+    b, ib = solve(V, dome, **kw)
     assert ia.n_visc_its == ib.n_visc_its and ia.n_Axb_its == ib.n_Axb_its
     assert np.array_equal(a["u_vav_b"], b["u_vav_b"]) and np.array_equal(a["v_vav_b"], b["v_vav_b"])
+
+
+@pytest.mark.parametrize("n", [131_072, 131_073])
+def test_bicgstab_on_either_side_of_the_folded_sums(V, L, monkeypatch, n):
+    """The last system whose 1,024 partials the updates add and the first that
+    takes the finishing kernels, against a solution known in advance
+    (diagonally dominant by a factor 2, condition at most 3 after scaling);
+    where the sums are folded, bit for bit the kernels' result."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n)
+    A = sp.csr_matrix((rng.uniform(-1, 1, 5 * n), (np.repeat(np.arange(n), 5), rng.integers(0, n, 5 * n))),
+                      shape=(n, n))
+    A.setdiag(0.0)
+    A = sp.csr_matrix(A + sp.diags(2.0 * np.asarray(abs(A).sum(axis=1)).ravel() + 1.0))
+    A = sp.csr_matrix(sp.diags(1.0 / A.diagonal()) @ A)
+    x_ex = rng.normal(size=n)
+    b = A @ x_ex
+    x, its, rel = V.csr_solve(A, b, rtol=1e-13, maxit=500)
+    assert its > 0 and rel <= 1.0001e-13 and np.linalg.norm(x - x_ex) < 1e-12 * np.linalg.norm(x_ex)
+    monkeypatch.setenv("UFE_KRYLOV_FOLD", "0")
+    y, its_y, _ = V.csr_solve(A, b, rtol=1e-13, maxit=500)
+    assert its_y == its and np.array_equal(x, y)
 
 
 @pytest.mark.parametrize("h", [9e3, 6e3, 4.5e3])

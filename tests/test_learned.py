@@ -56,10 +56,11 @@ def test_gradients_match_reference(graph):
         assert np.linalg.norm(got - ref) <= 2e-2 * np.linalg.norm(ref) + 1e-7, k
 
 
-@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 131, 40_000])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 131, 40_000, 140_001])
 def test_layer_kernels_at_the_edges_of_their_tiles(n):
-    """Fewer nodes than a tile, one more than a tile, more tiles than
-    workgroups; a chain graph with end nodes of one neighbour and, every
+    """Fewer nodes than a tile, one more than a tile, more tiles than the
+    backward kernels' 512 workgroups and (above 131,072 nodes) than the forward
+    ones' 2,048; a chain graph with end nodes of one neighbour and, every
     seventh node, none.  Bounds of the tests above (BF16 operands; a rounding
     to BF16 that flips is 2^-8 of one operand)."""
     from ufemism2_amd import learned as LN

@@ -29,6 +29,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <memory>
@@ -1073,13 +1074,15 @@ BsrT<double> bpa_bsr(const BpaState &b) {
 // rhs the residual y = rhs - A x and its partial sums (their number returned).
 void set_operator(ufe_ctx *c, BpaState &b) {
   BpaState *bp = &b;
-  b.kry->set_custom_op([c, bp](const double *x, double *y, const double *rhs, const RedSlot &slot,
+  const char *e = std::getenv("UFE_BPA_GRID");  // workgroups of a residual at most
+  const int cap = e ? std::min(xcd_grid(std::max(std::atoi(e), 1)), kMaxPartials) : kMaxPartials;
+  b.kry->set_custom_op([c, bp, cap](const double *x, double *y, const double *rhs, const RedSlot &slot,
                                const KrylovScalars *sc) -> int {
     const BpaSys sys = bpa_sys(c, *bp, bp->tribi.as<int>());
     int g = xcd_grid(blocks_for(bp->nT, kBlock / bp->nz));
     hipStream_t s = ctx_stream(c);
     if (rhs) {
-      g = std::min(g, kMaxPartials);
+      g = std::min(g, cap);
       hipLaunchKernelGGL(k_bpa_product<true>, dim3(g), dim3(kBlock), 0, s, sys, bp->zops(), bp->par,
                          reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y),
                          reinterpret_cast<const double2 *>(rhs), slot, sc);

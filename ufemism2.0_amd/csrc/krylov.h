@@ -132,6 +132,14 @@ class Krylov {
   // Run the coarse levels of the V-cycle with at most max_rows block rows in
   // one workgroup (0: one launch per pass on every level).
   void set_amg_tail(int max_rows) { amg_tail_rows_ = max_rows; }
+  // Residual and restriction of a level in one pass where its aggregates allow
+  // (default), or as two kernels.
+  void set_amg_fused(bool on) { amg_fused_ = on; }
+  // Where the last V-cycle ran its levels: the first of those taken by one
+  // workgroup (the coarsest alone: none), by which kernel (0 none, 1 from device
+  // memory, 2 from LDS), and the levels above it with the fused pass.
+  struct AmgRoute { int first_tail = -1, tail_kernel = 0, n_fused = 0; };
+  const AmgRoute &amg_route() const { return amg_route_; }
   // l1 block-Jacobi smoothing on every level (true) or plain block Jacobi;
   // the finest level's pre-smoothing is then not folded into its passes
   void set_amg_l1(bool on) { amg_l1_ = on; }
@@ -223,6 +231,9 @@ class Krylov {
   const int *A_diag_ = nullptr;
   const float4 *fine32_ = nullptr;
   int amg_tail_rows_ = 300;
+  bool amg_fused_ = true;
+  AmgRoute amg_route_;
+  int fold_parts_;  // partials up to which BiCGStab's updates add a dot product's sums
   bool tail_in_lds_ = false;  // the device gives a workgroup kTailLdsAll bytes of LDS
   bool amg_l1_ = false;
   bool unit_diag0_ = false;

@@ -178,12 +178,12 @@ inline int spmv_lanes(int nb, long nnzb) { return nnzb >= 20L * nb ? 8 : kSpmvLp
 constexpr int kFoldParts = 1024;
 
 // Returns the number of partial sums left in the slot for the next kernel to
-// add (fold, with a dot epilogue and few workgroups), else 0.
+// add (a dot epilogue of at most fold workgroups), else 0.
 template <typename T, int OP>
 static int spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T *w, const RedSlot &slot,
                         double *out, KrylovScalars *sc, hipStream_t s, double vmax = 0.0,
                         const typename VecT<T>::V4 *dblk = nullptr, int write_unscaled = 0,
-                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr, bool fold = false) {
+                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr, int fold = 0) {
   using V2 = typename VecT<T>::V2;
   const int lpr = spmv_lanes(A.nb, A.nnzb);
   long threads = (long)A.nb * lpr;
@@ -207,7 +207,7 @@ static int spmv_launch(const BsrT<T> &A, const T *x, T *y, const T *b, const T *
                        write_unscaled);
   UFE_LAUNCH_CHECK();
   if (ev1) UFE_HIP(hipEventRecord(ev1, s));
-  if (fold && nblk <= kFoldParts) return nblk;
+  if (nblk <= fold) return nblk;
   if (OP != OP_PLAIN) {
     hipLaunchKernelGGL((k_spmv_finish<OP>), dim3(OP == OP_RESID ? 3 : 1), dim3(kFinishBlock), 0, s, slot, nblk, out,
                        sc);
@@ -1354,8 +1354,9 @@ std::unique_ptr<AmgHierarchy> build_amg_hierarchy(int nT, const int *TriC, const
   return H;
 }
 
-Krylov::Krylov(int nb, hipStream_t s) : nb_(nb), s_(s) {
+Krylov::Krylov(int nb, hipStream_t s) : nb_(nb), s_(s), fold_parts_(kFoldParts) {
   if (const char *e = std::getenv("UFE_VERBOSE")) verbose_ = std::atoi(e);
+  if (const char *e = std::getenv("UFE_KRYLOV_FOLD")) fold_parts_ = std::min(std::max(std::atoi(e), 0), kFoldParts);
   for (auto &v : vec64_) v.alloc(sizeof(double) * 2 * (size_t)nb);
   for (auto &v : vec32_) v.alloc(sizeof(float) * 2 * (size_t)nb);
   scal_.alloc(sizeof(KrylovScalars));
@@ -1533,6 +1534,7 @@ void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, h
   int t = L - 1;
   for (int l = 1; l < L - 1; ++l)
     if (lev[l].nb <= std::min(amg_tail_rows_, kTailMaxRows) && L - l <= kTailMaxLevels) { t = l; break; }
+  amg_route_ = {t, 0, 0};
   for (int l = 0; l < t; ++l) {
     const AmgLevelPattern &P = *amg_->levels[l];
     const V2 *rin = l == 0 ? rl : av.r[l]->template as<V2>();
@@ -1542,7 +1544,8 @@ void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, h
     const V2 *zl = l == 0 ? zl0 : av.z[l]->template as<V2>();
     const T zs = l == 0 ? zs0 : T(1);
     V2 *zc = next_coarsest ? (V2 *)nullptr : av.z[l + 1]->template as<V2>();
-    if (P.n_wg) {
+    if (P.n_wg && amg_fused_) {
+      ++amg_route_.n_fused;
       const dim3 gw(xcd_grid(P.n_wg));
       if (l == 0 && fine32_ && std::is_same<T, double>::value)
         hipLaunchKernelGGL((k_amg_resid_restrict<T, float>), gw, dim3(kBlock), 0, s_, P.n_wg, P.wg_agg.as<int>(),
@@ -1636,9 +1639,11 @@ void Krylov::precond_apply(const BsrT<T> &A, const T *r, T *z, hipEvent_t ev0, h
         hipLaunchKernelGGL(k_amg_tail_lds<T>, dim3(1), dim3(kTailThreads), end, s_, ta, sc);
         UFE_LAUNCH_CHECK();
         tail_done = true;
+        amg_route_.tail_kernel = 2;
       }
     }
     if (!tail_done) {
+      amg_route_.tail_kernel = 1;
       for (int l = 0; l < ta.n; ++l) ta.lv[l].off_r = ta.lv[l].off_z = ta.lv[l].off_zt = -1;
       // the vectors that stay inside the kernel go to LDS: every level's zt and
       // the r and z of the levels below the top one
@@ -1700,7 +1705,8 @@ std::vector<uintptr_t> Krylov::graph_key(const BsrT<T> &A, const T *b, const T *
   std::vector<uintptr_t> k = {(uintptr_t)A.nb, (uintptr_t)A.nnzb, (uintptr_t)A.ptr, (uintptr_t)A.col,
                               (uintptr_t)A.val, (uintptr_t)A.dinv, (uintptr_t)b, (uintptr_t)x, (uintptr_t)nbx,
                               (uintptr_t)pc_, (uintptr_t)amg_, (uintptr_t)A_diag_, (uintptr_t)fine32_,
-                              (uintptr_t)amg_tail_rows_, (uintptr_t)unit_diag0_, (uintptr_t)amg_l1_,
+                              (uintptr_t)amg_tail_rows_, (uintptr_t)amg_fused_, (uintptr_t)unit_diag0_,
+                              (uintptr_t)amg_l1_,
                               bits(amg_omega_),
                               bits(amg_coarse_scale_), (uintptr_t)coarse_inv_.p, (uintptr_t)red_part_.p,
                               (uintptr_t)vec64_[0].p, (uintptr_t)vec32_[0].p, (uintptr_t)scal_.p};
@@ -1838,7 +1844,8 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
         precond_apply<T>(A, p, phat, timing ? tev_[8 * k + 4] : nullptr, timing ? tev_[8 * k + 5] : nullptr,
                          pre.z != nullptr);
       const int n1 = spmv_launch<T, OP_DOT1>(A, phat, v, nullptr, rhat, sl1, nullptr, sc, s_, 0.0, nullptr, 0,
-                                             timing ? tev_[8 * k] : nullptr, timing ? tev_[8 * k + 1] : nullptr, true);
+                                             timing ? tev_[8 * k] : nullptr, timing ? tev_[8 * k + 1] : nullptr,
+                                             fold_parts_);
       hipLaunchKernelGGL(k_bicg_s<T>, dim3(blocks_for(nb)), dim3(kBlock), 0, s_, nb,
                          reinterpret_cast<const V2 *>(r), reinterpret_cast<const V2 *>(v), reinterpret_cast<V2 *>(s),
                          reinterpret_cast<V2 *>(amg ? (T *)nullptr : shat), pcl, A.dinv, A.val, A_diag_, pre, sl1, n1,
@@ -1849,7 +1856,7 @@ SolveStats Krylov::bicgstab(const BsrT<T> &A, const T *b, T *x, double rtol, dou
                          pre.z != nullptr);
       const int n2 = spmv_launch<T, OP_DOT2>(A, shat, t, nullptr, s, sl2, nullptr, sc, s_, 0.0, nullptr, 0,
                                              timing ? tev_[8 * k + 2] : nullptr, timing ? tev_[8 * k + 3] : nullptr,
-                                             true);
+                                             fold_parts_);
       hipLaunchKernelGGL(k_bicg_x<T>, dim3(nbx), dim3(kBlock), 0, s_, nb, reinterpret_cast<V2 *>(x),
                          reinterpret_cast<const V2 *>(phat), reinterpret_cast<const V2 *>(shat),
                          reinterpret_cast<const V2 *>(s), reinterpret_cast<const V2 *>(t), reinterpret_cast<V2 *>(r),

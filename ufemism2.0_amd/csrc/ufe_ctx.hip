@@ -975,6 +975,7 @@ extern "C" int ufe_ctx_create(ufe_ctx **out, int device, const ufe_mesh_desc *md
       double cs = (e = std::getenv("UFE_AMG_SCALE")) ? std::atof(e) : 1.5;
       c->kry->set_amg_options(om, 0, cs);
       if ((e = std::getenv("UFE_AMG_TAIL_ROWS"))) c->kry->set_amg_tail(std::max(0, std::atoi(e)));
+      if ((e = std::getenv("UFE_AMG_FUSED"))) c->kry->set_amg_fused(std::atoi(e) != 0);
       if ((e = std::getenv("UFE_AMG_FOLD"))) c->amg_fold = std::atoi(e) != 0;
       if ((e = std::getenv("UFE_DIVA_COLUMNS"))) c->m.diva_columns = std::atoi(e) != 0;
       if ((e = std::getenv("UFE_GRAPHS"))) c->kry->set_graphs(std::atoi(e) != 0);
@@ -1020,6 +1021,19 @@ extern "C" int ufe_set_amg_options(ufe_ctx *c, double omega, double coarse_scale
     c->kry->set_amg_tail(tail_rows);
     return UFE_OK;
   });
+}
+
+extern "C" int ufe_amg_levels(const ufe_ctx *c, int max_levels, int *rows, int *route4) {
+  if (!c || !route4 || max_levels < 0 || (max_levels && !rows))
+    return fail(const_cast<ufe_ctx *>(c), UFE_ERR_ARGUMENT, "bad argument");
+  const int n = c->amg ? c->amg->n_levels() : 0;
+  for (int l = 0; l < std::min(n, max_levels); ++l) rows[l] = c->amg->levels[l]->nb;
+  const Krylov::AmgRoute &r = c->kry->amg_route();
+  route4[0] = n;
+  route4[1] = r.first_tail;
+  route4[2] = r.tail_kernel;
+  route4[3] = r.n_fused;
+  return UFE_OK;
 }
 
 extern "C" int ufe_set_sliding_cap(ufe_ctx *c, const double *alpha_sq, const double *effective_pressure) {

@@ -142,6 +142,16 @@ class VelocitySolver:
                                                  int(opts["tail_rows"])))
         self.amg_options = opts
 
+    def amg_levels(self):
+        """Block rows per multigrid level and where the last V-cycle ran them:
+        the levels one workgroup took together ("tail", empty: none) and its
+        kernel, and how many levels above had the fused pass."""
+        rows, route = np.zeros(64, np.int32), np.zeros(4, np.int32)
+        self._check(self.lib.ufe_amg_levels(self._ctx, rows.size, L.ptr(rows, L.ip), L.ptr(route, L.ip)))
+        rows = rows[:route[0]].tolist()
+        return {"rows": rows, "tail": rows[route[1]:] if route[2] else [],
+                "tail_kernel": ("none", "device", "lds")[route[2]], "fused": int(route[3])}
+
     def set_sliding_cap(self, alpha_sq=None, effective_pressure=None):
         """Coulomb limit alpha_sq * effective_pressure ([nV] each) of the
         Tsai2015 and Schoof2005 sliding laws (sliding_laws.f90:244-351), kept
