@@ -1,7 +1,7 @@
 """ctypes binding of oracle/_build/liboracle.so.
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and the
-cpu_baseline leg of bench.py, as the checker.  The engine never imports it.
+cpu_baseline leg of bench.py, as the oracle.  The engine never imports it.
 It reuses the engine package's ctypes structures only as a data layout.
 """
 

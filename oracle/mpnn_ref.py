@@ -1,5 +1,5 @@
 """NumPy restatement of the engine's mesh message-passing network (forward,
-loss and backward).  TEST INFRASTRUCTURE ONLY: the checker for the HIP
+loss and backward).  TEST INFRASTRUCTURE ONLY: the oracle for the HIP
 training and inference kernels; the engine never imports it.
 
 Network on the triangle graph (neighbours = TriC, mean aggregation):

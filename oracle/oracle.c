@@ -1,7 +1,7 @@
 /*
  * oracle.c -- FP64 CPU restatement of UFEMISM's velocity solve and vertical
  * heat columns.  TEST INFRASTRUCTURE ONLY: the parity tests, smoke() and the
- * cpu_baseline leg of bench.py call it as the checker.  The product never
+ * cpu_baseline leg of bench.py call it as the oracle.  The product never
  * links, loads or calls anything in this directory.
  *
  * Every function cites the reference routine it restates (paths relative to

@@ -1,4 +1,4 @@
-"""The network's NumPy restatement (the checker of the HIP kernels) is pinned
+"""The network's NumPy restatement (the oracle of the HIP kernels) is pinned
 by central finite differences of its float64 forward pass."""
 
 import numpy as np
